@@ -109,23 +109,36 @@ __device__ __forceinline__ float tanh_f32(float x) {
   return __builtin_copysignf(ax < 0.125f ? p : big, x);
 }
 
-// sin / cos: Cody-Waite reduction by pi/2 with a three-part constant (P1 + P2 + P3 = pi/2 to ~2^-75;
-// the first FMA is exact for the quadrants below 2^17), then Taylor polynomials for sin and cos on
-// [-pi/4, pi/4] (truncation below 2^-28). Arguments of magnitude 2^17 and beyond take the library's
-// sinf / cosf (Payne-Hanek reduction).
-__device__ __forceinline__ float sincos_core(float r, int q) {
+// The quadrant form of sin and cos: x = k pi/2 + r with k = rint(x / (pi/2)) read off the low mantissa
+// bits of x / (pi/2) + 1.5 * 2^23, r by a three-part reduction with FMAs (pi/2 = P1 + P2 + P3 to
+// ~2^-75, every part positive, so that x = -0 keeps r = -0; the first FMA is exact for the quadrants
+// below 2^17), then Taylor polynomials for sin and cos on [-pi/4, pi/4] (truncation below 2^-28): quadrant
+// q's value is sin r, cos r, -sin r, -cos r for q mod 4 = 0 .. 3. Arguments of magnitude 2^17 and
+// beyond take the library's sinf / cosf (Payne-Hanek reduction).
+__device__ __forceinline__ float quadrant_reduce(float x, u32_t& q) {
+  const float M = 0x1.8p+23f;
+  const float P1 = 0x1.921fb4p+0f, P2 = 0x1.4442d0p-24f, P3 = 0x1.84698ap-48f;
+  const float t = __builtin_fmaf(x, 0x1.45f306p-1f, M);
+  const float k = t - M;
+  q = __builtin_bit_cast(u32_t, t);
+  float r = __builtin_fmaf(-k, P1, x);
+  r = __builtin_fmaf(-k, P2, r);
+  return __builtin_fmaf(-k, P3, r);
+}
+__device__ __forceinline__ float sincos_core(float r, u32_t q) {
   const float r2 = r * r;
   float s = __builtin_fmaf(r2, 0x1.71de3ap-19f, -0x1.a01a02p-13f);  // 1/9!, -1/7!
   s = __builtin_fmaf(r2, s, 0x1.111112p-7f);                          // 1/5!
   s = __builtin_fmaf(r2, s, -0x1.555556p-3f);                         // -1/3!
   s = __builtin_fmaf(r * r2, s, r);
+  s = __builtin_copysignf(s, r);  // only matters for r = -0, which the FMA turns into +0
   float c = __builtin_fmaf(r2, -0x1.27e4fcp-22f, 0x1.a01a02p-16f);  // -1/10!, 1/8!
   c = __builtin_fmaf(r2, c, -0x1.6c16c2p-10f);                        // -1/6!
   c = __builtin_fmaf(r2, c, 0x1.555556p-5f);                          // 1/4!
   c = __builtin_fmaf(r2, c, -0.5f);
   c = __builtin_fmaf(r2, c, 1.0f);
   const float v = (q & 1) ? c : s;
-  return __builtin_bit_cast(float, __builtin_bit_cast(u32_t, v) ^ ((u32_t)(q & 2) << 30));
+  return __builtin_bit_cast(float, __builtin_bit_cast(u32_t, v) ^ ((q & 2) << 30));
 }
 
 // sin with one polynomial: x = k pi + r, k = rint(x / pi) read off the low mantissa bits of
@@ -165,13 +178,20 @@ __device__ __forceinline__ float sin_f32(float x) {
 }
 
 __device__ __forceinline__ float cos_f32(float x) {
-  const float P1 = 0x1.921fb6p+0f, P2 = -0x1.777a5cp-25f, P3 = -0x1.ee59dap-50f;
-  const float k = __builtin_rintf(x * 0x1.45f306p-1f);
-  float r = __builtin_fmaf(-k, P1, x);
-  r = __builtin_fmaf(-k, P2, r);
-  r = __builtin_fmaf(-k, P3, r);
-  float v = sincos_core(r, (int)k + 1);
+  u32_t q;
+  const float r = quadrant_reduce(x, q);
+  float v = sincos_core(r, q + 1);
   if (__builtin_fabsf(x) >= 0x1p+17f) v = cos_large(x);
+  return v;
+}
+
+// sin in cos_f32's form, for a value whose cosine the program takes as well: the two then share one
+// reduction and both polynomials (about 26 VALU operations for the pair where sin_f32 and cos_f32 take 38).
+__device__ __forceinline__ float sin_with_cos_f32(float x) {
+  u32_t q;
+  const float r = quadrant_reduce(x, q);
+  float v = sincos_core(r, q);
+  if (__builtin_fabsf(x) >= 0x1p+17f) v = sin_large(x);
   return v;
 }
 

@@ -231,6 +231,12 @@ std::string KernelWriter::store(int slot, const std::string& off, DType d, const
   }
 }
 
+bool KernelWriter::cosine_too(uint32_t arg) const {
+  for (const Op& op : g_.ops)
+    if (op.kind == Kind::unary && (Unary)op.code == Unary::cos && op.args[0] == arg) return true;
+  return false;
+}
+
 std::string KernelWriter::value(uint32_t vid, const std::vector<std::string>& coords, Scope& sc) {
   std::string key = std::to_string(vid) + "@";
   for (const auto& c : coords) key += c + ",";
@@ -284,7 +290,7 @@ std::string KernelWriter::value(uint32_t vid, const std::vector<std::string>& co
           case Unary::log: e = (f ? "logf(" : "log(") + x + ")"; break;
           case Unary::sqrt: e = (f ? "sqrtf(" : "sqrt(") + x + ")"; break;
           case Unary::tanh: e = (f ? "accy::tanh_f32(" : "tanh(") + x + ")"; break;
-          case Unary::sin: e = (f ? "accy::sin_f32(" : "sin(") + x + ")"; break;
+          case Unary::sin: e = (!f ? "sin(" : cosine_too(op.args[0]) ? "accy::sin_with_cos_f32(" : "accy::sin_f32(") + x + ")"; break;
           case Unary::cos: e = (f ? "accy::cos_f32(" : "cos(") + x + ")"; break;
           case Unary::tan: e = (f ? "tanf(" : "tan(") + x + ")"; break;
         }

@@ -82,6 +82,7 @@ class KernelWriter {
   std::string itype;
 
  private:
+  bool cosine_too(uint32_t arg) const;  // some operation takes the cosine of value `arg`
   const Graph& g_;
   Slots& slots_;
   int ntmp_ = 0;

@@ -247,6 +247,12 @@ class Planner {
   // ---- fold: one output per thread, serial left-to-right over the reduced index ----
   void fold(uint32_t v);
 
+  // The statements of one output of a fold kernel computing every reduction of `group` (same axes, same
+  // extents); without `commit`, only a trial (NotFusable when an operand is not ready).
+  std::string fold_body(KernelWriter& w, const std::vector<uint32_t>& group, const Type& in, const std::vector<size_t>& red,
+                        const std::vector<size_t>& keep, const std::vector<Dim>& rdims, const std::vector<Dim>& kdims,
+                        uint64_t nred, bool commit);
+
   // The value a chunk's fold starts from, so that folding the chunks' partials in order from the
   // program's init gives the serial fold's result: -0 for a float sum (x + -0 = x for every x,
   // including -0), NaN for a float max / min (fold_max / fold_min skip a NaN second operand and return
@@ -286,6 +292,9 @@ class Planner {
   void push_row(KernelStep k);
 
   bool try_row(const RowShape& rs, const RowKernel& rk);
+
+  // Per reduction of a row kernel: the pass over the row that computes it (0 first).
+  std::vector<int> reduction_passes(const RowKernel& rk) const;
 
   KernelStep gen_row(const RowShape& rs, const RowKernel& rk, bool commit);
 

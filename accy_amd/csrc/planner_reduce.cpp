@@ -11,9 +11,9 @@ void Planner::fold(uint32_t v) {
   const Op& op = g_.ops[v];
   const Type& in = g_.type(op.args[0]);
   const Type& rt = op.result;
-  int out = slots_.slot_of[v] >= 0 ? slots_.slot_of[v] : temp_slot(v);
   uint64_t nout = rt.elements();
   if (nout == 0) {
+    temp_slot(v);
     finish(v);
     return;
   }
@@ -30,44 +30,83 @@ void Planner::fold(uint32_t v) {
   // too few loads in flight), so the range is folded in chunks and the chunks' partials folded in
   // order (fold_chunked).
   if (nred >= 1024 && nout * nred >= (1ull << 22) && nout < (1ull << 18) && chunk_identity(d, r)) {
+    const int out = temp_slot(v);
     fold_chunked(v, out, in, red, keep, rdims, kdims, nout, nred, r, d);
     finish(v);
     return;
   }
+  // Later folds over the same axes of the same extents whose operands are ready join this one: one
+  // launch, and what their elementwise operands share (loads, a sine) is evaluated once. Each output
+  // keeps its own left-to-right order. (The README's mismatch and slope of eight guesses: 10.7 us a
+  // pass in two launches, 7.5 us in one.)
+  std::vector<uint32_t> group{v};
+  const std::set<int64_t> axes(op.ints.begin(), op.ints.end());
+  const bool long_range = nred >= 1024 && nout * nred >= (1ull << 22) && nout < (1ull << 18);
+  constexpr size_t kMaxFolds = 4;
+  for (uint32_t u = v + 1; !long_range && u < (uint32_t)g_.ops.size() && group.size() < kMaxFolds; ++u) {
+    const Op& uo = g_.ops[u];
+    if (!live_[u] || done_[u] || uo.kind != Kind::reduce || !(g_.type(uo.args[0]).dims == in.dims)) continue;
+    if (std::set<int64_t>(uo.ints.begin(), uo.ints.end()) != axes) continue;
+    // a product of two broadcasts may be a contraction spelled elementwise (mulsum), planned at its turn
+    const Op& x = g_.ops[uo.args[0]];
+    if (x.kind == Kind::binary && (Binary)x.code == Binary::mul && g_.ops[x.args[0]].kind == Kind::broadcast_in_dim &&
+        g_.ops[x.args[1]].kind == Kind::broadcast_in_dim)
+      continue;
+    group.push_back(u);
+    try {
+      KernelWriter trial(g_, slots_, itype());
+      fold_body(trial, group, in, red, keep, rdims, kdims, nred, false);
+    } catch (const NotFusable&) {
+      group.pop_back();
+    }
+  }
   KernelWriter w(g_, slots_, itype());
-  std::ostringstream body;
-  Scope outer(body, "    ");
-  std::vector<std::string> kc = delinearize("o", kdims);
-  std::string init = w.value(op.args[1], {}, outer);
-  std::string at = acc_type(d, r);
-  body << "    " << at << " acc = (" << at << ")" << init << ";\n";
-  body << "    for (I r = 0; r < (I)" << nred << "; ++r) {\n";
-  Scope inner(body, "      ");
-  std::vector<std::string> rc = delinearize("r", rdims);
-  std::vector<std::string> full(in.rank());
-  for (size_t i = 0; i < red.size(); ++i) full[red[i]] = rc[i];
-  for (size_t i = 0; i < keep.size(); ++i) full[keep[i]] = kc[i];
-  std::string x = w.value(op.args[0], full, inner);
-  body << "      acc = " << serial_fold_step(d, r, "acc", x) << ";\n    }\n";
-  std::string res = is_int(d) ? "(" + std::string(compute_type(d)) + ")acc" : round_to(d, "acc");
-  body << "    " << w.store(out, "o", d, res) << "\n";
+  const std::string body = fold_body(w, group, in, red, keep, rdims, kdims, nred, true);
   const uint32_t B = 256;
-  std::string nm = name("fold", v);
+  std::string nm = name("fold", v), label = "fold:%" + std::to_string(v);
+  for (size_t i = 1; i < group.size(); ++i) label += "&%" + std::to_string(group[i]);
   std::ostringstream src;
   src << "extern \"C\" __global__ void __launch_bounds__(" << B << ") " << nm << "(" << w.params() << ") {\n"
       << "  typedef " << w.itype << " I;\n"
       << "  for (I o = (I)blockIdx.x * " << B << " + threadIdx.x; o < (I)" << nout << "; o += (I)gridDim.x * "
       << B << ") {\n"
-      << body.str() << "  }\n}\n";
+      << body << "  }\n}\n";
   KernelStep k;
   k.source = src.str();
   k.name = nm;
   k.grid[0] = grid_for(nout, B, 65536);
   k.block[0] = B;
   k.klass = "fold";
-  k.label = "fold:%" + std::to_string(v);
+  k.label = label;
   push(std::move(k), w);
-  finish(v);
+  for (uint32_t u : group) finish(u);
+}
+
+std::string Planner::fold_body(KernelWriter& w, const std::vector<uint32_t>& group, const Type& in, const std::vector<size_t>& red,
+                               const std::vector<size_t>& keep, const std::vector<Dim>& rdims, const std::vector<Dim>& kdims,
+                               uint64_t nred, bool commit) {
+  std::ostringstream body, steps, stores;
+  Scope outer(body, "    "), inner(steps, "      ");
+  std::vector<std::string> kc = delinearize("o", kdims), rc = delinearize("r", rdims);
+  std::vector<std::string> full(in.rank());
+  for (size_t i = 0; i < red.size(); ++i) full[red[i]] = rc[i];
+  for (size_t i = 0; i < keep.size(); ++i) full[keep[i]] = kc[i];
+  for (size_t i = 0; i < group.size(); ++i) {
+    const Op& op = g_.ops[group[i]];
+    const Reducer r = (Reducer)op.code;
+    const DType d = op.result.dtype;
+    const std::string at = acc_type(d, r), acc = "acc" + (i ? std::to_string(i) : std::string());
+    const std::string init = w.value(op.args[1], {}, outer);
+    body << "    " << at << " " << acc << " = (" << at << ")" << init << ";\n";
+    const std::string x = w.value(op.args[0], full, inner);
+    steps << "      " << acc << " = " << serial_fold_step(d, r, acc, x) << ";\n";
+    if (!commit) continue;
+    const int out = slots_.slot_of[group[i]] >= 0 ? slots_.slot_of[group[i]] : temp_slot(group[i]);
+    const std::string res = is_int(d) ? "(" + std::string(compute_type(d)) + ")" + acc : round_to(d, acc);
+    stores << "    " << w.store(out, "o", d, res) << "\n";
+  }
+  body << "    for (I r = 0; r < (I)" << nred << "; ++r) {\n" << steps.str() << "    }\n" << stores.str();
+  return body.str();
 }
 
 std::optional<std::string> Planner::chunk_identity(DType d, Reducer r) {
@@ -249,6 +288,26 @@ bool Planner::try_row(const RowShape& rs, const RowKernel& rk) {
   }
 }
 
+std::vector<int> Planner::reduction_passes(const RowKernel& rk) const {
+  std::vector<int> pass(rk.reduces.size(), 0);
+  std::map<uint32_t, int> needs;  // value: the first pass that can evaluate it
+  std::function<int(uint32_t)> first_pass = [&](uint32_t v) -> int {
+    const auto known = needs.find(v);
+    if (known != needs.end()) return known->second;
+    int p = 0;
+    const auto own = std::find(rk.reduces.begin(), rk.reduces.end(), v);
+    if (own != rk.reduces.end()) {
+      p = pass[(size_t)(own - rk.reduces.begin())] + 1;
+    } else if (is_inlinable(g_.ops[v].kind) && slots_.available(v) < 0) {
+      for (uint32_t a : g_.ops[v].args) p = std::max(p, first_pass(a));
+    }
+    return needs[v] = p;
+  };
+  for (size_t j = 0; j < rk.reduces.size(); ++j)  // in program order: what j reads comes before it
+    for (uint32_t a : g_.ops[rk.reduces[j]].args) pass[j] = std::max(pass[j], first_pass(a));
+  return pass;
+}
+
 KernelStep Planner::gen_row(const RowShape& rs, const RowKernel& rk, bool commit) {
   uint64_t tn = prod(rs.T, 0, rs.T.size()), kn = prod(rs.K, 0, rs.K.size());
   const uint32_t VEC = tn % 4 == 0 ? 4 : 1;
@@ -260,7 +319,13 @@ KernelStep Planner::gen_row(const RowShape& rs, const RowKernel& rk, bool commit
   // meeting two waves at its barriers instead of four.
   uint32_t B = lanes >= 128 ? 128 : (uint32_t)std::max<uint64_t>(64, (lanes + 63) / 64 * 64);
   uint64_t E = (tn + (uint64_t)B * VEC - 1) / ((uint64_t)B * VEC);
-  size_t passes = rk.reduces.size() + (rk.full_vals.empty() ? 0 : 1);
+  // Reductions that need no other's result share one pass over the row: pass_of[j] is one more than the
+  // latest pass whose result reduction j reads. (A pass for each made every one of them load, or keep
+  // in registers, the same row and evaluate the same elementwise values again: the mismatch and its
+  // slope over 8192 x 16384 took 694 us in two passes of a cached, fully unrolled row, 82 us in one.)
+  const std::vector<int> pass_of = reduction_passes(rk);
+  const int reduce_passes = 1 + *std::max_element(pass_of.begin(), pass_of.end());
+  size_t passes = (size_t)reduce_passes + (rk.full_vals.empty() ? 0 : 1);
   // A row read by several passes is kept in registers when each thread holds at most 64 of its
   // elements; a row too long for that with 128 threads takes 256, 512 or 1024 threads if that makes it
   // fit (read once instead of once per pass; four waves per SIMD still have 128 registers each).
@@ -389,11 +454,11 @@ KernelStep Planner::gen_row(const RowShape& rs, const RowKernel& rk, bool commit
     return true;
   };
   std::vector<std::string> red_var(rk.reduces.size());
-  size_t avail = 0;
+  int passes_done = 0;
   w.provide = [&](uint32_t vid, const std::vector<std::string>& coords, std::string& out) -> bool {
     for (size_t j = 0; j < rk.reduces.size(); ++j) {
       if (rk.reduces[j] != vid) continue;
-      if (j >= avail || coords != kc) throw NotFusable("reduction used outside its row");
+      if (pass_of[j] >= passes_done || coords != kc) throw NotFusable("reduction used outside its row");
       out = red_var[j];
       return true;
     }
@@ -430,40 +495,49 @@ KernelStep Planner::gen_row(const RowShape& rs, const RowKernel& rk, bool commit
   };
   std::string loop_tail = guard ? "        }\n      }\n    }\n" : "      }\n    }\n";
   std::string lds_decl;
-  for (size_t j = 0; j < rk.reduces.size(); ++j) {
-    cur_pass = (int)j;
-    const Op& op = g_.ops[rk.reduces[j]];
-    Reducer r = (Reducer)op.code;
-    DType d = op.result.dtype;
-    std::string at = acc_type(d, r);
-    Scope pre(body, "    ");
-    std::string init = w.value(op.args[1], {}, pre);
-    std::string acc = "acc" + std::to_string(j);
-    // Every thread folds its share of the row, then the shares are combined. max / min may start
-    // every share from the init (it is idempotent under them); a sum takes the init once, in the
-    // first thread's share, and the others start from the additive identity (-0 for floats, so
-    // that a share of -0 elements stays -0).
-    if (r == Reducer::sum) {
-      const std::string zero = is_int(d) ? "(" + at + ")0" : (d == DType::f64 ? "-0.0" : "-0.0f");
-      body << "    " << at << " " << acc << " = " << tid << " == 0 ? (" << at << ")" << init << " : " << zero << ";\n";
-    } else {
-      body << "    " << at << " " << acc << " = (" << at << ")" << init << ";\n";
-    }
+  for (cur_pass = 0; cur_pass < reduce_passes; ++cur_pass) {
     std::ostringstream ib;
     Scope inner(ib, guard ? "          " : "        ");
-    std::string x = w.value(op.args[0], full, inner);
-    ib << inner.indent << acc << " = " << fold_step(d, r, acc, x) << ";\n";
+    for (size_t j = 0; j < rk.reduces.size(); ++j) {
+      if (pass_of[j] != cur_pass) continue;
+      const Op& op = g_.ops[rk.reduces[j]];
+      Reducer r = (Reducer)op.code;
+      DType d = op.result.dtype;
+      std::string at = acc_type(d, r);
+      Scope pre(body, "    ");
+      std::string init = w.value(op.args[1], {}, pre);
+      std::string acc = "acc" + std::to_string(j);
+      // Every thread folds its share of the row, then the shares are combined. max / min may start
+      // every share from the init (it is idempotent under them); a sum takes the init once, in the
+      // first thread's share, and the others start from the additive identity (-0 for floats, so
+      // that a share of -0 elements stays -0).
+      if (r == Reducer::sum) {
+        const std::string zero = is_int(d) ? "(" + at + ")0" : (d == DType::f64 ? "-0.0" : "-0.0f");
+        body << "    " << at << " " << acc << " = " << tid << " == 0 ? (" << at << ")" << init << " : " << zero << ";\n";
+      } else {
+        body << "    " << at << " " << acc << " = (" << at << ")" << init << ";\n";
+      }
+      std::string x = w.value(op.args[0], full, inner);
+      ib << inner.indent << acc << " = " << fold_step(d, r, acc, x) << ";\n";
+    }
     emit_loop(ib.str(), loop_tail);
-    std::string lds = "lds" + std::to_string(j);
-    lds_decl += "  __shared__ " + at + " " + lds + "[" + std::to_string(std::max<uint32_t>(B / 64, 1)) + "];\n";
-    body << "    " << acc << " = accy::block_reduce<" << B << ">(" << acc << ", " << reducer_op(r) << ", " << lds
-         << ");\n";
-    red_var[j] = "red" + std::to_string(j);
-    std::string res = is_int(d) ? "(" + std::string(compute_type(d)) + ")" + acc : round_to(d, acc);
-    body << "    const " << compute_type(d) << " " << red_var[j] << " = " << res << ";\n";
-    if (commit && slots_.slot_of[rk.reduces[j]] >= 0)
-      body << "    if (" << tid << " == 0) " << w.store(slots_.slot_of[rk.reduces[j]], "row", d, red_var[j]) << "\n";
-    avail = j + 1;
+    for (size_t j = 0; j < rk.reduces.size(); ++j) {
+      if (pass_of[j] != cur_pass) continue;
+      const Op& op = g_.ops[rk.reduces[j]];
+      Reducer r = (Reducer)op.code;
+      DType d = op.result.dtype;
+      std::string acc = "acc" + std::to_string(j);
+      std::string lds = "lds" + std::to_string(j);
+      lds_decl += "  __shared__ " + acc_type(d, r) + " " + lds + "[" + std::to_string(std::max<uint32_t>(B / 64, 1)) + "];\n";
+      body << "    " << acc << " = accy::block_reduce<" << B << ">(" << acc << ", " << reducer_op(r) << ", " << lds
+           << ");\n";
+      red_var[j] = "red" + std::to_string(j);
+      std::string res = is_int(d) ? "(" + std::string(compute_type(d)) + ")" + acc : round_to(d, acc);
+      body << "    const " << compute_type(d) << " " << red_var[j] << " = " << res << ";\n";
+      if (commit && slots_.slot_of[rk.reduces[j]] >= 0)
+        body << "    if (" << tid << " == 0) " << w.store(slots_.slot_of[rk.reduces[j]], "row", d, red_var[j]) << "\n";
+    }
+    passes_done = cur_pass + 1;
   }
   if (!rk.row_vals.empty()) {
     body << "    if (" << tid << " == 0) {\n";
@@ -475,7 +549,7 @@ KernelStep Planner::gen_row(const RowShape& rs, const RowKernel& rk, bool commit
     body << "    }\n";
   }
   if (!rk.full_vals.empty()) {
-    cur_pass = (int)rk.reduces.size();
+    cur_pass = reduce_passes;
     std::ostringstream ib;
     Scope sc(ib, guard ? "          " : "        ");
     for (uint32_t v : rk.full_vals) {
