@@ -175,6 +175,20 @@ std::string KernelWriter::params() const {
   return s;
 }
 
+KernelWriter::Members KernelWriter::members() const {
+  Members m;
+  const std::string pl = params();
+  for (size_t start = 0; start < pl.size();) {
+    const size_t comma = pl.find(", ", start);
+    const std::string decl = pl.substr(start, comma == std::string::npos ? std::string::npos : comma - start);
+    m.decls += "  " + decl + ";\n";
+    m.inits += (m.inits.empty() ? "" : ", ") + decl.substr(decl.rfind(' ') + 1);
+    if (comma == std::string::npos) break;
+    start = comma + 2;
+  }
+  return m;
+}
+
 std::string KernelWriter::align_hints() const {
   std::string s;
   for (size_t i = 0; i < args.size(); ++i) {

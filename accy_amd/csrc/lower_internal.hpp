@@ -70,6 +70,9 @@ class KernelWriter {
   std::string store(int slot, const std::string& off, DType d, const std::string& v);
   std::string tmp();
   std::string params() const;
+  // The parameters as members of a functor that a kernel template takes, and their initialisers.
+  struct Members { std::string decls, inits; };
+  Members members() const;
   std::string align_hints() const;  // tells the compiler every buffer is 16-byte aligned
 
   // Lets a kernel supply values itself (a row kernel's own reduction results).

@@ -377,63 +377,118 @@ void Planner::dot_serial(uint32_t v) {
   finish(v);
 }
 
-// ---- scatter_add: copy the input, then add updates in order, one (pre, post) position per thread ----
+// ---- scatter_add: one pass over the table, every row's updates added in order (kernels/scatter.h) ----
 
 void Planner::scatter_add(uint32_t v) {
   const Op& op = g_.ops[v];
   const Type& rt = op.result;
   int out = slots_.slot_of[v] >= 0 ? slots_.slot_of[v] : temp_slot(v);
-  map_into(op.args[0], out);
   const Type& it = g_.type(op.args[1]);
   size_t axis = (size_t)op.axis;
   uint64_t pre = prod(rt.dims, 0, axis), post = prod(rt.dims, axis + 1, rt.rank());
   uint64_t ni = it.elements();
   int64_t ext = rt.dims[axis].extent;
-  uint64_t work = pre * post;
-  if (work == 0 || ni == 0) {
+  if (pre * post == 0 || ni == 0) {
+    map_into(op.args[0], out);
     finish(v);
     return;
   }
   DType d = rt.dtype;
   KernelWriter w(g_, slots_, itype());
-  std::ostringstream body;
-  body << "    const I p = w / (I)" << post << ", q = w % (I)" << post << ";\n";
-  body << "    for (I j = 0; j < (I)" << ni << "; ++j) {\n";
-  Scope sc(body, "      ");
-  std::vector<std::string> jc = delinearize("j", it.dims);
-  std::string idx = w.value(op.args[1], jc, sc);
-  std::vector<Dim> udims = g_.type(op.args[2]).dims;
-  std::vector<std::string> pc = delinearize("p", std::vector<Dim>(rt.dims.begin(), rt.dims.begin() + axis));
-  std::vector<std::string> qc =
-      delinearize("q", std::vector<Dim>(rt.dims.begin() + axis + 1, rt.dims.end()));
-  std::vector<std::string> uc = pc;
-  uc.insert(uc.end(), jc.begin(), jc.end());
-  uc.insert(uc.end(), qc.begin(), qc.end());
-  std::string u = w.value(op.args[2], uc, sc);
-  body << "      const I kk = (I)(" << idx << " < 0 ? 0 : (" << idx << " > " << ext - 1 << " ? " << ext - 1 << " : "
-       << idx << "));\n";
-  body << "      const I dst = (p * (I)" << ext << " + kk) * (I)" << post << " + q;\n";
-  std::string cur = w.load(out, "dst", d);
-  std::string sum;
-  if (is_float_domain(d) || d == DType::f64) sum = round_to(d, "(" + cur + " + " + u + ")");
-  else sum = "accy::wadd<" + std::string(compute_type(d)) + "," + unsigned_type(d) + ">(" + cur + ", " + u + ")";
-  body << "      " << w.store(out, "dst", d, sum) << "\n    }\n";
-  // The output is read and written: drop the const qualifier on its parameter.
-  w.arg(out, true);
-  const uint32_t B = 256;
+  const std::vector<Dim> pre_dims(rt.dims.begin(), rt.dims.begin() + axis), post_dims(rt.dims.begin() + axis + 1, rt.dims.end());
+  const int vec = post % 4 == 0 ? 4 : 1;
+  // A method that evaluates `emit`'s statements for the VEC elements c0 .. of a row; a leaf read at
+  // `rest + c` is loaded once for all of them.
+  auto method = [&](const std::string& head, const std::function<void(std::ostringstream&, Scope&)>& emit) {
+    std::string hoisted;
+    std::map<std::string, std::string> hoisted_var;
+    w.leaf_hook = [&](int s, const std::string& off, DType ld, Scope& sc, std::string& res) -> bool {
+      const std::optional<std::string> base = vec == 4 ? quad_base(off) : std::nullopt;
+      if (!base) return false;
+      const std::string key = std::to_string(s) + "|" + off;
+      auto hv = hoisted_var.find(key);
+      if (hv == hoisted_var.end()) {
+        const std::string q = "q" + std::to_string(hoisted_var.size());
+        hoisted += "    " + w.quad_load(s, q, *base, ld) + "\n";
+        hv = hoisted_var.emplace(key, q).first;
+      }
+      res = w.tmp();
+      sc.out << sc.indent << "const " << compute_type(ld) << " " << res << " = " << KernelWriter::quad_elem(hv->second, "u", ld) << ";\n";
+      return true;
+    };
+    std::ostringstream body;
+    Scope sc(body, "      ");
+    emit(body, sc);
+    w.leaf_hook = nullptr;
+    return "  __device__ __forceinline__ void " + head + " const {\n" + hoisted + "#pragma unroll\n    for (int u = 0; u < VEC; ++u) {\n      const I c = c0 + u;\n" +
+           body.str() + "    }\n  }\n";
+  };
+  auto coords = [&](const std::vector<std::string>& middle) {
+    std::vector<std::string> c = delinearize("p", pre_dims), q = delinearize("c", post_dims);
+    c.insert(c.end(), middle.begin(), middle.end());
+    c.insert(c.end(), q.begin(), q.end());
+    return c;
+  };
+  const std::string at = "(p * (I)" + std::to_string(ext) + " + k) * (I)" + std::to_string(post) + " + c0";
+  std::ostringstream index_body;
+  Scope isc(index_body, "    ");
+  const std::vector<std::string> jc = delinearize("j", it.dims);
+  const std::string idx = w.value(op.args[1], jc, isc);
+  const std::string init = method("init(I p, I k, I c0, T (&v)[VEC])", [&](std::ostringstream& o, Scope& sc) {
+    const std::string x = w.value(op.args[0], coords({ext == 1 ? "0" : "k"}), sc);
+    o << "      v[u] = " << x << ";\n";
+  });
+  const std::string update = method("update(I p, I j, I c0, T (&v)[VEC])", [&](std::ostringstream& o, Scope& sc) {
+    const std::string x = w.value(op.args[2], coords(jc), sc);
+    o << "      v[u] = " << x << ";\n";
+  });
+  const std::string plus = is_float_domain(d) || d == DType::f64
+                               ? round_to(d, "(a + u)")
+                               : std::string("accy::wadd<") + compute_type(d) + "," + unsigned_type(d) + ">(a, u)";
+  const std::string o = w.arg(out, true), st = storage_type(d), quad = "accy::Quad<" + st + ">";
+  std::string again, store;
+  if (vec == 4) {
+    const std::string bits = d == DType::f16 ? "accy::f32_to_f16(v[u])" : d == DType::bf16 ? "accy::f32_to_bf16(v[u])"
+                             : d == DType::i1 ? "(u8_t)(v[u] ? 1 : 0)" : "v[u]";
+    again = "    const " + quad + " q = *(const " + quad + "*)(" + o + " + " + at + ");\n#pragma unroll\n    for (int u = 0; u < VEC; ++u) v[u] = " +
+            KernelWriter::quad_elem("q", "u", d) + ";\n";
+    store = "    " + quad + " q;\n#pragma unroll\n    for (int u = 0; u < VEC; ++u) q.v[u] = " + bits + ";\n    *(" + quad + "*)(" + o + " + " + at + ") = q;\n";
+  } else {
+    again = "    v[0] = " + w.load(out, at, d) + ";\n";
+    store = "    " + w.store(out, at, d, "v[0]") + "\n";
+  }
+  // Threads along a row: enough for its vectors, more (idle while adding) where the rows are too few for
+  // a workgroup on every CU. Each workgroup reads the whole index list, so it owns more rows when
+  // tiles x updates passes 2^28 reads (about the time of a table of 1 GiB), while 1024 tiles remain.
+  const uint64_t vecs = post / vec;
+  uint64_t tc = 1;
+  while (tc < 256 && tc < vecs) tc *= 2;
+  auto tiles_of = [&](uint64_t rows) { return ((uint64_t)ext + rows - 1) / rows * ((vecs + tc - 1) / tc) * pre; };
+  while (tc < 256 && tiles_of(256 / tc * 4) < 512) tc *= 2;
+  const uint64_t group_rows = 256 / tc * 4;
+  uint64_t loop = 1;
+  while (2 * loop * group_rows <= 4096 && tiles_of(2 * loop * group_rows) >= 1024 &&
+         tiles_of(loop * group_rows) > (1ull << 28) / ni)
+    loop *= 2;
   std::string nm = name("scatter", v);
+  const KernelWriter::Members members = w.members();
   std::ostringstream src;
-  std::string params = w.params();
-  src << "extern \"C\" __global__ void __launch_bounds__(" << B << ") " << nm << "(" << params << ") {\n"
-      << "  typedef " << w.itype << " I;\n"
-      << "  for (I w = (I)blockIdx.x * " << B << " + threadIdx.x; w < (I)" << work << "; w += (I)gridDim.x * " << B
-      << ") {\n"
-      << body.str() << "  }\n}\n";
+  src << "#include \"scatter\"\n"
+      << "struct Tab_" << nm << " {\n" << members.decls << "  typedef " << w.itype << " I;\n  typedef " << compute_type(d) << " T;\n"
+      << "  static constexpr long NI = " << ni << ", EXT = " << ext << ", POST = " << post << ", PRE = " << pre << ";\n"
+      << "  static constexpr int VEC = " << vec << ", TC = " << tc << ", LOOP = " << loop << ";\n"
+      << "  __device__ __forceinline__ I index(I j) const {\n" << index_body.str() << "    return (I)(" << idx << " < 0 ? 0 : ("
+      << idx << " > " << ext - 1 << " ? " << ext - 1 << " : " << idx << "));\n  }\n"
+      << "  static __device__ __forceinline__ T plus(T a, T u) { return " << plus << "; }\n" << init << update
+      << "  __device__ __forceinline__ void again(I p, I k, I c0, T (&v)[VEC]) const {\n" << again << "  }\n"
+      << "  __device__ __forceinline__ void store(I p, I k, I c0, const T (&v)[VEC]) const {\n" << store << "  }\n};\n"
+      << "extern \"C\" __global__ void __launch_bounds__(256) " << nm << "(" << w.params() << ") {\n"
+      << "  accy::scatter::rows(Tab_" << nm << "{" << members.inits << "});\n}\n";
   KernelStep k;
   k.source = src.str();
   k.name = nm;
-  k.grid[0] = grid_for(work, B, 65536);
-  k.block[0] = B;
+  k.grid[0] = (uint32_t)std::min<uint64_t>(tiles_of(loop * group_rows), 1u << 20);
+  k.block[0] = 256;
   k.klass = "scatter";
   k.label = "scatter:%" + std::to_string(v);
   push(std::move(k), w);

@@ -37,7 +37,9 @@ inline bool is_inlinable(Kind k) {
 }
 
 // An offset of the form `(rest + c)` (c the innermost coordinate, stride 1; no other term mentions
-// c), as `(rest) + c0`: where the VEC adjacent elements c0 .. c0 + VEC - 1 of one thread start.
+// c), as `(rest) + c0`: where the VEC adjacent elements c0 .. c0 + VEC - 1 of one thread start. Not an
+// offset that reads a temporary (v0, v1, ...: a gathered index), which is only known inside the
+// element's own statements.
 inline std::optional<std::string> quad_base(const std::string& off) {
   if (off.size() < 2 || off.front() != '(' || off.back() != ')') return std::nullopt;
   std::string body = off.substr(1, off.size() - 2), rest;
@@ -51,6 +53,7 @@ inline std::optional<std::string> quad_base(const std::string& off) {
       bool ident_start = i == 0 || !(isalnum((unsigned char)term[i - 1]) || term[i - 1] == '_');
       bool ident_end = i + 1 == term.size() || !(isalnum((unsigned char)term[i + 1]) || term[i + 1] == '_');
       if (term[i] == 'c' && ident_start && ident_end) has_c = true;
+      if (term[i] == 'v' && ident_start && i + 1 < term.size() && isdigit((unsigned char)term[i + 1])) return std::nullopt;
     }
     if (term == "c" && !found) found = true;
     else if (has_c) return std::nullopt;
@@ -541,7 +544,7 @@ class Planner {
   // ---- dot_general with runCpu's per-output serial k order ----
   void dot_serial(uint32_t v);
 
-  // ---- scatter_add: copy the input, then add updates in order, one (pre, post) position per thread ----
+  // ---- scatter_add: one pass over the table, every row's updates added in order ----
   void scatter_add(uint32_t v);
 };
 

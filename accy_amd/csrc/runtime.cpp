@@ -15,6 +15,7 @@ namespace accy {
 extern const char* const kCommonDeviceSource;
 extern const char* const kGemmDeviceSource;
 extern const char* const kAttentionDeviceSource;
+extern const char* const kScatterDeviceSource;
 
 namespace {
 
@@ -58,7 +59,8 @@ hipFunction_t load_kernel(const std::string& body, const std::string& name) {
 std::string full_kernel_source(const std::string& body) {
   std::string out = std::string(kCommonDeviceSource) + "\n";
   const std::pair<const char*, const char*> templates[] = {{"#include \"gemm\"\n", kGemmDeviceSource},
-                                                           {"#include \"attention\"\n", kAttentionDeviceSource}};
+                                                           {"#include \"attention\"\n", kAttentionDeviceSource},
+                                                           {"#include \"scatter\"\n", kScatterDeviceSource}};
   std::string rest = body;
   for (const auto& t : templates) {
     size_t p = rest.find(t.first);

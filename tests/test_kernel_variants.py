@@ -84,3 +84,58 @@ def test_sine_and_cosine_of_one_value_against_float64():
         assert np.isnan(got[len(x):len(x) + 3]).all()
     s, c = hip_run(prog, [xs])
     assert np.signbit(s[-2]) and s[-2] == 0 and s[-1] == 0 and not np.signbit(s[-1]) and c[-2] == c[-1] == 1.0
+
+
+# ---- scatter_add: one pass over the table ----
+
+def scatter(dtype, pre, ext, post, n, computed=False):
+    dims = lambda k, e: [d for d in (("p", pre), (k, e), ("q", post)) if d[1]]
+
+    def body(b, a):
+        table, ids, up = a
+        if computed:    # table and updates that no buffer holds
+            table, up = table.add(table), up.mul(up)
+        return table.scatter_add(ids, up, "k")
+    return T.define("scatter", [T.spec(dtype, *dims("k", ext)), T.spec("i32", j=n), T.spec(dtype, *dims("j", n))], body)
+
+
+# (pre, rows, row elements, updates): a row per workgroup column tile and tails of it; one element per
+# row; fewer rows than a tile; several batches of hits on one row; several row tiles per workgroup
+SCATTERS = [(0, 10, 0, 5), (0, 33, 7, 64), (3, 1001, 4, 513), (0, 37, 1028, 2500), (2, 5, 2052, 40), (0, 1, 12, 3000),
+            (0, 5000, 3, 60000), (0, 9000, 64, 511), (0, 40000, 0, 30000)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", SCATTERS, ids=str)
+@pytest.mark.parametrize("dtype", ["f32", "i32", "bf16"])
+def test_scatter_add_keeps_the_order_of_the_updates(shape, dtype):
+    pre, ext, post, n = shape
+    rng = np.random.default_rng(ext)
+    # half of the indices on a few rows, some out of range (clamped)
+    ids = np.where(rng.random(n) < 0.5, rng.integers(0, min(ext, 3), n), rng.integers(-2, ext + 2, n)).astype(np.int32)
+    size = lambda e: [x for x in (pre, e, post) if x]
+
+    def values(e):
+        x = rng.standard_normal(size(e)) * 8
+        return x.astype(np.int32) if dtype == "i32" else W.to_dtype(x, dtype)
+    ins = [values(ext), ids, values(n)]
+    for computed in (False, True):
+        prog = scatter(dtype, pre, ext, post, n, computed)
+        got, ref = hip_run(prog, ins)[0], oracle_run(prog, ins)[0]
+        assert np.array_equal(got.view(np.uint8), ref.view(np.uint8))   # every sum rounded in order: bit for bit
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("width", [64, 63])
+def test_scatter_add_of_gathered_updates(width):
+    """Updates at a gathered row: their offsets read a temporary, so no vector load is hoisted."""
+    def body(b, a):
+        table, ids, rows, up = a
+        return [table.scatter_add(ids, up.gather(rows, "u"), "k"), up.gather(rows, "u")]
+    prog = T.define("gathered", [T.spec("f32", k=50, q=width), T.spec("i32", j=200), T.spec("i32", j=200),
+                                 T.spec("f32", u=30, q=width)], body)
+    rng = np.random.default_rng(8)
+    ins = [rng.standard_normal((50, width)).astype(np.float32), rng.integers(0, 50, 200).astype(np.int32),
+           rng.integers(0, 30, 200).astype(np.int32), rng.standard_normal((30, width)).astype(np.float32)]
+    for got, ref in zip(hip_run(prog, ins), oracle_run(prog, ins)):
+        assert np.array_equal(got, ref)
