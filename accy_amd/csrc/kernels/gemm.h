@@ -791,7 +791,7 @@ __device__ __forceinline__ void f32_issue(const float* __restrict__ Ab, const fl
 }
 
 template <class C, class Epi>
-__device__ __forceinline__ void mma32f(const float* __restrict__ A, const float* __restrict__ B, const Epi& epi) {
+__device__ __forceinline__ void mma32f_direct(const float* __restrict__ A, const float* __restrict__ B, const Epi& epi) {
   constexpr int BM = 256, BN = 256, BKF = 32;
   constexpr long TILES_M = (C::M + BM - 1) / BM, TILES_N = (C::N + BN - 1) / BN, KT = C::K / BKF;
   static_assert(C::K % BKF == 0 && C::N % 4 == 0, "whole K steps, 16-byte chunks of B rows");
@@ -873,5 +873,248 @@ __device__ __forceinline__ void mma32f(const float* __restrict__ A, const float*
         }
 }
 
+// ---------------------------------------------------------------------------------------------
+// f32 contraction staged through registers: any extents, operands whose K or row axis has stride 1 at
+// any alignment, tiles of BM x BN in {32, 64, 128}, optionally split along K over workgroups.
+//
+// For problems that 256 x 256 tiles of 32 k do not divide or do not spread over 256 CUs. The f32
+// matrix instruction takes 64 cycles for two k, so LDS reads and index arithmetic hide behind it even
+// with the 32 x 32 tile per wave; what bounds these sizes is filling the CUs and the latency of
+// the first loads. WAVES_K groups of waves take separate 32-deep slices of each K step, so that a
+// small tile still has two waves per SIMD; their sums meet in LDS at the end.
+//
+// A stage holds BKT = 32 WAVES_K values of k per row. Loads of the next stage go to registers before
+// the products of this one and to the other LDS buffer after them, one barrier per stage. A
+// K-contiguous operand is stored as [row][k] with rows of BKT + 4 floats (16 consecutive rows of a
+// 16-byte read fall on distinct banks), a row-contiguous one as [k][row]. A lane of half h supplies k =
+// 8 c + 4 h + u to product u of chunk c, for both operands. Rows past the end repeat the last one (they
+// feed outputs that are not stored); k past the end is zero in both operands.
+// ---------------------------------------------------------------------------------------------
+
+struct __attribute__((packed, aligned(4))) F32x4Any { float v[4]; };
+
+// One operand's stage of ROWS x BKT floats: O its offset functions, R its row extent.
+template <int ROWS, int BKT, int THREADS, bool KC, class O, long R, long K>
+struct StageF32 {
+  static constexpr int PER = ROWS * BKT / 4 / THREADS;
+  static constexpr int LD = KC ? BKT + 4 : ROWS, SIZE = KC ? ROWS * LD : BKT * LD;
+  static_assert(PER * THREADS * 4 == ROWS * BKT, "whole vectors per thread");
+  F32x4Any v[PER];
+
+  // No divergent branches: a load behind one is waited for where its registers meet the other side.
+  template <bool TAIL>
+  __device__ __forceinline__ void load(const float* __restrict__ base, long r0, long k0, int t) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int idx = t + i * THREADS;
+      if constexpr (KC) {
+        const long row = r0 + idx / (BKT / 4), k = k0 + idx % (BKT / 4) * 4;
+        const float* __restrict__ p = base + O::row(row < R ? row : R - 1);
+        if constexpr (!TAIL) {
+          v[i] = *(const F32x4Any*)(p + O::k(k));
+        } else if constexpr (K >= 4) {
+          // the last four values of the row, moved down to k's place
+          const long from = k + 4 <= K ? k : K - 4, d = k - from;
+          const F32x4Any w = *(const F32x4Any*)(p + O::k(from));
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            float x = 0.0f;
+#pragma unroll
+            for (int e = j; e < 4; ++e) x = j + d == e ? w.v[e] : x;
+            v[i].v[j] = x;
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const float x = p[O::k(k + j < K ? k + j : K - 1)];
+            v[i].v[j] = k + j < K ? x : 0.0f;
+          }
+        }
+      } else {
+        const long k = k0 + idx / (ROWS / 4), kc = TAIL && k >= K ? K - 1 : k, row = first_row(r0, idx);
+        const float* __restrict__ p = base + O::k(kc);
+        if constexpr (R >= 4) {
+          v[i] = *(const F32x4Any*)(p + O::row(row));
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[i].v[j] = p[O::row(row + j < R ? row + j : R - 1)];
+        }
+        if constexpr (TAIL) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[i].v[j] = k < K ? v[i].v[j] : 0.0f;
+        }
+      }
+    }
+  }
+
+  // First row of vector `idx` of a row-contiguous stage: the last whole vector of the operand where
+  // its own reaches past the end (it then stores rows that another vector stores too).
+  static __device__ __forceinline__ long first_row(long r0, int idx) {
+    const long row = r0 + idx % (ROWS / 4) * 4;
+    if constexpr (R % ROWS == 0 || R < 4) return row;
+    return row < R - 4 ? row : R - 4;
+  }
+
+  __device__ __forceinline__ void store(float* lds, long r0, int t) const {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int idx = t + i * THREADS;
+      const f32x4 w = {v[i].v[0], v[i].v[1], v[i].v[2], v[i].v[3]};
+      if constexpr (KC) {
+        *(f32x4*)(lds + idx / (BKT / 4) * LD + idx % (BKT / 4) * 4) = w;
+      } else {
+        float* const line = lds + idx / (ROWS / 4) * LD;
+        const int at = (int)(first_row(r0, idx) - r0);
+        if constexpr (R % 4 == 0 || R < 4) {
+          *(f32x4*)(line + at) = w;
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if (at + j >= 0) line[at + j] = w[j];  // the last vector may begin before the tile
+        }
+      }
+    }
+  }
+
+  // The four values of row `row` at k .. k + 3 of a stage.
+  static __device__ __forceinline__ f32x4 frag(const float* lds, int row, int k) {
+    if constexpr (KC) return *(const f32x4*)(lds + row * LD + k);
+    else return f32x4{lds[k * LD + row], lds[(k + 1) * LD + row], lds[(k + 2) * LD + row], lds[(k + 3) * LD + row]};
+  }
+};
+
+template <class C, class Epi>
+__device__ __forceinline__ void mma32f_staged(const float* __restrict__ A, const float* __restrict__ B, const Epi& epi) {
+  constexpr int BM = C::BM, BN = C::BN, WM = C::WAVES_M, WN = C::WAVES_N, WK = C::WAVES_K;
+  constexpr int THREADS = 64 * WM * WN * WK, BKT = 32 * WK;
+  constexpr int TM = BM / WM / 32, TN = BN / WN / 32;
+  constexpr long TILES_M = (C::M + BM - 1) / BM, TILES_N = (C::N + BN - 1) / BN;
+  constexpr long STEPS = (C::K + BKT - 1) / BKT, SPLIT_STEPS = (STEPS + C::SPLITS - 1) / C::SPLITS;
+  typedef StageF32<BM, BKT, THREADS, C::A_KC, AOff<C>, C::M, C::K> SA;
+  typedef StageF32<BN, BKT, THREADS, C::B_KC, BOff<C>, C::N, C::K> SB;
+  constexpr int STAGE = SA::SIZE + SB::SIZE, SUMS = (WK - 1) * WM * WN * TM * TN * 1024;
+  __shared__ __attribute__((aligned(16))) float lds[2 * STAGE > SUMS ? 2 * STAGE : SUMS];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wk = wave / (WM * WN), wmn = wave % (WM * WN), wm = wmn / WN, wn = wmn % WN;
+  const int h = lane >> 5, l32 = lane & 31;
+  long tm, tn;
+  tile_of<TILES_M, TILES_N, 8>((long)blockIdx.x, tm, tn);
+  const long m0 = tm * BM, n0 = tn * BN, batch = blockIdx.y, split = blockIdx.z;
+  const float* __restrict__ Ab = A + C::a_b(batch);
+  const float* __restrict__ Bb = B + C::b_b(batch);
+  const long first = split * SPLIT_STEPS, end = first + SPLIT_STEPS < STEPS ? first + SPLIT_STEPS : STEPS;
+
+  f32x16 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = f32x16{};
+
+  SA sa;
+  SB sb;
+  auto load = [&](long s) {
+    if (C::K % BKT == 0 || s + 1 < STEPS) {
+      sa.template load<false>(Ab, m0, s * BKT, tid);
+      sb.template load<false>(Bb, n0, s * BKT, tid);
+    } else {
+      sa.template load<true>(Ab, m0, s * BKT, tid);
+      sb.template load<true>(Bb, n0, s * BKT, tid);
+    }
+  };
+  load(first);
+  sa.store(lds, m0, tid);
+  sb.store(lds + SA::SIZE, n0, tid);
+  __syncthreads();
+  for (long s = first; s < end; ++s) {
+    const float* const as = lds + (s - first & 1) * STAGE;
+    const float* const bs = as + SA::SIZE;
+    const bool more = s + 1 < end;
+    if (more) load(s + 1);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int k = 32 * wk + 8 * c + 4 * h;
+      f32x4 a[TM], b[TN];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) a[i] = SA::frag(as, wm * (BM / WM) + i * 32 + l32, k);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) b[j] = SB::frag(bs, wn * (BN / WN) + j * 32 + l32, k);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) acc[i][j] = mfma32x32x2f32(a[i][u], b[j][u], acc[i][j]);
+    }
+    if (more) {
+      float* const next = lds + (s + 1 - first & 1) * STAGE;
+      sa.store(next, m0, tid);
+      sb.store(next + SA::SIZE, n0, tid);
+    }
+    __syncthreads();
+  }
+  if constexpr (WK > 1) {  // the k groups' sums, added in group order
+    if (wk > 0) {
+      float* const mine = lds + (wk - 1) * (WM * WN * TM * TN * 1024) + wmn * (TM * TN * 1024) + lane;
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) mine[((i * TN + j) * 16 + e) * 64] = acc[i][j][e];
+    }
+    __syncthreads();
+    if (wk > 0) return;
+#pragma unroll
+    for (int g = 1; g < WK; ++g) {
+      const float* const other = lds + (g - 1) * (WM * WN * TM * TN * 1024) + wmn * (TM * TN * 1024) + lane;
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc[i][j][e] += other[((i * TN + j) * 16 + e) * 64];
+    }
+  }
+  const long col_base = n0 + wn * (BN / WN) + l32, row_base = m0 + wm * (BM / WM) + 4 * h;
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const long m = row_base + i * 32 + (e >> 2) * 8 + (e & 3), n = col_base + j * 32;
+        if ((C::M % BM == 0 || m < C::M) && (C::N % BN == 0 || n < C::N)) epi(batch, m, n, acc[i][j][e]);
+      }
+}
+
+// The f32 contraction of a configuration: staged where it names the waves' K groups.
+template <class C, class = void> struct HasWavesK { static constexpr bool value = false; };
+template <class C> struct HasWavesK<C, decltype((void)C::WAVES_K)> { static constexpr bool value = true; };
+
+template <class C, class Epi>
+__device__ __forceinline__ void mma32f(const float* __restrict__ A, const float* __restrict__ B, const Epi& epi) {
+  if constexpr (HasWavesK<C>::value) mma32f_staged<C>(A, B, epi);
+  else mma32f_direct<C>(A, B, epi);
+}
+
 }  // namespace gemm
+
+namespace split {
+
+// Sums of a contraction split along K: part[s][b][m][n] of SPLITS workgroup columns, added in split
+// order, then the epilogue. One thread per output.
+template <class C, class Epi>
+__device__ __forceinline__ void sum(const float* __restrict__ part, const Epi& epi) {
+  constexpr long MN = C::M * C::N, ALL = C::BATCH * MN;
+  const long step = (long)gridDim.x * blockDim.x;
+  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < ALL; i += step) {
+    float v = part[i];
+#pragma unroll
+    for (int s = 1; s < C::SPLITS; ++s) v += part[s * ALL + i];
+    epi(i / MN, i % MN / C::N, i % C::N, v);
+  }
+}
+
+}  // namespace split
 }  // namespace accy

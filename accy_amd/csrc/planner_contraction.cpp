@@ -25,6 +25,8 @@ int tile_group_m(int64_t m, int64_t n) {
 
 }  // namespace
 
+double Planner::macs(const GemmShape& gs) { return (double)gs.m * (double)gs.n * (double)gs.k * (double)gs.batch; }
+
 // ---- strided views: a value that is a transpose / rename / broadcast of a buffer ----
 
 bool Planner::gemm_shape(const Op& op, GemmShape& gs) const {
@@ -173,6 +175,65 @@ void Planner::pack_f32_operands(GemmShape& gs) {
   }
 }
 
+bool Planner::f32_direct(const GemmShape& gs) {
+  // 256 x 256 x 32 tiles, A K-contiguous and B N-contiguous with 16-byte aligned rows. Exact tiles, or
+  // M / N off the tile grid (N a multiple of 4) when the problem is large (2^27 multiply-adds and more).
+  // Large problems with another operand layout (an A stored M-contiguous, a B stored K-contiguous,
+  // rows not 16-byte aligned) copy that operand into a contiguous temporary first (pack_f32).
+  const bool exact = gs.m % 256 == 0 && gs.n % 256 == 0;
+  const bool large = macs(gs) >= (double)(1ull << 27);
+  if (gs.multi || !(exact || (large && gs.n % 4 == 0)) || gs.k % 32 != 0) return false;
+  return f32_layout_ok(gs) || large;
+}
+
+bool Planner::f32_staged_layout(const GemmShape& gs, bool& a_kc, bool& b_kc) {
+  auto operand = [](const Group& rows, const Group& k, bool& kc) {
+    auto whole = [](const Group& g) { return g.inner_str() == 1 && (g.single() || g.inner_ext() % 4 == 0); };
+    kc = whole(k);
+    return kc || whole(rows);
+  };
+  return operand(gs.ga_m, gs.ga_k, a_kc) && operand(gs.gb_n, gs.gb_k, b_kc);
+}
+
+// The staged f32 kernel's tile and K split by an estimate of its time in clocks: rounds of 256
+// workgroups x a tile's products (128 multiply-adds per CU and clock, of which the kernel reaches about
+// 76 %), or its operands' bytes at the 2800 B per clock that the L2s were seen to serve to 2048 waves and
+// more, plus the first loads of each round and, where K is split, another launch and the partials'
+// traffic. Measured (one box, us a pass; 128- / 64-wide tiles): 2048^3 167 / 182, 4096 x 1024 x
+// 4096 303 / 307, 1000^3 78 (33 in 4 splits) / 28, 300 x 4000 x 700 292 / 87 (30 in 4 splits), 16 x 4096 x 4096
+// 180 / 85 (19 as 32 x 64 tiles in 8 splits). The direct kernel's 256-wide tiles reach 137 TFLOP/s where
+// they fill every round and the staged ones 100-114, so the line between them lies at 0.8 full
+// rounds (2048^3, 64 tiles: 496 us).
+Planner::Tile Planner::f32_tile(const GemmShape& gs) {
+  bool a_kc, b_kc;
+  Tile best;
+  if (!f32_staged_layout(gs, a_kc, b_kc)) return best;
+  auto up = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+  const int64_t direct = up(gs.m, 256) * up(gs.n, 256) * gs.batch;
+  if (f32_direct(gs) && (double)direct >= 0.8 * 256.0 * (double)up(direct, 256)) return best;
+  static const Tile kTiles[] = {{128, 128, 4, 2, 1}, {64, 64, 2, 2, 2}, {32, 64, 1, 2, 2}, {64, 32, 2, 1, 2}};
+  double best_cost = 0;
+  for (Tile t : kTiles) {
+    const int64_t tiles = up(gs.m, t.bm) * up(gs.n, t.bn) * gs.batch, steps = up(gs.k, 32 * t.wk);
+    for (int splits = 1; splits <= 64 && (splits == 1 || steps / splits >= 4); splits *= 2) {
+      const int64_t per = up(steps, splits), used = up(steps, per);  // every split has a step
+      const double groups = (double)(tiles * used), rounds = (double)up(tiles * used, 256);
+      const double k = (double)per * 32 * t.wk;
+      const double waves = groups * t.wm * t.wn * t.wk;
+      const double products = rounds * t.bm * t.bn * k / (0.76 * 128.0);
+      const double bytes = groups * (t.bm + t.bn) * k * 4.0 / (2800.0 * std::min(1.0, waves / 2048.0));
+      double cost = std::max(products, bytes) + rounds * 2500.0;
+      if (used > 1) cost += 6000.0 + (double)used * (double)(gs.m * gs.n * gs.batch) * 8.0 / 2100.0;
+      if (!best.bm || cost < best_cost) {
+        best = t;
+        best.splits = (int)used;
+        best_cost = cost;
+      }
+    }
+  }
+  return best;
+}
+
 bool Planner::gemm_eligible(const Op& op, GemmShape& gs) const {
   if (!opt_.allow_gemm) return false;
   DType d = op.result.dtype;
@@ -181,15 +242,10 @@ bool Planner::gemm_eligible(const Op& op, GemmShape& gs) const {
   if (gs.m == 0 || gs.n == 0 || gs.k == 0) return false;
   if (gs.batch > 65535) return false;  // the batch index is gridDim.y, at most 65535 on gfx950
   if (d == DType::f32) {
-    // The f32 MFMA kernel: 256 x 256 x 32 tiles, A K-contiguous and B N-contiguous with 16-byte
-    // aligned rows. Exact tiles, or M / N off the tile grid (N a multiple of 4) when the problem is
-    // large (2^27 multiply-adds and more); other f32 contractions keep runCpu's serial k order.
-    // Large problems with another operand layout (an A stored M-contiguous, a B stored K-contiguous,
-    // rows not 16-byte aligned) copy that operand into a contiguous temporary first (pack_f32).
-    const bool exact = gs.m % 256 == 0 && gs.n % 256 == 0;
-    const bool large = (double)gs.m * (double)gs.n * (double)gs.k * (double)gs.batch >= (double)(1ull << 27);
-    if (gs.multi || !(exact || (large && gs.n % 4 == 0)) || gs.k % 32 != 0) return false;
-    return f32_layout_ok(gs) || large;
+    bool akc, bkc;
+    // Small and shallow contractions keep runCpu's serial k order: 962 x 67 x 130 takes 5.5 us there, a
+    // launch's time, but a fold of k = 1000 on few threads hundreds (1000^3: 262 us).
+    return f32_direct(gs) || ((gs.k >= 128 || macs(gs) >= (double)(1ull << 23)) && f32_staged_layout(gs, akc, bkc));
   }
   if (gs.multi) {
     int dm, dn;
@@ -254,7 +310,7 @@ void Planner::dot(uint32_t v) {
   }
   GemmShape gs;
   if (gemm_eligible(op, gs)) {
-    if (op.result.dtype == DType::f32 && !f32_layout_ok(gs)) pack_f32_operands(gs);
+    if (op.result.dtype == DType::f32 && f32_direct(gs) && !f32_layout_ok(gs)) pack_f32_operands(gs);
     std::vector<std::pair<uint32_t, GemmShape>> group;
     if (gemm_siblings(v, gs, group)) {
       gemm_group(group);
@@ -446,6 +502,14 @@ void Planner::gemm(uint32_t v, const GemmShape& gs, const OutStrides& os) {
   std::string nm = name("gemm", v);
   uint32_t target = v;
   std::unique_ptr<KernelWriter> w;
+  // Split along K: the contraction stores f32 sums of its part of K and split::sum adds them and runs the
+  // epilogue, whose kernel then reads no operand.
+  const Tile tile = d == DType::f32 ? f32_tile(gs) : Tile();
+  const bool split = tile.splits > 1;
+  auto operands = [&](KernelWriter& kw) {
+    kw.arg(gs.a.slot, false);
+    kw.arg(gs.b.slot, false);
+  };
   std::ostringstream epi;
   std::string table_members;  // a lookup-table epilogue's interface (gemm.h HasTable)
   // The fused epilogue (dot_general results only: os is their row-major layout).
@@ -453,8 +517,7 @@ void Planner::gemm(uint32_t v, const GemmShape& gs, const OutStrides& os) {
   if (op.kind == Kind::dot_general && rowmajor && epilogue_target(v, target)) {
     try {
       w.reset(new KernelWriter(g_, slots_, "i64_t"));
-      w->arg(gs.a.slot, false);
-      w->arg(gs.b.slot, false);
+      if (!split) operands(*w);
       const Type& rt = op.result;
       const size_t nb = op.lhs_batch.size();
       const size_t nlf = rt.rank() - nb - (g_.type(op.args[1]).rank() - op.rhs_batch.size() - op.rhs_contract.size());
@@ -526,27 +589,24 @@ void Planner::gemm(uint32_t v, const GemmShape& gs, const OutStrides& os) {
   }
   if (!w) {
     w.reset(new KernelWriter(g_, slots_, "i64_t"));
-    w->arg(gs.a.slot, false);
-    w->arg(gs.b.slot, false);
+    if (!split) operands(*w);
     int out = slots_.slot_of[v] >= 0 ? slots_.slot_of[v] : temp_slot(v);
     epi << "    " << w->store(out, cidx, d, "v") << "\n";
   }
-  const std::string a = w->arg(gs.a.slot, false), b = w->arg(gs.b.slot, false);
-  // Epilogue functor: every buffer of the kernel as a member named like the kernel parameter.
-  std::ostringstream members, inits;
-  {
-    std::string pl = w->params();
-    size_t start = 0;
-    while (start < pl.size()) {
-      size_t comma = pl.find(", ", start);
-      std::string decl = pl.substr(start, comma == std::string::npos ? std::string::npos : comma - start);
-      members << "  " << decl << ";\n";
-      size_t sp = decl.rfind(' ');
-      inits << (inits.tellp() > 0 ? ", " : "") << decl.substr(sp + 1);
-      if (comma == std::string::npos) break;
-      start = comma + 2;
-    }
+  // A split contraction's own kernel: operands and partial sums.
+  std::unique_ptr<KernelWriter> pw;
+  std::string partial;
+  if (split) {
+    pw.reset(new KernelWriter(g_, slots_, "i64_t"));
+    operands(*pw);
+    const int part = slots_.add(SlotInfo::Temp, -1, DType::f32, (uint64_t)tile.splits * (uint64_t)(gs.batch * gs.m * gs.n) * 4);
+    partial = pw->arg(part, true);
+    w->arg(part, false);
   }
+  KernelWriter& kw = split ? *pw : *w;
+  const std::string a = kw.arg(gs.a.slot, false), b = kw.arg(gs.b.slot, false);
+  // Epilogue functor: every buffer of the kernel as a member named like the kernel parameter.
+  const KernelWriter::Members members = w->members();
   // A 16-bit epilogue that reads buffers besides A, B and its output (a residual, a bias) goes
   // through LDS in whole row segments (gemm.h staged_epilogue; measured on C5's MLP-down: 224 ->
   // 219.7 us). A plain store does not (58.2 against 60.3 us staged for C5's q projection).
@@ -557,22 +617,39 @@ void Planner::gemm(uint32_t v, const GemmShape& gs, const OutStrides& os) {
   std::ostringstream src;
   KernelStep k;
   src << "#include \"gemm\"\n";
-  src << "struct Epi_" << nm << " {\n" << members.str()
+  src << "struct Epi_" << nm << " {\n" << members.decls
       << table_members << (staged ? "  static constexpr bool kStaged = true;\n" : "")
       << "  __device__ __forceinline__ void operator()(long b, long m, long n, float v) const {\n"
       << (target != v && table_members.empty() ? "    const float vv = " + round_to(d, "v") + ";\n" : "") << epi.str()
       << "  }\n};\n";
   if (d == DType::f32) {
-    // f32 on v_mfma_f32_32x32x2_f32: exact 256 x 256 x 32 tiles (gemm_eligible checked the layout).
+    // f32 on v_mfma_f32_32x32x2_f32: 256 x 256 x 32 tiles straight to LDS, or staged tiles (f32_tile).
     src << "struct Cfg_" << nm << " {\n"
-        << "  static constexpr long M = " << gs.m << ", N = " << gs.n << ", K = " << gs.k << ";\n"
+        << "  static constexpr long BATCH = " << gs.batch << ", M = " << gs.m << ", N = " << gs.n << ", K = " << gs.k << ";\n"
         << gs.ga_b.fn("a_b") << gs.ga_m.fn("a_m") << gs.ga_k.fn("a_k") << gs.gb_b.fn("b_b") << gs.gb_k.fn("b_k")
-        << gs.gb_n.fn("b_n") << "};\n";
-    src << "extern \"C\" __global__ void __launch_bounds__(256) " << nm << "(" << w->params() << ") {\n"
+        << gs.gb_n.fn("b_n");
+    if (tile.bm) {
+      bool a_kc = false, b_kc = false;
+      f32_staged_layout(gs, a_kc, b_kc);
+      src << "  static constexpr bool A_KC = " << (a_kc ? "true" : "false") << ", B_KC = " << (b_kc ? "true" : "false")
+          << ";\n  static constexpr int BM = " << tile.bm << ", BN = " << tile.bn << ", WAVES_M = " << tile.wm
+          << ", WAVES_N = " << tile.wn << ", WAVES_K = " << tile.wk << ", SPLITS = " << tile.splits << ";\n";
+    }
+    src << "};\n";
+    const int bm = tile.bm ? tile.bm : 256, bn = tile.bm ? tile.bn : 256;
+    k.block[0] = tile.bm ? 64u * (uint32_t)(tile.wm * tile.wn * tile.wk) : 256u;
+    k.grid[0] = (uint32_t)(((gs.m + bm - 1) / bm) * ((gs.n + bn - 1) / bn));
+    k.grid[2] = (uint32_t)tile.splits;
+    std::string functor = "Epi_" + nm + "{" + members.inits + "}";
+    if (split) {
+      src << "struct Part_" << nm << " {\n  float* __restrict__ p;\n"
+          << "  __device__ __forceinline__ void operator()(long b, long m, long n, float v) const {\n    p[(blockIdx.z * "
+          << gs.batch << "L + b) * " << gs.m * gs.n << "L + m * " << gs.n << "L + n] = v;\n  }\n};\n";
+      functor = "Part_" + nm + "{" + partial + "}";
+    }
+    src << "extern \"C\" __global__ void __launch_bounds__(" << k.block[0] << ") " << nm << "(" << kw.params() << ") {\n"
         << "  accy::gemm::mma32f<Cfg_" << nm << ">(" << a << " + " << gs.a.offset << "L, " << b << " + "
-        << gs.b.offset << "L, Epi_" << nm << "{" << inits.str() << "});\n}\n";
-    k.grid[0] = (uint32_t)(((gs.m + 255) / 256) * ((gs.n + 255) / 256));
-    k.block[0] = 256;
+        << gs.b.offset << "L, " << functor << ");\n}\n";
   } else {
     // 256 x 256 x 64 tiles; the wave grid (4 x 2 waves of 64 x 128, or 2 x 2 waves of 128 x 128)
     // can be overridden with ACCY_GEMM_WAVES=MxN for tuning.
@@ -621,7 +698,7 @@ void Planner::gemm(uint32_t v, const GemmShape& gs, const OutStrides& os) {
     int threads = dma ? 256 : WM * WN * 64;
     src << "extern \"C\" __global__ void __launch_bounds__(" << threads << ") " << nm << "(" << w->params() << ") {\n"
         << "  accy::gemm::" << (dma ? "mma16_dma" : "mma16") << "<Cfg_" << nm << ">(" << a << " + " << gs.a.offset
-        << "L, " << b << " + " << gs.b.offset << "L, Epi_" << nm << "{" << inits.str() << "});\n}\n";
+        << "L, " << b << " + " << gs.b.offset << "L, Epi_" << nm << "{" << members.inits << "});\n}\n";
     k.source = src.str();
     if (placeholder) {
       k.tuning_key = tuning_key("gemm", k.source, "m=" + std::to_string(gs.m) + ",n=" + std::to_string(gs.n) +
@@ -642,8 +719,21 @@ void Planner::gemm(uint32_t v, const GemmShape& gs, const OutStrides& os) {
   k.grid[1] = (uint32_t)gs.batch;
   k.klass = "gemm";
   k.label = "gemm:%" + std::to_string(v) + (target != v ? "+%" + std::to_string(target) : "");
-  k.algorithmic_flops = 2.0 * (double)gs.batch * (double)gs.m * (double)gs.n * (double)gs.k;
-  push(std::move(k), *w);
+  k.algorithmic_flops = 2.0 * macs(gs);
+  push(std::move(k), kw);
+  if (split) {
+    KernelStep sum;
+    sum.name = name("split_sum", v);
+    const std::string both = src.str();
+    sum.source = both.substr(0, both.find("struct Part_")) + "extern \"C\" __global__ void __launch_bounds__(256) " + sum.name + "(" +
+                 w->params() + ") {\n  accy::split::sum<Cfg_" + nm + ">(" + w->arg(pw->args.back(), false) + ", Epi_" + nm +
+                 "{" + members.inits + "});\n}\n";
+    sum.grid[0] = grid_for((uint64_t)(gs.batch * gs.m * gs.n), 256);
+    sum.block[0] = 256;
+    sum.klass = "gemm";
+    sum.label = "split_sum:%" + std::to_string(target);
+    push(std::move(sum), *w);
+  }
   if (target != v) {
     done_[v] = true;
     finish(target);

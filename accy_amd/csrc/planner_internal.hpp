@@ -393,6 +393,8 @@ class Planner {
 
   bool gemm_shape(const Op& op, GemmShape& gs) const;
 
+  static double macs(const GemmShape& gs);  // multiply-adds of the whole contraction
+
   // Direct-to-LDS tile sizes for the 16-bit kernel (0: not applicable).
   static int dma_rows(int64_t extent);
 
@@ -405,6 +407,22 @@ class Planner {
 
   // The f32 MFMA kernel's operand layouts: A K-contiguous, B N-contiguous, rows 16-byte aligned.
   static bool f32_layout_ok(const GemmShape& gs);
+
+  // Tile of a contraction kernel and the workgroups along K; bm = 0: none applies.
+  struct Tile {
+    int bm = 0, bn = 0, wm = 0, wn = 0, wk = 0, splits = 1;
+  };
+
+  // Whether the staged f32 kernel can read the operands: K or the row axis of each has stride 1 (in whole
+  // vectors of four, where several axes make up the group).
+  static bool f32_staged_layout(const GemmShape& gs, bool& a_kc, bool& b_kc);
+
+  // Tile and split of the staged f32 kernel; none (bm = 0) where the 256 x 256 direct-to-LDS kernel
+  // applies and spreads its tiles over the CUs.
+  static Tile f32_tile(const GemmShape& gs);
+
+  // Extents and layout the 256 x 256 direct-to-LDS f32 kernel takes (large problems are repacked for it).
+  static bool f32_direct(const GemmShape& gs);
 
   // Copies an f32 operand view (batch x R x C with strides sb, sr, sc from offset `off` of `slot`) into
   // a new contiguous temporary [batch][R][C] and returns its slot. One workgroup per 64 x 64 tile: when

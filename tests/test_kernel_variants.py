@@ -139,3 +139,63 @@ def test_scatter_add_of_gathered_updates(width):
            rng.integers(0, 30, 200).astype(np.int32), rng.standard_normal((30, width)).astype(np.float32)]
     for got, ref in zip(hip_run(prog, ins), oracle_run(prog, ins)):
         assert np.array_equal(got, ref)
+
+
+# ---- f32 contractions in staged tiles, split along K or not ----
+
+def contraction(dtype, m, k, n, layout="NN", batch=0, epilogue=False):
+    b_ = [("b", batch)] if batch else []
+    sa = b_ + ([("m", m), ("k", k)] if layout[0] == "N" else [("k", k), ("m", m)])
+    sb = b_ + ([("k", k), ("n", n)] if layout[1] == "N" else [("n", n), ("k", k)])
+
+    def body(b, a):
+        c = a[0].contract(a[1], "k")
+        return c.mul(b.full_float(T.Type(dtype, ()), 0.5)).add(a[2]) if epilogue else c
+    specs = [T.spec(dtype, *sa), T.spec(dtype, *sb)] + ([T.spec(dtype, n=n)] if epilogue else [])
+    return T.define("contraction", specs, body)
+
+
+def contraction_inputs(dtype, m, k, n, layout, batch, epilogue, seed):
+    rng = np.random.default_rng(seed)
+    b_ = (batch,) if batch else ()
+    a, b = rng.standard_normal(b_ + (m, k)), rng.standard_normal(b_ + (k, n))
+    a, b = to_f32(W.to_dtype(a, dtype), dtype).astype(np.float64), to_f32(W.to_dtype(b, dtype), dtype).astype(np.float64)
+    bias = to_f32(W.to_dtype(rng.standard_normal(n), dtype), dtype).astype(np.float64)
+    swap = lambda x, side: x if layout[side] == "N" else np.ascontiguousarray(np.swapaxes(x, -1, -2))
+    ins = [W.to_dtype(np.ascontiguousarray(swap(a, 0)), dtype), W.to_dtype(np.ascontiguousarray(swap(b, 1)), dtype)]
+    return ins + ([W.to_dtype(bias, dtype)] if epilogue else []), a, b, bias
+
+
+# tile remainders on both sides, rows shorter than a vector, K below a vector / a step and past it,
+# one output, one row, few rows (splits), batches
+F32_SHAPES = [(1, 128, 1, 0), (1, 4096, 300, 0), (3, 129, 2, 0), (31, 1023, 66, 0), (33, 130, 65, 0), (127, 131, 129, 0),
+              (962, 133, 130, 0), (3000, 3, 1001, 0), (2900, 1, 2899, 0), (64, 5000, 64, 0), (300, 2050, 70, 0),
+              (513, 1030, 770, 0), (5, 200, 37, 7), (130, 256, 66, 3)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", ["NN", "NT", "TN", "TT"])
+@pytest.mark.parametrize("shape", F32_SHAPES, ids=str)
+def test_staged_f32_contractions_within_the_summation_bound(shape, layout):
+    """|error| <= (K + 2) u sum|a b| for a sum of K products in any order (u = 2^-24), doubled for the
+    epilogue's product and sum."""
+    m, k, n, batch = shape
+    for epilogue in (False, True):
+        prog = contraction("f32", m, k, n, layout, batch, epilogue)
+        assert "WAVES_K" in hip.plan_source(prog)
+        ins, a, b, bias = contraction_inputs("f32", m, k, n, layout, batch, epilogue, m + k)
+        got = hip_run(prog, ins)[0].astype(np.float64)
+        ref, size = a @ b, np.abs(a) @ np.abs(b)
+        if epilogue:
+            ref, size = ref * 0.5 + bias, size + 2 * np.abs(bias)
+        assert np.all(np.abs(got - ref) <= 2 * (k + 2) * 2.0 ** -24 * size)
+
+
+def test_f32_contractions_choose_their_kernel_by_size():
+    plan = lambda m, k, n: hip.plan_source(contraction("f32", m, k, n))
+    assert "WAVES_K" not in plan(8192, 8192, 8192) and "mma32f<" in plan(8192, 8192, 8192)   # whole rounds of 256-wide tiles
+    assert "BM = 128" in plan(2048, 2048, 2048) and "SPLITS = 1" in plan(2048, 2048, 2048)
+    assert "BM = 64" in plan(1000, 1000, 1000) and "SPLITS = 1" in plan(1000, 1000, 1000)
+    assert "BM = 32" in plan(16, 4096, 4096) and "split_sum" in plan(16, 4096, 4096)
+    assert "accy::gemm::" not in plan(200, 100, 200)
+    hip.plan_source(contraction("f32", 16, 4096, 4096, epilogue=True), compile=True)
