@@ -52,6 +52,20 @@ template <typename I> __device__ __forceinline__ bool ld_i1(const u8_t* __restri
 // of a thread this way at the top of an iteration); alignment capped at the 16 bytes every buffer
 // base guarantees.
 template <typename T> struct alignas(4 * sizeof(T) < 16 ? 4 * sizeof(T) : 16) Quad { T v[4]; };
+// Four consecutive elements at any alignment of the element (rows whose length is not a multiple of
+// four start anywhere): one unaligned vector access, which gfx950 serves for global memory.
+template <typename T> struct __attribute__((packed, aligned(sizeof(T)))) QuadAny { T v[4]; };
+// 16-bit elements that a row kernel keeps between passes: two to a register, elements 2 i and 2 i + 1 of a
+// loaded vector in word i, and the value of the low (i even) or high one.
+template <template <typename> class Q> __device__ __forceinline__ u32_t pair_of(const Q<u16_t>& q, int i) {
+  return (u32_t)q.v[2 * i] | ((u32_t)q.v[2 * i + 1] << 16);
+}
+__device__ __forceinline__ float bf16_of(u32_t pair, int i) { return __builtin_bit_cast(float, i & 1 ? pair & 0xffff0000u : pair << 16); }
+__device__ __forceinline__ float f16_of(u32_t pair, int i) { return f16_to_f32((u16_t)(i & 1 ? pair >> 16 : pair)); }
+// Stops the compiler from carrying the unpacked values of one pass over to the next in twice the registers.
+__device__ __forceinline__ void opaque(u32_t& pair) { asm("" : "+v"(pair)); }
+// Sets the low (i even; the high one follows) or high half of a pair.
+__device__ __forceinline__ void put_half(u32_t& pair, int i, u16_t h) { pair = i & 1 ? pair | ((u32_t)h << 16) : (u32_t)h; }
 // The same four elements with the non-temporal hint, for data that a kernel reads exactly once (each
 // element by one workgroup, in one pass): the lines stream through the caches without displacing
 // lines that are reused, and a streaming read of HBM sustains about 7.0 TB/s instead of about 6.3.

@@ -219,8 +219,9 @@ std::string KernelWriter::load_at(int slot, const std::string& base, const std::
   }
 }
 
-std::string KernelWriter::quad_load(int slot, const std::string& var, const std::string& base, DType d, bool stream) {
-  const std::string q = std::string("accy::Quad<") + storage_type(d) + ">";
+std::string KernelWriter::quad_load(int slot, const std::string& var, const std::string& base, DType d, bool stream, bool any) {
+  const std::string q = std::string(any ? "accy::QuadAny<" : "accy::Quad<") + storage_type(d) + ">";
+  if (any) return "const " + q + " " + var + " = *(const " + q + "*)(" + arg(slot, false) + " + " + base + ");";
   if (stream) return "const " + q + " " + var + " = accy::ld_quad_stream(" + arg(slot, false) + " + " + base + ");";
   return "const " + q + " " + var + " = *(const " + q + "*)(" + arg(slot, false) + " + " + base + ");";
 }
@@ -232,6 +233,15 @@ std::string KernelWriter::quad_elem(const std::string& var, const std::string& i
     case DType::bf16: return "accy::bf16_to_f32(" + e + ")";
     case DType::i1: return "(" + e + " != 0)";
     default: return e;
+  }
+}
+
+std::string KernelWriter::bits(DType d, const std::string& v) {
+  switch (d) {
+    case DType::f16: return "accy::f32_to_f16(" + v + ")";
+    case DType::bf16: return "accy::f32_to_bf16(" + v + ")";
+    case DType::i1: return "(u8_t)(" + v + " ? 1 : 0)";
+    default: return v;
   }
 }
 

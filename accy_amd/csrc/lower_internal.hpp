@@ -65,9 +65,12 @@ class KernelWriter {
   std::string load_at(int slot, const std::string& base, const std::string& idx, DType d);
   // Declaration of an aligned four-element load of slot at element offset base (an accy::Quad), and
   // element idx of such a variable converted to the compute type.
-  std::string quad_load(int slot, const std::string& var, const std::string& base, DType d, bool stream = false);
+  // With `any`, at any alignment of the element (an accy::QuadAny).
+  std::string quad_load(int slot, const std::string& var, const std::string& base, DType d, bool stream = false, bool any = false);
   static std::string quad_elem(const std::string& var, const std::string& idx, DType d);
   std::string store(int slot, const std::string& off, DType d, const std::string& v);
+  // The storage value of a compute-domain value.
+  static std::string bits(DType d, const std::string& v);
   std::string tmp();
   std::string params() const;
   // The parameters as members of a functor that a kernel template takes, and their initialisers.

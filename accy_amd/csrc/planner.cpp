@@ -448,8 +448,7 @@ void Planner::scatter_add(uint32_t v) {
   const std::string o = w.arg(out, true), st = storage_type(d), quad = "accy::Quad<" + st + ">";
   std::string again, store;
   if (vec == 4) {
-    const std::string bits = d == DType::f16 ? "accy::f32_to_f16(v[u])" : d == DType::bf16 ? "accy::f32_to_bf16(v[u])"
-                             : d == DType::i1 ? "(u8_t)(v[u] ? 1 : 0)" : "v[u]";
+    const std::string bits = KernelWriter::bits(d, "v[u]");
     again = "    const " + quad + " q = *(const " + quad + "*)(" + o + " + " + at + ");\n#pragma unroll\n    for (int u = 0; u < VEC; ++u) v[u] = " +
             KernelWriter::quad_elem("q", "u", d) + ";\n";
     store = "    " + quad + " q;\n#pragma unroll\n    for (int u = 0; u < VEC; ++u) q.v[u] = " + bits + ";\n    *(" + quad + "*)(" + o + " + " + at + ") = q;\n";

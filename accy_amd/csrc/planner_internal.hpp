@@ -301,7 +301,14 @@ class Planner {
 
   KernelStep gen_row(const RowShape& rs, const RowKernel& rk, bool commit);
 
+  // What the last trial of a row kernel read: per leaf and per value of the whole row, the passes.
   std::map<std::string, std::set<int>> probe_use_;
+  std::map<uint32_t, std::set<int>> probe_values_;
+  // Values of the whole row that the pass given keeps in registers for later passes.
+  std::map<uint32_t, int> row_keep_;
+  // Every leaf that several passes of the last trial read is a row of 16-bit floats.
+  bool row_leaves_16bit() const;
+  void keep_row_values(const RowShape& rs, const RowKernel& rk, uint64_t per_thread, bool pairs);
 
   // ---- launch tuning ----
   size_t kernel_index() const;

@@ -308,9 +308,71 @@ std::vector<int> Planner::reduction_passes(const RowKernel& rk) const {
   return pass;
 }
 
+bool Planner::row_leaves_16bit() const {
+  for (const auto& [key, uses] : probe_use_) {
+    const DType d = plan_.slots[std::stoul(key)].dtype;  // keys are "slot|offset"
+    const bool row_major = quad_base(key.substr(key.find('|') + 1)).has_value();
+    if (uses.size() >= 2 && !(row_major && (d == DType::bf16 || d == DType::f16))) return false;
+  }
+  return true;
+}
+
+// Values of the whole row that cost more than a register to evaluate again (a transcendental, a division) and
+// that a later pass reads too: the pass that computes them first leaves them in registers, as a row
+// read by several passes is. The outermost such value is taken first (what it was computed from is
+// then often not read again), while the arrays live between two passes hold at most 64 registers per
+// thread. (Cross-entropy with its gradient, 2048 x 50257 bf16, whose gradient reads the exponentials: 217 us
+// with one row to a CU, evaluated twice or kept, as its loads, arithmetic and stores then take turns;
+// 151 us kept, in pairs, with two rows to a CU.)
+void Planner::keep_row_values(const RowShape& rs, const RowKernel& rk, uint64_t per_thread, bool pairs) {
+  auto costly = [&](uint32_t v) {
+    const Op& op = g_.ops[v];
+    if (op.kind == Kind::binary) return (Binary)op.code == Binary::div || (Binary)op.code == Binary::pow;
+    return op.kind == Kind::unary && (Unary)op.code != Unary::neg && (Unary)op.code != Unary::abs;
+  };
+  auto fits = [&]() {
+    int last = 0;
+    std::map<int, uint64_t> live;  // pass: registers holding values needed after it
+    auto count = [&](const std::set<int>& uses, bool bits16) {
+      for (int p = *uses.begin(); p < *uses.rbegin(); ++p) live[p] += pairs && bits16 ? per_thread / 2 : per_thread;
+      last = std::max(last, *uses.rbegin());
+    };
+    for (const auto& leaf : probe_use_) count(leaf.second, dtype_size(plan_.slots[std::stoul(leaf.first)].dtype) == 2);
+    for (const auto& kept : row_keep_) {
+      const auto uses = probe_values_.find(kept.first);
+      if (uses != probe_values_.end()) count(uses->second, dtype_size(g_.type(kept.first).dtype) == 2);
+    }
+    for (int p = 0; p < last; ++p)
+      if (live[p] > 64) return false;
+    return true;
+  };
+  std::set<uint32_t> refused;
+  for (int round = 0; round < 8; ++round) {
+    uint32_t best = 0;
+    bool found = false;
+    for (const auto& [v, uses] : probe_values_) {
+      if (uses.size() < 2 || row_keep_.count(v) || refused.count(v) || !costly(v)) continue;
+      best = v;  // in program order: the last is the outermost
+      found = true;
+    }
+    if (!found) return;
+    row_keep_[best] = *probe_values_.at(best).begin();
+    gen_row(rs, rk, false);
+    if (!fits()) {
+      row_keep_.erase(best);
+      refused.insert(best);
+      gen_row(rs, rk, false);
+    }
+  }
+}
+
 KernelStep Planner::gen_row(const RowShape& rs, const RowKernel& rk, bool commit) {
   uint64_t tn = prod(rs.T, 0, rs.T.size()), kn = prod(rs.K, 0, rs.K.size());
-  const uint32_t VEC = tn % 4 == 0 ? 4 : 1;
+  // Four consecutive elements per thread, also of rows whose length is no multiple of four (their vectors
+  // begin at any element). Shorter ones than one vector per lane of a wave keep one element per thread
+  // (30000 rows of 67 f16: 7.4 us against 9.0 with 17 of 64 lanes at work), rows of several axes too.
+  const bool flat = rs.T.size() == 1;
+  const uint32_t VEC = tn % 4 == 0 || (flat && tn >= 256) ? 4 : 1;
   uint64_t lanes = (tn + VEC - 1) / VEC;
   // Two waves per row: against one workgroup of four waves per row, C2's logsumexp went from 163-165 to
   // 159-161 µs and C1's tone from 58 to 56 µs on one box (four rounds), 162.0 -> 159.0 and 53.4 ->
@@ -325,14 +387,24 @@ KernelStep Planner::gen_row(const RowShape& rs, const RowKernel& rk, bool commit
   // slope over 8192 x 16384 took 694 us in two passes of a cached, fully unrolled row, 82 us in one.)
   const std::vector<int> pass_of = reduction_passes(rk);
   const int reduce_passes = 1 + *std::max_element(pass_of.begin(), pass_of.end());
+  if (commit) {
+    row_keep_.clear();
+    gen_row(rs, rk, false);  // what the passes read
+  }
+  // Elements of a row that a thread may keep in registers: 64. 16-bit rows too long for that are kept two
+  // elements to a register, up to 104 of them (with 128 the addresses and sums beside them spill:
+  // 4096 x 32000 bf16 cross-entropy took 264 us with 256 threads of 128, 174 us with 512 of 64), or 128
+  // where a row has no shorter share.
+  const bool pairs_ok = commit && VEC == 4 && flat && row_leaves_16bit();
+  auto keepable = [&](uint32_t threads) -> uint64_t { return !pairs_ok ? 64 : threads == 1024 ? 128 : 104; };
   size_t passes = (size_t)reduce_passes + (rk.full_vals.empty() ? 0 : 1);
-  // A row read by several passes is kept in registers when each thread holds at most 64 of its
+  // A row read by several passes is kept in registers when each thread holds at most 64 (128) of its
   // elements; a row too long for that with 128 threads takes 256, 512 or 1024 threads if that makes it
   // fit (read once instead of once per pass; four waves per SIMD still have 128 registers each).
-  if (passes >= 2 && E * VEC > 64) {
+  if (passes >= 2 && E * VEC > keepable(B)) {
     for (uint32_t wide : {256u, 512u, 1024u}) {
       const uint64_t e = (tn + (uint64_t)wide * VEC - 1) / ((uint64_t)wide * VEC);
-      if (e * VEC <= 64) {
+      if (e * VEC <= keepable(wide)) {
         B = wide;
         E = e;
         break;
@@ -349,9 +421,17 @@ KernelStep Planner::gen_row(const RowShape& rs, const RowKernel& rk, bool commit
     E = (tn + (uint64_t)B * VEC - 1) / ((uint64_t)B * VEC);
   }
   const std::string tid = R > 1 ? "(I)(threadIdx.x & 63)" : "(I)threadIdx.x";
-  bool unrolled = E * VEC <= 64;
+  bool unrolled = E * VEC <= (passes >= 2 ? keepable(B) : 64);
+  const bool pairs = pairs_ok && E * VEC > 64;  // (pairs cost an operation per element and pass)
   bool cache = unrolled && passes >= 2;
-  bool guard = tn % ((uint64_t)B * VEC) != 0;
+  // Where the threads' vectors do not cover the row exactly, the last iteration is written apart: its
+  // vectors past the end move back to the last four elements, and the elements another vector holds are
+  // skipped (c < cr). Every other iteration loads and stores whole vectors without a test. (Each
+  // element tested and loaded by itself, as a row of several axes still is: cross-entropy and its
+  // gradient over 2048 rows of 50257 bf16 took 681 us, now 151.)
+  const bool partial = tn % ((uint64_t)B * VEC) != 0, tail = partial && flat && VEC == 4, guard = partial && !tail;
+  const uint64_t whole = tail ? tn / ((uint64_t)B * VEC) : E;  // iterations without a test
+  const bool any = tn % 4 != 0;
   KernelWriter w(g_, slots_, itype());
   std::vector<std::string> kc = delinearize("row", rs.K);
   std::vector<std::string> tc = delinearize("c", rs.T);
@@ -365,8 +445,7 @@ KernelStep Planner::gen_row(const RowShape& rs, const RowKernel& rk, bool commit
   std::string decls;
   std::set<std::string> declared;
   if (commit) {
-    KernelStep probe = gen_row(rs, rk, false);
-    (void)probe;
+    if (cache) keep_row_values(rs, rk, E * VEC, pairs);
     leaf_use = probe_use_;
     int na = 0;
     for (auto& [key, uses] : leaf_use) {
@@ -377,6 +456,7 @@ KernelStep Planner::gen_row(const RowShape& rs, const RowKernel& rk, bool commit
     }
   }
   std::map<std::string, std::set<int>> use_record;
+  std::map<uint32_t, std::set<int>> value_use;
   // A load whose offset is `rest + c` (c the row's element index, rank-1 row) is written as
   // (ptr + rest + c0)[u] so that the VEC adjacent loads of one thread merge into one vector load.
   // The `rest` of an offset `(rest + c)` (empty optional when the offset has another form).
@@ -415,12 +495,15 @@ KernelStep Planner::gen_row(const RowShape& rs, const RowKernel& rk, bool commit
     const uint64_t elems = plan_.slots[(size_t)slot].bytes / dtype_size(d);
     return once && elems == kn * tn && mentions_row(off);
   };
+  auto reread = [](const std::string& array) {
+    return "      accy::opaque(" + array + "[e * 2]);\n      accy::opaque(" + array + "[e * 2 + 1]);\n";
+  };
   // The hoisted vector load of a leaf for this iteration (emitted once per pass), as the lane `u`.
   auto hoisted_elem = [&](int slot, const std::string& base, DType d, const std::string& key, bool stream) {
     auto hv = hoisted_var.find(key);
     if (hv == hoisted_var.end()) {
       std::string q = "q" + std::to_string(nquad++);
-      hoisted += "      " + w.quad_load(slot, q, base, d, stream) + "\n";
+      hoisted += "      " + w.quad_load(slot, q, base, d, stream, any) + "\n";
       hv = hoisted_var.emplace(key, q).first;
     }
     return KernelWriter::quad_elem(hv->second, "u", d);
@@ -442,10 +525,29 @@ KernelStep Planner::gen_row(const RowShape& rs, const RowKernel& rk, bool commit
       return true;
     }
     std::string elem = it->second + "[e * " + std::to_string(VEC) + " + u]";
+    const std::optional<std::string> pair_base = pairs && hoist && dtype_size(d) == 2 && is_float_domain(d) ? row_rest(off) : std::nullopt;
+    if (pair_base) {
+      // two 16-bit elements to a register, filled from the vector load at the top of the first pass's iteration
+      if (leaf_first[key] == cur_pass && !hoisted_var.count(key)) {
+        hoisted_elem(slot, *pair_base, d, key, streamed(slot, off, d, key));
+        for (int i = 0; i < 2; ++i)
+          hoisted += "      " + it->second + "[e * 2 + " + std::to_string(i) + "] = accy::pair_of(" + hoisted_var[key] + ", " + std::to_string(i) + ");\n";
+        if (declared.insert(key).second) decls += "    u32_t " + it->second + "[" + std::to_string(E * 2) + "];\n";
+      }
+      if (leaf_first[key] != cur_pass && !hoisted_var.count(key)) {
+        hoisted += reread(it->second);
+        hoisted_var.emplace(key, it->second);
+      }
+      out = w.tmp();
+      sc.out << sc.indent << "const float " << out << " = accy::" << (d == DType::bf16 ? "bf16_of(" : "f16_of(") << it->second
+             << "[e * 2 + (u >> 1)], u);\n";
+      return true;
+    }
     if (leaf_first[key] == cur_pass) {
       // The cache is filled by the first pass; a streamed leaf through the hoisted vector load.
-      std::optional<std::string> base = hoist && streamed(slot, off, d, key) ? row_rest(off) : std::nullopt;
-      sc.out << sc.indent << elem << " = " << (base ? hoisted_elem(slot, *base, d, key, true) : direct_load(slot, off, d))
+      const bool stream = streamed(slot, off, d, key);
+      std::optional<std::string> base = hoist && (stream || tail) ? row_rest(off) : std::nullopt;
+      sc.out << sc.indent << elem << " = " << (base ? hoisted_elem(slot, *base, d, key, stream) : direct_load(slot, off, d))
              << ";\n";
       if (declared.insert(key).second)
         decls += "    " + std::string(compute_type(d)) + " " + it->second + "[" + std::to_string(E * VEC) + "];\n";
@@ -464,9 +566,39 @@ KernelStep Planner::gen_row(const RowShape& rs, const RowKernel& rk, bool commit
     }
     const Op& op = g_.ops[vid];
     if (!is_inlinable(op.kind) && slots_.available(vid) < 0) throw NotFusable("value not produced yet");
+    if (coords == full && slots_.available(vid) < 0) {
+      const auto kept = row_keep_.find(vid);
+      if (kept != row_keep_.end() && cur_pass > kept->second) {
+        value_use[vid].insert(cur_pass);
+        const std::string array = "kept" + std::to_string(vid);
+        const DType d = g_.type(vid).dtype;
+        if (pairs && dtype_size(d) == 2 && is_float_domain(d) && hoisted_var.emplace(array, array).second) hoisted += reread(array);
+        if (pairs && dtype_size(d) == 2 && is_float_domain(d))
+          out = std::string(d == DType::bf16 ? "accy::bf16_of(" : "accy::f16_of(") + array + "[e * 2 + (u >> 1)], u)";
+        else
+          out = array + "[e * " + std::to_string(VEC) + " + u]";
+        return true;
+      }
+      value_use[vid].insert(cur_pass);
+    }
     return false;
   };
   std::ostringstream body;
+  // The values kept for later passes, once the pass that computes them has done so.
+  auto emit_kept = [&](std::ostringstream& to, Scope& sc) {
+    for (const auto& [vid, pass] : row_keep_) {
+      if (pass != cur_pass) continue;
+      const std::string x = w.value(vid, full, sc), array = "kept" + std::to_string(vid);
+      const DType d = g_.type(vid).dtype;
+      if (pairs && dtype_size(d) == 2 && is_float_domain(d)) {  // rounded already: its 16 bits hold it exactly
+        to << sc.indent << "accy::put_half(" << array << "[e * 2 + (u >> 1)], u, " << KernelWriter::bits(d, x) << ");\n";
+        decls += "    u32_t " + array + "[" + std::to_string(E * 2) + "] = {};\n";
+        continue;
+      }
+      to << sc.indent << array << "[e * " << VEC << " + u] = " << x << ";\n";
+      decls += "    " + std::string(compute_type(d)) + " " + array + "[" + std::to_string(E * VEC) + "];\n";
+    }
+  };
   // Element loop: fully unrolled when the thread's elements are cached in registers across passes;
   // otherwise unrolled by a few iterations (all of them would keep every hoisted load live at once).
   // Launch candidates when not cached: the unroll factor (first = default); the source carries a
@@ -475,25 +607,30 @@ KernelStep Planner::gen_row(const RowShape& rs, const RowKernel& rk, bool commit
   const std::vector<int> unroll_candidates =
       cache ? std::vector<int>{0} : (unrolled ? std::vector<int>{4, 2, 1, 8} : std::vector<int>{2, 1, 4});
   std::string unroll = cache ? "#pragma unroll\n" : kUnrollMark;
-  std::string loop_head_a, loop_head_b;
-  {
-    std::ostringstream la, lb;
-    la << unroll << "    for (int e = 0; e < " << E << "; ++e) {\n"
-       << "      const I c0 = ((I)e * " << B << " + " << tid << ") * " << VEC << ";\n";
-    lb << "#pragma unroll\n"
-       << "      for (int u = 0; u < " << VEC << "; ++u) {\n"
-       << "        const I c = c0 + u;\n";
-    if (guard) lb << "        if (c < (I)" << tn << ") {\n";
-    loop_head_a = la.str();
-    loop_head_b = lb.str();
-  }
-  // One element loop: head, the pass's hoisted loads, per-element code, tail.
-  auto emit_loop = [&](const std::string& inner_code, const std::string& tail) {
-    body << loop_head_a << hoisted << loop_head_b << inner_code << tail;
+  // A wide row's passes each compute their own offsets (carried from pass to pass they would take as many
+  // registers as the row: 316 bytes of scratch for the loss above).
+  const bool wide = cache && B >= 256;
+  const std::string first_elem = "((I)e * " + std::to_string(B) + " + " + tid + ") * " + std::to_string(VEC);
+  const std::string vec_elem = wide ? "(I)e * " + std::to_string(B * VEC) + " + t0" : first_elem;
+  const std::string head = "      const I c0 = " + vec_elem + ";\n";
+  const std::string elements = "#pragma unroll\n      for (int u = 0; u < " + std::to_string(VEC) + "; ++u) {\n        const I c = c0 + u;\n";
+  // One element loop: the pass's hoisted loads, the per-element code and what follows a vector's elements;
+  // then the last iteration with its own per-element code.
+  auto emit_loop = [&](const std::string& inner_code, const std::string& after, const std::string& tail_code) {
+    if (wide)
+      body << "    {\n    u32_t t = threadIdx.x * " << VEC << "u;\n    accy::opaque(t);\n    const I t0 = (I)(t & " << B * VEC - 1 << "u);\n";
+    if (whole)
+      body << unroll << "    for (int e = 0; e < " << whole << "; ++e) {\n" << head << hoisted << elements
+           << (guard ? "        if (c < (I)" + std::to_string(tn) + ") {\n" : "") << inner_code
+           << (guard ? "        }\n      }\n" : "      }\n") << after
+           << (wide && cur_pass > 0 ? "      __builtin_amdgcn_sched_barrier(0);\n" : "") << "    }\n";
+    if (tail)
+      body << "    {\n      const int e = " << whole << ";\n      const I cr = " << vec_elem << ", c0 = cr < (I)" << tn - VEC << " ? cr : (I)" << tn - VEC << ";\n"
+           << hoisted << elements << "        if (c >= cr) {\n" << tail_code << "        }\n      }\n    }\n";
+    if (wide) body << "    }\n";
     hoisted.clear();
     hoisted_var.clear();
   };
-  std::string loop_tail = guard ? "        }\n      }\n    }\n" : "      }\n    }\n";
   std::string lds_decl;
   for (cur_pass = 0; cur_pass < reduce_passes; ++cur_pass) {
     std::ostringstream ib;
@@ -520,7 +657,8 @@ KernelStep Planner::gen_row(const RowShape& rs, const RowKernel& rk, bool commit
       std::string x = w.value(op.args[0], full, inner);
       ib << inner.indent << acc << " = " << fold_step(d, r, acc, x) << ";\n";
     }
-    emit_loop(ib.str(), loop_tail);
+    emit_kept(ib, inner);
+    emit_loop(ib.str(), "", ib.str());
     for (size_t j = 0; j < rk.reduces.size(); ++j) {
       if (pass_of[j] != cur_pass) continue;
       const Op& op = g_.ops[rk.reduces[j]];
@@ -552,22 +690,44 @@ KernelStep Planner::gen_row(const RowShape& rs, const RowKernel& rk, bool commit
     cur_pass = reduce_passes;
     std::ostringstream ib;
     Scope sc(ib, guard ? "          " : "        ");
-    for (uint32_t v : rk.full_vals) {
+    std::string after, tail_stores;
+    for (size_t i = 0; i < rk.full_vals.size(); ++i) {
+      const uint32_t v = rk.full_vals[i];
       std::string x = w.value(v, full, sc);
-      if (commit) ib << sc.indent << w.store(slots_.slot_of[v], "row * (I)" + std::to_string(tn) + " + c", g_.type(v).dtype, x) << "\n";
+      if (!commit) continue;
+      const DType d = g_.type(v).dtype;
+      const std::string store = sc.indent + w.store(slots_.slot_of[v], "row * (I)" + std::to_string(tn) + " + c", d, x) + "\n";
+      if (!tail) {
+        ib << store;
+        continue;
+      }
+      // whole vectors are stored at once after their elements, the last iteration's element by element
+      const std::string q = "out" + std::to_string(i), type = std::string(any ? "accy::QuadAny<" : "accy::Quad<") + storage_type(d) + ">";
+      ib << sc.indent << q << ".v[u] = " << KernelWriter::bits(d, x) << ";\n";
+      hoisted += "      " + type + " " + q + ";\n";
+      after += "      *(" + type + "*)(" + w.arg(slots_.slot_of[v], true) + " + row * (I)" + std::to_string(tn) + " + c0) = " + q + ";\n";
+      tail_stores += store;
     }
-    emit_loop(ib.str(), loop_tail);
+    emit_loop(ib.str(), after, ib.str() + tail_stores);
   }
   probe_use_ = use_record;
+  probe_values_ = value_use;
   KernelStep k;
   if (!commit) return k;
+  row_keep_.clear();
   std::string nm = name("row", rk.reduces[0]);
   std::ostringstream src;
-  src << "extern \"C\" __global__ void __launch_bounds__(" << B * R << ") " << nm << "(" << w.params() << ") {\n"
+  // A wide row kept in registers: four waves per SIMD, so that two workgroups of 512 threads share a CU and
+  // one computes while the other loads or stores.
+  src << "extern \"C\" __global__ void __launch_bounds__(" << B * R << ") "
+      << (wide ? "__attribute__((amdgpu_waves_per_eu(4))) " : "") << nm << "(" << w.params() << ") {\n"
       << "  typedef " << w.itype << " I;\n" << w.align_hints() << lds_decl;
   if (R > 1)
     src << "  for (I row = (I)blockIdx.x * " << R << " + (I)(threadIdx.x >> 6); row < (I)" << kn
         << "; row += (I)gridDim.x * " << R << ") {\n";
+  else if (wide && kn <= (1u << 20))
+    // one row per workgroup; written as a loop, every vector's address is carried across it in registers
+    src << "  {\n    const I row = blockIdx.x;\n";
   else
     src << "  for (I row = blockIdx.x; row < (I)" << kn << "; row += gridDim.x) {\n";
   src << decls << body.str() << "  }\n}\n";

@@ -28,7 +28,8 @@ def statistics(b, a):
 def test_independent_reductions_share_a_pass(rows, cols, passes):
     src = hip.plan_source(T.define("stats", [T.spec("f32", r=rows, c=cols)], statistics))
     if passes:   # one element loop per dependency level, and one for the full row
-        assert src.count("__global__") == 1 and src.count("for (int e = 0;") == passes
+        loops = max(src.count("for (int e = 0;"), src.count("const I cr ="))   # whole iterations, the last one
+        assert src.count("__global__") == 1 and loops == passes
 
 
 @pytest.mark.gpu
@@ -199,3 +200,40 @@ def test_f32_contractions_choose_their_kernel_by_size():
     assert "BM = 32" in plan(16, 4096, 4096) and "split_sum" in plan(16, 4096, 4096)
     assert "accy::gemm::" not in plan(200, 100, 200)
     hip.plan_source(contraction("f32", 16, 4096, 4096, epilogue=True), compile=True)
+
+
+# ---- rows whose length is no multiple of four, or that the threads' vectors do not cover exactly ----
+
+def softmax_rows(b, a):
+    x, gain, bias = a
+    e = x.sub(x.max("c")).exp()
+    p = e.div(e.sum("c"))
+    return [p.mul(gain).add(bias), x.mul(x).sum("c"), p.max("c")]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("rows,cols", [(3, 65), (1100, 67), (1030, 258), (5, 510), (4, 513), (2, 2047), (1, 30001), (2, 50000)])
+def test_ragged_rows_match_the_oracle(rows, cols, dtype):
+    """A row input, a vector broadcast over the rows, a scalar broadcast over the columns, a whole-row
+    output. Sums of positive terms in another order: 1e-5 of the value in f32; one rounding step of each of
+    the 16-bit operations that read such a sum (division, product, sum)."""
+    prog = T.define("ragged", [T.spec(dtype, r=rows, c=cols), T.spec(dtype, c=cols), T.spec(dtype, r=rows)], softmax_rows)
+    assert hip.plan_source(prog).count("__global__") == 1
+    rng = np.random.default_rng(cols)
+    ins = [W.to_dtype(x, dtype) for x in (rng.standard_normal((rows, cols)), 1 + rng.random(cols), 1 + rng.random(rows))]
+    tol = {"f32": 1e-5, "bf16": 3 * 2.0 ** -7, "f16": 3 * 2.0 ** -10}[dtype]
+    for got, ref in zip(hip_run(prog, ins), oracle_run(prog, ins)):
+        g, r = to_f32(got, dtype).astype(np.float64), to_f32(ref, dtype).astype(np.float64)
+        assert np.all(np.abs(g - r) <= tol * np.abs(r))
+
+
+@pytest.mark.gpu
+def test_ragged_rows_write_only_their_own_elements():
+    """Exact integer rows of 67 and 70 next to each other: every element of the full-row output, and the
+    sums, bit for bit."""
+    for rows, cols in [(1, 67), (1300, 67), (9, 70), (3, 4099)]:
+        prog = T.define("rows", [T.spec("i32", r=rows, c=cols)], lambda b, a: [a[0].sub(a[0].sum("c")), a[0].max("c")])
+        x = np.random.default_rng(cols).integers(-1000, 1000, (rows, cols)).astype(np.int32)
+        for got, ref in zip(hip_run(prog, [x]), oracle_run(prog, [x])):
+            assert np.array_equal(got, ref)
