@@ -339,8 +339,10 @@ struct Strided {
 // RMAX is the operand's row extent (M or N). When it is not a multiple of the tile the last tile
 // reaches past it: a row past the end reads the last row (KC), a 16-byte chunk past the end of a k
 // row reads the last chunk (RMAX a multiple of 8), so every load stays inside the operand; those
-// rows and columns only feed outputs that the epilogue does not store.
-template <int ROWS, bool KC, class O, long RMAX>
+// rows and columns only feed outputs that the epilogue does not store. KMAX is the contraction's
+// extent: where it is no multiple of 32, loads past it read the last row (the last 8 of k) again, and
+// zero_k_tail clears what they brought before it is used.
+template <int ROWS, bool KC, class O, long RMAX, long KMAX>
 __device__ __forceinline__ void dma_part(const u16_t* __restrict__ base, long r0, long k0, u16_t* lds, int wave,
                                          int lane, int i) {
   constexpr int INSTRS = ROWS * 64 / 1024;
@@ -354,7 +356,13 @@ __device__ __forceinline__ void dma_part(const u16_t* __restrict__ base, long r0
     const int row = 16 * gi + 4 * (lane >> 4) + (q >> 2);
     long r = r0 + row;
     if constexpr (RAGGED) r = r < RMAX ? r : RMAX - 1;
-    src = base + O::row(r) + O::k(k0) + 8 * (q & 3);
+    if constexpr (KMAX % 32 == 0) {
+      src = base + O::row(r) + O::k(k0) + 8 * (q & 3);
+    } else {
+      static_assert(KMAX % 8 == 0 && KMAX >= 8, "whole 16-byte chunks");
+      const long k = k0 + 8 * (q & 3);
+      src = base + O::row(r) + O::k(k <= KMAX - 8 ? k : KMAX - 8);
+    }
   } else {
     static_assert(!RAGGED || RMAX % 8 == 0, "whole 16-byte chunks");
     constexpr int ROWB = ROWS * 2;    // bytes per k row
@@ -363,22 +371,41 @@ __device__ __forceinline__ void dma_part(const u16_t* __restrict__ base, long r0
     const int row = RPI * gi + lane / LPR;
     const int p = lane % LPR;
     const int u = (p >> 1) ^ tr_swizzle(row);
+    long k = k0 + row;
+    if constexpr (KMAX % 32 != 0) k = k < KMAX ? k : KMAX - 1;
     if constexpr (RAGGED) {
       long col = r0 + 16 * u + 8 * (p & 1);
       col = col <= RMAX - 8 ? col : RMAX - 8;
-      src = base + O::k(k0 + row) + O::row(col);
+      src = base + O::k(k) + O::row(col);
     } else {
       // whole tiles lie inside one contiguous run of the row group: affine there
-      src = base + O::k(k0 + row) + O::row(r0) + 16 * u + 8 * (p & 1);
+      src = base + O::k(k) + O::row(r0) + 16 * u + 8 * (p & 1);
     }
   }
   dma16(src, (ACCY_LDS void*)(lds + gi * 512));
 }
 
-template <int ROWS, bool KC, class O, long RMAX>
+template <int ROWS, bool KC, class O, long RMAX, long KMAX>
 __device__ __forceinline__ void dma_tile(const u16_t* __restrict__ base, long r0, long k0, u16_t* lds, int wave, int lane) {
 #pragma unroll
-  for (int i = 0; i < ROWS * 64 / 1024 / 4; ++i) dma_part<ROWS, KC, O, RMAX>(base, r0, k0, lds, wave, lane, i);
+  for (int i = 0; i < ROWS * 64 / 1024 / 4; ++i) dma_part<ROWS, KC, O, RMAX, KMAX>(base, r0, k0, lds, wave, lane, i);
+}
+
+// Clears k = VALID .. 31 of a stage (the same layouts as dma_part): 256 threads, 16 bytes at a time. A
+// stage past K keeps products of the last row's values, which must add nothing (0 x inf would be NaN, so
+// both operands are cleared).
+template <int ROWS, bool KC, int VALID>
+__device__ __forceinline__ void zero_k_tail(u16_t* lds, int tid) {
+  constexpr int CHUNKS = KC ? ROWS * (4 - VALID / 8) : (32 - VALID) * ROWS / 8;
+  static_assert(!KC || VALID % 8 == 0, "whole 16-byte chunks");
+  for (int i = tid; i < CHUNKS; i += 256) {
+    u16_t* p = lds + VALID * ROWS + 8 * i;
+    if constexpr (KC) {
+      const int r = i % ROWS, line = r >> 2, slot = ((r & 3) << 2) | (VALID / 8 + i / ROWS);
+      p = lds + line * 128 + ((slot ^ (line & 3)) << 3);
+    }
+    *(u32x4*)p = u32x4{0, 0, 0, 0};
+  }
 }
 
 // Fragment of 32 rows (M or N) x 16 k for one MFMA, read from a stage.
@@ -408,6 +435,11 @@ __device__ __forceinline__ u32x4 frag(const u16_t* lds, int row0, int s, int lan
   }
 }
 
+// Workgroups along K (C::SPLITS where the configuration sets it, else 1): split z takes an equal share of
+// the K steps.
+template <class C, class = void> struct Splits { static constexpr int value = 1; };
+template <class C> struct Splits<C, decltype((void)C::SPLITS)> { static constexpr int value = C::SPLITS; };
+
 // The fragments of one 16-deep sub-step for this wave's (BM / 2) x (BN / 2) sub-tile: TM A
 // fragments, then TN B fragments (fragment q of the set is loaded by load_one(q)).
 template <class C>
@@ -435,7 +467,9 @@ struct Frags {
 // second half runs the MFMAs of f1 with the reads of tile kt + 1's first sub-step (the next f0)
 // between them. The explicit interleave keeps at most one sub-step of LDS reads in flight, so the
 // compiler's lgkmcnt waits stay exact instead of draining the counter.
-template <class C, int STAGE, int WAIT, bool ISSUE, bool HAS_NEXT>
+// LAST_NEXT: the next tile is the contraction's last, whose k past the end is cleared (in the last
+// split).
+template <class C, int STAGE, int WAIT, bool ISSUE, bool HAS_NEXT, bool LAST_NEXT = false>
 struct DmaStep {
   static constexpr int S = C::STAGES, NEXT = (STAGE + S - 1) % S;
   template <class Acc>
@@ -457,9 +491,9 @@ struct DmaStep {
         if (k < NF) {
           f1.load_one(k, as[STAGE], bs[STAGE], 1, lane, wm, wn);
         } else if (k - NF < DA) {
-          dma_part<C::BM, C::A_KC, AOff<C>, C::M>(Ab, m0, (kt + S - 1) * 32, as[NEXT], wave, lane, k - NF);
+          dma_part<C::BM, C::A_KC, AOff<C>, C::M, C::K>(Ab, m0, (kt + S - 1) * 32, as[NEXT], wave, lane, k - NF);
         } else {
-          dma_part<C::BN, C::B_KC, BOff<C>, C::N>(Bb, n0, (kt + S - 1) * 32, bs[NEXT], wave, lane, k - NF - DA);
+          dma_part<C::BN, C::B_KC, BOff<C>, C::N, C::K>(Bb, n0, (kt + S - 1) * 32, bs[NEXT], wave, lane, k - NF - DA);
         }
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -467,6 +501,13 @@ struct DmaStep {
     if constexpr (HAS_NEXT) {
       wait_vmcnt<WAIT>();
       lds_reads_done_barrier();
+    }
+    if constexpr (LAST_NEXT && C::K % 32 != 0) {
+      if (Splits<C>::value == 1 || (kt + 2) * 32 >= C::K) {
+        zero_k_tail<C::BM, C::A_KC, C::K % 32>(as[(STAGE + 1) % S], wave * 64 + lane);
+        zero_k_tail<C::BN, C::B_KC, C::K % 32>(bs[(STAGE + 1) % S], wave * 64 + lane);
+        lds_reads_done_barrier();
+      }
     }
 #pragma unroll
     for (int t = 0; t < NM; ++t) {
@@ -498,7 +539,7 @@ struct DmaTail {
     constexpr int LEFT = S - 2 - J;
     constexpr int WAIT = LEFT > 0 ? LEFT * PER : 0;
     constexpr bool HAS_NEXT = J < S - 1;
-    DmaStep<C, I % S, WAIT, ISSUE, HAS_NEXT>::run(Ab, Bb, m0, n0, kt, as, bs, f0, acc, wave, lane, wm, wn);
+    DmaStep<C, I % S, WAIT, ISSUE, HAS_NEXT, J == S - 2>::run(Ab, Bb, m0, n0, kt, as, bs, f0, acc, wave, lane, wm, wn);
     if constexpr (HAS_NEXT) DmaTail<C, I + 1, R, PER>::run(Ab, Bb, m0, n0, kt + 1, as, bs, f0, acc, wave, lane, wm, wn);
   }
 };
@@ -574,8 +615,8 @@ __device__ __forceinline__ void staged_epilogue(const f32x16 (&acc)[TM][TN], u16
   }
 }
 
-// Requires K % 32 == 0 with at least STAGES K steps and 16-byte aligned rows (M or N not a multiple
-// of the tile: see dma_part);
+// Requires at least STAGES K steps of 32 per split and 16-byte aligned rows (M, N or K not a multiple of
+// the tile: see dma_part);
 // 256 threads (2 x 2 waves). LDS: STAGES x (BM + BN) x 64 bytes (STAGES = 4 with a 256 x 256 tile:
 // 128 KiB, one workgroup per CU; 3 with 256 x 128: 72 KiB, two per CU when the kernel is compiled for
 // two waves per SIMD, so that one workgroup's epilogue runs beside the other's matrix work).
@@ -584,8 +625,9 @@ __device__ __forceinline__ void mma16_dma_tile(const u16_t* __restrict__ A, cons
                                                long tm, long tn) {
   constexpr int BM = C::BM, BN = C::BN, S = C::STAGES;
   constexpr int TM = BM / 64, TN = BN / 64;
-  constexpr long TILES_M = (C::M + BM - 1) / BM, TILES_N = (C::N + BN - 1) / BN, KT = C::K / 32;
-  static_assert(C::K % 32 == 0, "whole K steps");
+  constexpr long TILES_M = (C::M + BM - 1) / BM, TILES_N = (C::N + BN - 1) / BN, KT = (C::K + 31) / 32 / Splits<C>::value;
+  static_assert((C::K + 31) / 32 % Splits<C>::value == 0, "equal splits");
+  static_assert(C::K % 32 == 0 || S >= 3, "the step before the last drains");
   static_assert(S >= 2 && S <= 4 && KT >= S, "two to four stages, at least one K step per stage");
   constexpr int PER = (BM * 64 / 1024) / 4 + (BN * 64 / 1024) / 4;  // DMA instructions per wave per step
   static_assert((S - 2) * PER < 64, "vmcnt range");
@@ -617,10 +659,11 @@ __device__ __forceinline__ void mma16_dma_tile(const u16_t* __restrict__ A, cons
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] = f32x16{};
 
+  long kt = Splits<C>::value > 1 ? (long)blockIdx.z * KT : 0;
 #pragma unroll
   for (int s = 0; s < S - 1; ++s) {
-    dma_tile<BM, C::A_KC, AOff<C>, C::M>(Ab, m0, s * 32, as[s], wave, lane);
-    dma_tile<BN, C::B_KC, BOff<C>, C::N>(Bb, n0, s * 32, bs[s], wave, lane);
+    dma_tile<BM, C::A_KC, AOff<C>, C::M, C::K>(Ab, m0, (kt + s) * 32, as[s], wave, lane);
+    dma_tile<BN, C::B_KC, BOff<C>, C::N, C::K>(Bb, n0, (kt + s) * 32, bs[s], wave, lane);
   }
   // Tile 0 complete everywhere (tiles 1 .. S - 2 may still be in flight), then its first sub-step.
   Frags<C> f0;
@@ -632,7 +675,6 @@ __device__ __forceinline__ void mma16_dma_tile(const u16_t* __restrict__ A, cons
   // G full groups of S, then the tail.
   constexpr long ISSUING = KT - S + 1, G = ISSUING / S;
   constexpr int R = (int)(ISSUING % S);
-  long kt = 0;
   for (long g = 0; g < G; ++g, kt += S) DmaGroup<C, 0, PER>::run(Ab, Bb, m0, n0, kt, asc, bsc, f0, acc, wave, lane, wm, wn);
   DmaTail<C, 0, R, PER>::run(Ab, Bb, m0, n0, kt, asc, bsc, f0, acc, wave, lane, wm, wn);
 

@@ -84,7 +84,7 @@ bool Planner::dma_operand(const Group& rows, const Group& k, const Group& batch,
     return true;
   };
   if (!aligned8(batch, false)) return false;
-  if (k.inner_str() == 1 && k.inner_ext() % 32 == 0 && aligned8(k, true) && aligned8(rows, false)) {
+  if (k.inner_str() == 1 && k.inner_ext() % (k.single() ? 8 : 32) == 0 && aligned8(k, true) && aligned8(rows, false)) {
     kc = true;
     return true;
   }
@@ -96,16 +96,18 @@ bool Planner::dma_operand(const Group& rows, const Group& k, const Group& batch,
 }
 
 bool Planner::dma_eligible(const GemmShape& gs, int& dm, int& dn, bool& a_kc, bool& b_kc) const {
-  // whole K steps of 32, at least as many as pipeline stages
-  if (gs.k % 32 != 0 || gs.k < 128 || std::getenv("ACCY_GEMM_NO_DMA")) return false;
+  // at least as many K steps of 32 as pipeline stages; a last one that K does not fill only for
+  // single-axis groups (the kernel clears what its loads read past K)
+  if (gs.k < 128 || (gs.k % 32 != 0 && gs.multi) || std::getenv("ACCY_GEMM_NO_DMA")) return false;
   dm = dma_rows(gs.m);
   dn = dma_rows(gs.n);
   if (dm && dn)
     return dma_operand(gs.ga_m, gs.ga_k, gs.ga_b, gs.a.offset, dm, a_kc) &&
            dma_operand(gs.gb_n, gs.gb_k, gs.gb_b, gs.b.offset, dn, b_kc);
-  // M or N not a multiple of 128: single-axis groups with extents a multiple of 8, tiles that reach
-  // past the end (the kernel clamps those loads to the last row / chunk and stores only in range).
-  if (gs.multi || gs.m % 8 != 0 || gs.n % 8 != 0) return false;
+  // M or N not a multiple of 128: single-axis groups, tiles that reach past the end (the kernel clamps those
+  // loads to the last row / chunk, so a row-contiguous operand's extent is a multiple of 8, and stores
+  // only in range).
+  if (gs.multi) return false;
   dm = dm ? dm : (gs.m > 128 ? 256 : 128);
   dn = dn ? dn : (gs.n > 128 ? 256 : 128);
   return dma_operand(gs.ga_m, gs.ga_k, gs.ga_b, gs.a.offset, 8, a_kc) &&
@@ -227,6 +229,46 @@ Planner::Tile Planner::f32_tile(const GemmShape& gs) {
       if (!best.bm || cost < best_cost) {
         best = t;
         best.splits = (int)used;
+        best_cost = cost;
+      }
+    }
+  }
+  return best;
+}
+
+// The direct-to-LDS kernel's tile and K split by an estimate of its time in microseconds: a CU with its
+// tile of 256 x 256, 128 x 256, 256 x 128 or 128 x 128 does 5.4, 4.6, 3.9 or 4.05 TFLOP/s (4096^3, every CU at
+// work: 105, 117, 139, 135 us) and up to 1.45 times that where few CUs share the board's power, a round of 256 of
+// them starts and drains in about 4 us, and a split costs a launch and the partials' traffic. Measured (one
+// box, us a pass, 256 x 256 against 128 x 128): 2048 x 8192 x 2048 134 / 66, 3000 x 2048 x 2048 45.6 / 34.1 (128 x 256:
+// 31.9), 1024^3 21.4 / 9.7, 512 x 4096 x 4096 69.6 / 30.8, 16 x 2048 x 8192 22.4 / 13.1.
+Planner::Tile Planner::dma_tile(const GemmShape& gs) {
+  auto up = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+  static const struct { int bm, bn; double rate; } kTiles[] = {{256, 256, 5.4}, {128, 256, 4.6}, {256, 128, 3.9}, {128, 128, 4.05}};
+  const int64_t steps = up(gs.k, 32);
+  Tile best;
+  double best_cost = 0;
+  for (const auto& t : kTiles) {
+    if (gs.multi && (gs.m % t.bm != 0 || gs.n % t.bn != 0)) continue;
+    bool akc, bkc;
+    if (!dma_operand(gs.ga_m, gs.ga_k, gs.ga_b, gs.a.offset, gs.m % t.bm == 0 ? t.bm : 8, akc) ||
+        !dma_operand(gs.gb_n, gs.gb_k, gs.gb_b, gs.b.offset, gs.n % t.bn == 0 ? t.bn : 8, bkc))
+      continue;
+    for (int splits = 1; splits <= 8; ++splits) {
+      if (steps % splits != 0 || (splits > 1 && steps / splits < 8)) continue;
+      const double groups = (double)(up(gs.m, t.bm) * up(gs.n, t.bn) * gs.batch) * splits;
+      const double full = std::floor(groups / 256.0), rest = groups - 256.0 * full;
+      // microseconds of one round of `active` workgroups
+      auto round = [&](double active) {
+        const double boost = active >= 256 ? 1.0 : std::min(1.45, 1.0 + 0.45 * (256.0 - active) / 128.0);
+        return 2e-6 * t.bm * t.bn * 32.0 * (double)(steps / splits) / (t.rate * boost) + 4.0;
+      };
+      double cost = full * round(256) + (rest > 0 ? round(rest) : 0.0);
+      if (splits > 1) cost += 3.0 + (double)splits * (double)(gs.m * gs.n * gs.batch) * 8.0 / 4e6;
+      if (!best.bm || cost < best_cost) {
+        best.bm = t.bm;
+        best.bn = t.bn;
+        best.splits = splits;
         best_cost = cost;
       }
     }
@@ -504,7 +546,14 @@ void Planner::gemm(uint32_t v, const GemmShape& gs, const OutStrides& os) {
   std::unique_ptr<KernelWriter> w;
   // Split along K: the contraction stores f32 sums of its part of K and split::sum adds them and runs the
   // epilogue, whose kernel then reads no operand.
-  const Tile tile = d == DType::f32 ? f32_tile(gs) : Tile();
+  int dm = 0, dn = 0;
+  bool akc = gs.a_k == 1, bkc = gs.b_k == 1;
+  const bool dma = d != DType::f32 && dma_eligible(gs, dm, dn, akc, bkc);
+  const Tile tile = d == DType::f32 ? f32_tile(gs) : dma ? dma_tile(gs) : Tile();
+  if (dma && tile.bm) {
+    dm = tile.bm;
+    dn = tile.bn;
+  }
   const bool split = tile.splits > 1;
   auto operands = [&](KernelWriter& kw) {
     kw.arg(gs.a.slot, false);
@@ -616,6 +665,14 @@ void Planner::gemm(uint32_t v, const GemmShape& gs, const OutStrides& os) {
                       !std::getenv("ACCY_GEMM_NO_STAGE");
   std::ostringstream src;
   KernelStep k;
+  std::string functor = "Epi_" + nm + "{" + members.inits + "}", part_struct;
+  if (split) {
+    part_struct = "struct Part_" + nm + " {\n  float* __restrict__ p;\n"
+                  "  __device__ __forceinline__ void operator()(long b, long m, long n, float v) const {\n    p[(blockIdx.z * " +
+                  std::to_string(gs.batch) + "L + b) * " + std::to_string(gs.m * gs.n) + "L + m * " + std::to_string(gs.n) +
+                  "L + n] = v;\n  }\n};\n";
+    functor = "Part_" + nm + "{" + partial + "}";
+  }
   src << "#include \"gemm\"\n";
   src << "struct Epi_" << nm << " {\n" << members.decls
       << table_members << (staged ? "  static constexpr bool kStaged = true;\n" : "")
@@ -640,13 +697,7 @@ void Planner::gemm(uint32_t v, const GemmShape& gs, const OutStrides& os) {
     k.block[0] = tile.bm ? 64u * (uint32_t)(tile.wm * tile.wn * tile.wk) : 256u;
     k.grid[0] = (uint32_t)(((gs.m + bm - 1) / bm) * ((gs.n + bn - 1) / bn));
     k.grid[2] = (uint32_t)tile.splits;
-    std::string functor = "Epi_" + nm + "{" + members.inits + "}";
-    if (split) {
-      src << "struct Part_" << nm << " {\n  float* __restrict__ p;\n"
-          << "  __device__ __forceinline__ void operator()(long b, long m, long n, float v) const {\n    p[(blockIdx.z * "
-          << gs.batch << "L + b) * " << gs.m * gs.n << "L + m * " << gs.n << "L + n] = v;\n  }\n};\n";
-      functor = "Part_" + nm + "{" + partial + "}";
-    }
+    src << part_struct;
     src << "extern \"C\" __global__ void __launch_bounds__(" << k.block[0] << ") " << nm << "(" << kw.params() << ") {\n"
         << "  accy::gemm::mma32f<Cfg_" << nm << ">(" << a << " + " << gs.a.offset << "L, " << b << " + "
         << gs.b.offset << "L, " << functor << ");\n}\n";
@@ -662,14 +713,11 @@ void Planner::gemm(uint32_t v, const GemmShape& gs, const OutStrides& os) {
         WN = nn;
       }
     }
-    // Direct-to-LDS pipeline when the tiles divide the problem exactly (every row start 16-byte
-    // aligned); otherwise the register-staged kernel, which guards edges (single strides only).
-    int dm = 0, dn = 0;
-    bool akc = gs.a_k == 1, bkc = gs.b_k == 1;
-    bool dma = dma_eligible(gs, dm, dn, akc, bkc);
+    // Direct-to-LDS pipeline (dma_eligible: every row start 16-byte aligned); otherwise the
+    // register-staged kernel, which guards edges (single strides only).
     src << "struct Cfg_" << nm << " {\n"
         << "  static constexpr int DT = " << (d == DType::bf16 ? 0 : 1) << ";\n"
-        << "  static constexpr long M = " << gs.m << ", N = " << gs.n << ", K = " << gs.k << ";\n"
+        << "  static constexpr long BATCH = " << gs.batch << ", M = " << gs.m << ", N = " << gs.n << ", K = " << gs.k << ";\n"
         << "  static constexpr long A_B = " << gs.a_b << ", A_M = " << gs.a_m << ", A_K = " << gs.a_k << ";\n"
         << "  static constexpr long B_B = " << gs.b_b << ", B_K = " << gs.b_k << ", B_N = " << gs.b_n << ";\n"
         << "  static constexpr bool A_KC = " << (akc ? "true" : "false") << ", B_KC = " << (bkc ? "true" : "false")
@@ -677,28 +725,32 @@ void Planner::gemm(uint32_t v, const GemmShape& gs, const OutStrides& os) {
         << gs.ga_b.fn("a_b") << gs.ga_m.fn("a_m") << gs.ga_k.fn("a_k") << gs.gb_b.fn("b_b") << gs.gb_k.fn("b_k")
         << gs.gb_n.fn("b_n");
     // Launch candidates of the direct-to-LDS kernel (bit-identical results: every output keeps its
-    // k order): the N tile, 256 (4 stages, one workgroup per CU, 128 KiB of LDS), then 128 where
-    // B's layout allows it. (256 x 128 with 3 stages and two workgroups per CU was measured too:
-    // its LDS traffic per MFMA is half as large again as the 256 x 256 tile's, and it ran 20-40 %
-    // slower on every benchmark contraction.) The source carries a placeholder until the candidate
-    // is chosen.
+    // k order and split): the N tile dma_tile chose, then the other of 256 and 128 where B's layout and
+    // extent allow it. (256 x 128 with 3 stages and two workgroups per CU was measured too: its LDS
+    // traffic per MFMA is half as large again as the 256 x 256 tile's, and it ran 20-40 % slower on
+    // every benchmark contraction.) The source carries a placeholder until the candidate is chosen.
     std::vector<int> n_tiles{dn};
-    if (dma && dn == 256) {
+    if (dma && gs.n > 128) {
+      const int other = 384 - dn;
       bool kc2 = bkc;
-      if (dma_operand(gs.gb_n, gs.gb_k, gs.gb_b, gs.b.offset, 128, kc2) && kc2 == bkc) n_tiles.push_back(128);
+      if (dma_operand(gs.gb_n, gs.gb_k, gs.gb_b, gs.b.offset, gs.n % other == 0 || gs.multi ? other : 8, kc2) && kc2 == bkc &&
+          (!gs.multi || gs.n % other == 0))
+        n_tiles.push_back(other);
     }
     const bool placeholder = n_tiles.size() > 1;
     if (dma) {
       src << "  static constexpr int BM = " << dm << ", BN = " << (placeholder ? "ACCY_N_TILE" : std::to_string(dn))
-          << ", STAGES = 4, GROUP_M = " << tile_group_m(gs.m, gs.n) << ";\n};\n";
+          << ", STAGES = 4, GROUP_M = " << tile_group_m(gs.m, gs.n) << (split ? ", SPLITS = " + std::to_string(tile.splits) : "")
+          << ";\n};\n";
     } else {
       src << "  static constexpr int BM = " << BM << ", BN = " << BN << ", BK = " << BK << ", WAVES_M = " << WM
           << ", WAVES_N = " << WN << ";\n};\n";
     }
     int threads = dma ? 256 : WM * WN * 64;
-    src << "extern \"C\" __global__ void __launch_bounds__(" << threads << ") " << nm << "(" << w->params() << ") {\n"
-        << "  accy::gemm::" << (dma ? "mma16_dma" : "mma16") << "<Cfg_" << nm << ">(" << a << " + " << gs.a.offset
-        << "L, " << b << " + " << gs.b.offset << "L, Epi_" << nm << "{" << members.inits << "});\n}\n";
+    src << part_struct << "extern \"C\" __global__ void __launch_bounds__(" << threads << ") " << nm << "(" << kw.params()
+        << ") {\n  accy::gemm::" << (dma ? "mma16_dma" : "mma16") << "<Cfg_" << nm << ">(" << a << " + " << gs.a.offset
+        << "L, " << b << " + " << gs.b.offset << "L, " << functor << ");\n}\n";
+    k.grid[2] = (uint32_t)tile.splits;
     k.source = src.str();
     if (placeholder) {
       k.tuning_key = tuning_key("gemm", k.source, "m=" + std::to_string(gs.m) + ",n=" + std::to_string(gs.n) +
@@ -724,7 +776,7 @@ void Planner::gemm(uint32_t v, const GemmShape& gs, const OutStrides& os) {
   if (split) {
     KernelStep sum;
     sum.name = name("split_sum", v);
-    const std::string both = src.str();
+    const std::string both = plan_.steps.back().kernel.source;  // with the launch candidate chosen
     sum.source = both.substr(0, both.find("struct Part_")) + "extern \"C\" __global__ void __launch_bounds__(256) " + sum.name + "(" +
                  w->params() + ") {\n  accy::split::sum<Cfg_" + nm + ">(" + w->arg(pw->args.back(), false) + ", Epi_" + nm +
                  "{" + members.inits + "});\n}\n";

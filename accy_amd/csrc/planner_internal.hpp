@@ -412,13 +412,16 @@ class Planner {
 
   bool dma_eligible(const GemmShape& gs, int& dm, int& dn, bool& a_kc, bool& b_kc) const;
 
-  // The f32 MFMA kernel's operand layouts: A K-contiguous, B N-contiguous, rows 16-byte aligned.
-  static bool f32_layout_ok(const GemmShape& gs);
-
   // Tile of a contraction kernel and the workgroups along K; bm = 0: none applies.
   struct Tile {
     int bm = 0, bn = 0, wm = 0, wn = 0, wk = 0, splits = 1;
   };
+
+  // Tile and K split of the direct-to-LDS 16-bit kernel.
+  static Tile dma_tile(const GemmShape& gs);
+
+  // The f32 MFMA kernel's operand layouts: A K-contiguous, B N-contiguous, rows 16-byte aligned.
+  static bool f32_layout_ok(const GemmShape& gs);
 
   // Whether the staged f32 kernel can read the operands: K or the row axis of each has stride 1 (in whole
   // vectors of four, where several axes make up the group).

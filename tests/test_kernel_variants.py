@@ -237,3 +237,56 @@ def test_ragged_rows_write_only_their_own_elements():
         x = np.random.default_rng(cols).integers(-1000, 1000, (rows, cols)).astype(np.int32)
         for got, ref in zip(hip_run(prog, [x]), oracle_run(prog, [x])):
             assert np.array_equal(got, ref)
+
+
+# ---- 16-bit contractions straight to LDS: tiles by size, K split, K past the last whole step ----
+
+# (m, k, n, layout, batch): K steps that K does not fill for every layout; rows of any number where the operand
+# is K-contiguous; one row; splits; batches
+DMA_SHAPES = [(1, 136, 8, "NN", 0), (1, 4096, 1024, "NN", 0), (3, 1000, 264, "NN", 0), (129, 1000, 135, "NT", 0),
+              (136, 1001, 264, "TN", 0), (128, 129, 128, "TN", 0), (264, 159, 520, "TN", 0), (1000, 3000, 512, "NN", 0),
+              (17, 2048, 8192, "NN", 0), (300, 4096, 304, "NT", 0), (256, 8192, 256, "TN", 0), (5, 264, 8, "NN", 3),
+              (200, 456, 130, "NT", 2)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("shape", DMA_SHAPES, ids=str)
+def test_direct_to_lds_contractions_within_the_summation_bound(shape, dtype):
+    """|error| <= (K + 2) u sum|a b| for an f32 sum of exact products in any order (u = 2^-24), and the result's
+    rounding (bf16 truncates: 2^-7; f16: 2^-11), once more per operation of the epilogue."""
+    m, k, n, layout, batch = shape
+    for epilogue in (False, True):
+        prog = contraction(dtype, m, k, n, layout, batch, epilogue)
+        assert "mma16_dma<" in hip.plan_source(prog)
+        ins, a, b, bias = contraction_inputs(dtype, m, k, n, layout, batch, epilogue, m + k)
+        got = to_f32(hip_run(prog, ins)[0], dtype).astype(np.float64)
+        ref, size, r = a @ b, np.abs(a) @ np.abs(b), {"bf16": 2.0 ** -7, "f16": 2.0 ** -11}[dtype]
+        bound = (k + 2) * 2.0 ** -24 * size + r * np.abs(ref)
+        if epilogue:
+            half = 0.5 * ref
+            ref = half + bias
+            bound = bound + r * (np.abs(half) + np.abs(ref) + bound)
+        assert np.all(np.abs(got - ref) <= bound + 2.0 ** -24)
+
+
+@pytest.mark.gpu
+def test_contraction_tail_ignores_what_lies_past_k():
+    """Infinities and NaN in the rows and columns that follow K in memory, or that the clamped loads
+    repeat, do not reach other outputs: row 0 of A and column 0 of B are not finite, everything else is."""
+    m, k, n = 130, 1005, 136
+    prog = contraction("bf16", m, k, n, "TN")
+    ins, a, b, _ = contraction_inputs("bf16", m, k, n, "TN", 0, False, 4)
+    clean = hip_run(prog, ins)[0]
+    ins[0][:, 0] = 0x7f80      # +inf in row 0
+    ins[1][:, 0] = 0x7fc0      # NaN in column 0
+    got = hip_run(prog, ins)[0]
+    assert np.array_equal(got[1:, 1:], clean[1:, 1:])
+
+
+def test_contractions_choose_their_tile_by_size():
+    plan = lambda m, k, n, layout="NN": hip.plan_source(contraction("bf16", m, k, n, layout))
+    assert "BM = 256, BN = 256" in plan(8192, 8192, 8192) and "SPLITS" not in plan(8192, 8192, 8192)
+    assert "BM = 128, BN = 128" in plan(2048, 8192, 2048) and "BM = 128, BN = 128" in plan(2048, 3000, 2048, "TN")
+    assert "SPLITS" in plan(256, 8192, 256) and plan(256, 8192, 256).count("__global__") == 2
+    hip.plan_source(contraction("bf16", 136, 1001, 264, "TN"), compile=True)
