@@ -608,11 +608,18 @@ __device__ __forceinline__ void flash(const u16_t* __restrict__ Q, const u16_t* 
 // f32 attention with a head dimension of 64: the reference's own flash pattern (f32 Q, K, V of head
 // dimension 64, src/preparation/kernelization/lowering/flash.zig:24-31), on v_mfma_f32_32x32x2_f32.
 //
-// A workgroup of WAVES waves owns 32 * WAVES queries of one batch index; each wave keeps its 32
-// queries' Q^T in registers and streams the keys in blocks of 32 through two LDS buffers. Lane half
-// h = lane / 32 supplies head dims 32 h .. 32 h + 31 to both MFMA operands (any split of the
-// contracted dims is valid when A and B agree), so one ds_read_b128 of a K row feeds four MFMAs.
-// Per block of 32 keys:
+// A workgroup owns 32 * WAVES queries of one batch index, and GROUPS groups of WAVES waves share them: group
+// g takes the key blocks g, g + GROUPS, ... of 32 keys, each through its own two LDS buffers, with its own
+// running maximum, sum and O, which group 0 puts together at the end. So a SIMD has two waves (one's
+// softmax runs beside the other's MFMAs) while a workgroup has few queries, of which there are then
+// enough to even out: under a causal mask the workgroups take between one and all of the key blocks, and
+// the longest start first. (16 x 2048 queries, causal: 256 workgroups of 128 queries with one wave per SIMD
+// ran as long as the longest, 174 us; 512 of 64 queries in four groups 93 us. With 32 queries to a K and V tile, 126 us,
+// the tiles' bytes from L2 bound it.)
+//
+// Each wave keeps its 32 queries' Q^T in registers. Lane half h = lane / 32 supplies head dims 32 h ..
+// 32 h + 31 to both MFMA operands (any split of the contracted dims is valid when A and B agree), so one
+// ds_read_b128 of a K row feeds four MFMAs. Per block of 32 keys:
 //  * S^T = K Q^T: 32 MFMAs into one 32 x 32 accumulator (lane l: query l % 32, keys 8 g + 4 h + j in
 //    register 4 g + j);
 //  * online softmax in f32 in the log2 domain: the scores are scaled by SL = scale * log2 e, the
@@ -620,36 +627,46 @@ __device__ __forceinline__ void flash(const u16_t* __restrict__ Q, const u16_t* 
 //    O and the row sum are rescaled by exp2(m_old - m_new) every block;
 //  * O^T += V^T P^T: two head-dim tiles x 16 key steps; step (g, j) takes key 8 g + j from lanes
 //    0-31 and key 8 g + 4 + j from lanes 32-63, exactly the keys those lanes' score registers 4 g + j
-//    hold, so P is the B operand as it stands; V is stored transposed in LDS so that one
-//    ds_read_b128 gives the A operands of four steps;
-// then O = O / l. LDS layouts (conflict-free 16-lane b128 reads on the 64-bank LDS): K as [key][64]
-// with the 16-byte chunk c of key row r at chunk c ^ (r & 15); V^T as [64][32 keys] with the chunk of
-// keys 4 kc .. 4 kc + 3 of row d at chunk kc ^ ((d / 2) & 7).
-// The configuration struct C supplies WAVES, SQ, SK, NB, Q_S, K_S, V_S (element strides of a query /
+//    hold, so P is the B operand as it stands, and 32 lanes read 32 consecutive dims of one V row;
+// then O = O / l. LDS layouts: K as [key][64] with the 16-byte chunk c of key row r at chunk c ^ (r & 15)
+// (conflict-free 16-lane b128 reads on the 64-bank LDS), V as [key][64].
+// The configuration struct C supplies WAVES, GROUPS, SQ, SK, NB, Q_S, K_S, V_S (element strides of a query /
 // key row; head dims have stride 1), CAUSAL, SL and q_off / k_off / v_off (batch offsets). O is
-// written row-major as [b][q][64]. Launched with 64 * WAVES threads, NB * SQ / (32 * WAVES) workgroups.
+// written row-major as [b][q][64]. Launched with 64 * WAVES * GROUPS threads, NB * SQ / (32 * WAVES) workgroups.
 template <class C>
 __device__ __forceinline__ void flash_f32(const float* __restrict__ Q, const float* __restrict__ K,
                                           const float* __restrict__ V, float* __restrict__ O) {
   typedef float f32x4 __attribute__((ext_vector_type(4)));
-  constexpr int WAVES = C::WAVES, D = 64, THREADS = 64 * WAVES, LD = 512 / THREADS;
+  constexpr int WAVES = C::WAVES, GROUPS = C::GROUPS, D = 64, THREADS = 64 * WAVES, LD = 512 / THREADS;
+  constexpr int TILE = 32 * D, PART = 34 * 64;  // floats of a K or V tile; of a wave's m, l and O
   constexpr long BQ = 32 * WAVES, NQB = C::SQ / BQ;
   static_assert(C::SQ % BQ == 0 && C::SK % 32 == 0 && 512 % THREADS == 0, "exact blocks only");
-  __shared__ __attribute__((aligned(16))) float ks[2][32 * D];
-  __shared__ __attribute__((aligned(16))) float vt[2][D * 32];
+  static_assert((GROUPS - 1) * WAVES * PART <= GROUPS * 4 * TILE, "the groups' parts fit the tiles");
+  __shared__ __attribute__((aligned(16))) float lds[GROUPS * 4 * TILE];  // per group: two K tiles, two V tiles
 
   // Workgroups of one batch index go to one XCD (they share its K and V); under a causal mask the
-  // query blocks with the most keys start first.
+  // query blocks with the most keys start first, of every batch index in turn.
   const long total = (long)gridDim.x;
-  long t = (long)blockIdx.x;
-  if (total % 8 == 0) t = (t % 8) * (total / 8) + t / 8;
-  const long b = t / NQB, qb = C::CAUSAL ? NQB - 1 - t % NQB : t % NQB;
-  if (b >= C::NB) return;  // a grid larger than the work
-  const int tid = (int)threadIdx.x, wave = tid >> 6, lane = tid & 63, h = lane >> 5, l32 = lane & 31;
+  long t = (long)blockIdx.x, b, qb;
+  if constexpr (C::CAUSAL && C::NB % 8 == 0) {
+    const long xcd = t % 8, per = C::NB / 8, i = t / 8;
+    b = xcd * per + i % per;
+    qb = NQB - 1 - i / per;
+  } else {
+    if (total % 8 == 0) t = (t % 8) * (total / 8) + t / 8;
+    b = t / NQB;
+    qb = C::CAUSAL ? NQB - 1 - t % NQB : t % NQB;
+  }
+  if (b >= C::NB || qb < 0) return;  // a grid larger than the work
+  const int lane = (int)threadIdx.x & 63, h = lane >> 5, l32 = lane & 31;
+  const int all = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), group = all / WAVES, wave = all % WAVES;
+  const int tid = 64 * wave + lane;  // within the group
   const long q0 = qb * BQ, query = q0 + 32 * wave + l32;
   const float* __restrict__ qp = Q + C::q_off(b);
   const float* __restrict__ kp = K + C::k_off(b);
   const float* __restrict__ vp = V + C::v_off(b);
+  float* const ks = lds + group * 4 * TILE;
+  float* const vs = ks + 2 * TILE;
 
   float qf[32];
 #pragma unroll
@@ -663,10 +680,13 @@ __device__ __forceinline__ void flash_f32(const float* __restrict__ Q, const flo
     const long last = (q0 + BQ - 1) / 32 + 1;
     nkb = last < nkb ? last : nkb;
   }
+  const long steps = (nkb + GROUPS - 1) / GROUPS;
 
-  // A block's K and V tiles (32 x 64 f32 each, 512 16-byte chunks): LD chunks of each per thread.
+  // A block's K and V tiles (32 x 64 f32 each, 512 16-byte chunks): LD chunks of each per thread. (A group
+  // with no block left reads the last one again and does not use it.)
   f32x4 kr[LD], vr[LD];
-  auto fetch = [&](long k0) {
+  auto fetch = [&](long j) {
+    const long k0 = (j < nkb ? j : nkb - 1) * 32;
 #pragma unroll
     for (int i = 0; i < LD; ++i) {
       const int idx = tid + i * THREADS, row = idx >> 4, c = idx & 15;
@@ -678,69 +698,89 @@ __device__ __forceinline__ void flash_f32(const float* __restrict__ Q, const flo
 #pragma unroll
     for (int i = 0; i < LD; ++i) {
       const int idx = tid + i * THREADS, row = idx >> 4, c = idx & 15;
-      *(f32x4*)(&ks[buf][row * D + 4 * (c ^ (row & 15))]) = kr[i];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int d = 4 * c + e;
-        vt[buf][d * 32 + 4 * ((row >> 2) ^ ((d >> 1) & 7)) + (row & 3)] = vr[i][e];
-      }
+      *(f32x4*)(&ks[buf * TILE + row * D + 4 * (c ^ (row & 15))]) = kr[i];
+      *(f32x4*)(&vs[buf * TILE + row * D + 4 * c]) = vr[i];
     }
   };
 
   float m = -__builtin_inff(), l = 0.0f;
   f32x16 o[2] = {f32x16{}, f32x16{}};
-  fetch(0);
+  fetch(group);
   stash(0);
   __syncthreads();
-  for (long j = 0; j < nkb; ++j) {
-    const int buf = (int)(j & 1);
-    if (j + 1 < nkb) fetch((j + 1) * 32);
-    const float* kl = ks[buf];
-    const float* vl = vt[buf];
-    f32x16 s = f32x16{};
+  for (long step = 0; step < steps; ++step) {
+    const int buf = (int)(step & 1);
+    const long j = step * GROUPS + group, k0 = j * 32;
+    if (step + 1 < steps) fetch(j + GROUPS);
+    // blocks past the last one, or above the diagonal for all of the wave's queries, add nothing
+    if (j < nkb && (!C::CAUSAL || k0 <= q0 + 32 * wave + 31)) {
+      const float* kl = ks + buf * TILE;
+      const float* vl = vs + buf * TILE;
+      f32x16 s = f32x16{};
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const f32x4 a = *(const f32x4*)(kl + l32 * D + 4 * ((8 * h + i) ^ (l32 & 15)));
+      for (int i = 0; i < 8; ++i) {
+        const f32x4 a = *(const f32x4*)(kl + l32 * D + 4 * ((8 * h + i) ^ (l32 & 15)));
 #pragma unroll
-      for (int e = 0; e < 4; ++e) s = gemm::mfma32x32x2f32(a[e], qf[4 * i + e], s);
-    }
-    const long k0 = j * 32;
-    float mx = -__builtin_inff();
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      float x = s[r] * C::SL;
-      if constexpr (C::CAUSAL) {
-        if (k0 + 8 * (r >> 2) + 4 * h + (r & 3) > query) x = -__builtin_inff();
+        for (int e = 0; e < 4; ++e) s = gemm::mfma32x32x2f32(a[e], qf[4 * i + e], s);
       }
-      s[r] = x;
-      mx = fmaxf(mx, x);
-    }
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float mn = fmaxf(m, mx);
-    const float msub = mn == -__builtin_inff() ? 0.0f : mn;
-    const float alpha = __builtin_amdgcn_exp2f(m - msub);
-    float ps = 0.0f;
+      float mx = -__builtin_inff();
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      s[r] = __builtin_amdgcn_exp2f(s[r] - msub);
-      ps += s[r];
-    }
-    l = l * alpha + ps;
-    m = mn;
-    o[0] *= alpha;
-    o[1] *= alpha;
-#pragma unroll
-    for (int dt = 0; dt < 2; ++dt)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int d = dt * 32 + l32;
-        const f32x4 a = *(const f32x4*)(vl + d * 32 + 4 * ((2 * g + h) ^ ((d >> 1) & 7)));
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj) o[dt] = gemm::mfma32x32x2f32(a[jj], s[4 * g + jj], o[dt]);
+      for (int r = 0; r < 16; ++r) {
+        float x = s[r] * C::SL;
+        if constexpr (C::CAUSAL) {
+          if (k0 + 8 * (r >> 2) + 4 * h + (r & 3) > query) x = -__builtin_inff();
+        }
+        s[r] = x;
+        mx = fmaxf(mx, x);
       }
-    // Buffer (j + 1) % 2 was last read in block j - 1, before the barrier that ended it.
-    if (j + 1 < nkb) stash((int)((j + 1) & 1));
+      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      const float mn = fmaxf(m, mx);
+      const float msub = mn == -__builtin_inff() ? 0.0f : mn;
+      const float alpha = __builtin_amdgcn_exp2f(m - msub);
+      float ps = 0.0f;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        s[r] = __builtin_amdgcn_exp2f(s[r] - msub);
+        ps += s[r];
+      }
+      l = l * alpha + ps;
+      m = mn;
+      o[0] *= alpha;
+      o[1] *= alpha;
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) {
+          const float* row = vl + (8 * g + 4 * h + jj) * D + l32;
+#pragma unroll
+          for (int dt = 0; dt < 2; ++dt) o[dt] = gemm::mfma32x32x2f32(row[32 * dt], s[4 * g + jj], o[dt]);
+        }
+    }
+    // Buffer (step + 1) % 2 was last read in step - 1, before the barrier that ended it.
+    if (step + 1 < steps) stash((int)((step + 1) & 1));
     __syncthreads();
+  }
+  // The other groups' parts join group 0's in group order.
+  if constexpr (GROUPS > 1) {
+    if (group > 0) {
+      float* const part = lds + ((group - 1) * WAVES + wave) * PART + lane;
+      part[0] = m;
+      part[64] = l;
+#pragma unroll
+      for (int e = 0; e < 32; ++e) part[(2 + e) * 64] = o[e >> 4][e & 15];
+    }
+    __syncthreads();
+    if (group > 0) return;
+#pragma unroll 1
+    for (int g = 0; g < GROUPS - 1; ++g) {
+      const float* const part = lds + (g * WAVES + wave) * PART + lane;
+      const float mg = part[0], mn = fmaxf(m, mg), msub = mn == -__builtin_inff() ? 0.0f : mn;
+      const float alpha = __builtin_amdgcn_exp2f(m - msub), beta = __builtin_amdgcn_exp2f(mg - msub);
+      l = l * alpha + part[64] * beta;
+      m = mn;
+#pragma unroll
+      for (int e = 0; e < 32; ++e) o[e >> 4][e & 15] = o[e >> 4][e & 15] * alpha + part[(2 + e) * 64] * beta;
+    }
   }
   const float inv = 1.0f / (l + __shfl_xor(l, 32, 64));
   float* __restrict__ orow = O + (b * C::SQ + query) * D;

@@ -51,7 +51,7 @@ extern "C" __global__ void __launch_bounds__(256) accy_check_attention_causal_bf
 }
 
 struct CheckAttnF32Causal {
-  static constexpr int WAVES = 4;
+  static constexpr int WAVES = 4, GROUPS = 2;
   static constexpr long SQ = 1024, SK = 1024, NB = 4;
   static constexpr long Q_S = 64, K_S = 64, V_S = 64;
   static constexpr bool CAUSAL = true;

@@ -318,7 +318,18 @@ double Planner::attention_pairs(const Attn& at, const AttnLayout& L) {
 
 void Planner::attention_f32(uint32_t pv, const Attn& at, const AttnLayout& L) {
   int out = slots_.slot_of[pv] >= 0 ? slots_.slot_of[pv] : temp_slot(pv);
-  const int waves = L.sq % 128 == 0 ? 4 : (L.sq % 64 == 0 ? 2 : 1);
+  // Eight waves: 128 queries in two key groups where that makes two workgroups for every CU and more, else
+  // 64 queries in four; four waves of 32 queries where even 64 would leave half of the CUs idle. (us a pass,
+  // 4 x 2 / 2 x 4 / 1 x 4: 64 x 1024 causal 91 / 102 / 145, 16 x 2048 causal 149 / 93 / 126, 1 x 4096 283 / 157 / 108; before,
+  // four waves of 128 queries: 158, 174, 325.)
+  const int64_t queries = L.nb * L.sq;
+  int waves = 1, groups = 4;
+  if (L.sq % 128 == 0 && queries / 128 >= 512) {
+    waves = 4;
+    groups = 2;
+  } else if (L.sq % 64 == 0 && queries / 64 > 128) {
+    waves = 2;
+  }
   KernelWriter w(g_, slots_, "i64_t");
   std::string q = w.arg(L.q.slot, false), k = w.arg(L.k.slot, false), v = w.arg(L.v.slot, false),
               o = w.arg(out, true);
@@ -328,7 +339,7 @@ void Planner::attention_f32(uint32_t pv, const Attn& at, const AttnLayout& L) {
   std::ostringstream src;
   src << "#include \"gemm\"\n#include \"attention\"\n";
   src << "struct Cfg_" << nm << " {\n"
-      << "  static constexpr int WAVES = " << waves << ";\n"
+      << "  static constexpr int WAVES = " << waves << ", GROUPS = " << groups << ";\n"
       << "  static constexpr long SQ = " << L.sq << ", SK = " << L.sk << ", NB = " << L.nb << ";\n"
       << "  static constexpr long Q_S = " << L.q_s << ", K_S = " << L.k_s << ", V_S = " << L.v_s << ";\n"
       << "  static constexpr bool CAUSAL = " << (at.causal ? "true" : "false") << ";\n"
@@ -345,13 +356,13 @@ void Planner::attention_f32(uint32_t pv, const Attn& at, const AttnLayout& L) {
     params += "const float* __restrict__ " + x + ", ";
   }
   params += "float* __restrict__ " + o;
-  src << "extern \"C\" __global__ void __launch_bounds__(" << 64 * waves << ") " << nm << "(" << params
+  src << "extern \"C\" __global__ void __launch_bounds__(" << 64 * waves * groups << ") " << nm << "(" << params
       << ") {\n  accy::attn::flash_f32<Cfg_" << nm << ">(" << q << ", " << k << ", " << v << ", " << o << ");\n}\n";
   KernelStep ks;
   ks.source = src.str();
   ks.name = nm;
   ks.grid[0] = (uint32_t)(L.nb * (L.sq / (32 * waves)));
-  ks.block[0] = 64 * waves;
+  ks.block[0] = 64 * waves * groups;
   ks.klass = "attention";
   ks.label = "attention:%" + std::to_string(pv);
   ks.algorithmic_flops = 4.0 * (double)L.nb * attention_pairs(at, L) * (double)L.hd;

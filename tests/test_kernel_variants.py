@@ -6,7 +6,7 @@ import pytest
 from accy_amd import hip
 from accy_amd import tensor as T
 from accy_amd import workloads as W
-from conftest import assert_rel, hip_run, oracle_run, to_f32
+from conftest import exact_attention, hip_run, oracle_run, to_f32
 
 F32 = T.Type("f32", ())
 
@@ -290,3 +290,33 @@ def test_contractions_choose_their_tile_by_size():
     assert "BM = 128, BN = 128" in plan(2048, 8192, 2048) and "BM = 128, BN = 128" in plan(2048, 3000, 2048, "TN")
     assert "SPLITS" in plan(256, 8192, 256) and plan(256, 8192, 256).count("__global__") == 2
     hip.plan_source(contraction("bf16", 136, 1001, 264, "TN"), compile=True)
+
+
+# ---- f32 attention of head dimension 64: key groups ----
+
+# (heads, queries, keys, causal, waves, groups): fewer key blocks than groups, a last round that not every group
+# takes part in, more keys than queries and fewer, every workgroup shape
+F32_ATTENTION = [(1, 32, 32, False, 1, 4), (3, 32, 160, False, 1, 4), (2, 96, 96, True, 1, 4), (2, 128, 64, True, 1, 4),
+                 (70, 128, 96, False, 2, 4), (72, 192, 192, True, 2, 4), (512, 128, 160, True, 4, 2), (520, 128, 32, False, 4, 2)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", F32_ATTENTION, ids=str)
+def test_f32_attention_key_groups(case):
+    """Against float64, 1e-4 of the largest magnitude (as the fused f32 attention's other shapes)."""
+    heads, queries, keys, causal, waves, groups = case
+    specs = [T.spec("f32", head=heads, query=queries, dim=64)] + [T.spec("f32", head=heads, key=keys, dim=64)] * 2
+    def body(b, a):
+        q, k, v = a
+        s = q.contract(k, "dim").mul(b.full_float(F32, 0.125))
+        if causal:
+            dims = [d for d in s.ty.dims if d[0] in ("query", "key")]
+            s = b.iota("i32", "query", *dims).compare("ge", b.iota("i32", "key", *dims)).select(s, b.full_float(F32, -np.inf))
+        e = s.sub(s.max("key")).exp()
+        return e.div(e.sum("key")).contract(v, "key")
+    prog = T.define("attention", specs, body)
+    assert f"WAVES = {waves}, GROUPS = {groups};" in hip.plan_source(prog)
+    rng = np.random.default_rng(queries + keys)
+    ins = [rng.standard_normal((heads, n, 64)).astype(np.float32) for n in (queries, keys, keys)]
+    exact = exact_attention(*ins, 0.125, causal, "f32")
+    assert np.abs(hip_run(prog, ins)[0] - exact).max() <= 1e-4 * np.abs(exact).max()
