@@ -1,19 +1,11 @@
 // Dense contraction C[b, m, n] = sum_k A[b, m, k] * B[b, k, n] on gfx950 matrix cores.
 //
-// Hand-written for CDNA4: f32 accumulation in v_mfma_f32_32x32x16_{bf16,f16}; a 256 x 256 x 64
-// block tile computed by 8 wavefronts (4 along M x 2 along N), each owning a 64 x 128 sub-tile of
-// 2 x 4 MFMA 32x32 accumulators; both operands staged through LDS with K innermost (rows padded by
-// 16 bytes so that the 16-byte fragment reads of 8 consecutive lanes hit distinct banks) and double
-// buffered, so one barrier per K step separates the LDS writes of tile k+1 from the reads of tile k
-// while the global loads of tile k+1 are in flight under the MFMAs of tile k.
-//
-// Operand layouts: an operand whose K stride is 1 is loaded as 16-byte vectors along K and written
-// to LDS unchanged; an operand whose M (or N) stride is 1 is loaded as 8 x 8 blocks (8 vectors along
-// M/N at 8 consecutive k) and transposed in registers before the LDS write. Neighbouring lanes take
-// neighbouring k-groups of one row group, so the 8 lanes of one LDS store cycle write 8 different
-// 16-byte columns of the padded rows (distinct banks) while each global load instruction still covers
-// whole 128-byte lines (8 lanes x 16 bytes of one k row). Blocks are renumbered so
-// that the tiles dispatched to one XCD are neighbours (shared A rows / B columns in that XCD's L2).
+// Hand-written for CDNA4: f32 accumulation in v_mfma_f32_32x32x16_{bf16,f16} and
+// v_mfma_f32_32x32x2_f32, operands staged in LDS. 16-bit operands go straight from memory to LDS
+// (mma16_dma) where their rows are 16-byte aligned, else through registers (mma16_staged); f32 operands
+// straight to LDS in 256 x 256 tiles (mma32f_direct) or through registers in smaller ones (mma32f_staged).
+// Blocks are renumbered so that the tiles dispatched to one XCD are neighbours (shared A rows / B columns
+// in that XCD's L2).
 //
 // The configuration struct C supplies extents, strides (elements), tile shape and dtype; the
 // epilogue functor receives (batch, m, n, f32 accumulator) for every in-range output element.
@@ -35,21 +27,6 @@ __device__ __forceinline__ f32x16 mfma32x32x16(u32x4 a, u32x4 b, f32x16 c) {
   } else {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0,
                                                   0, 0);
-  }
-}
-
-// 8 x 8 transpose of 16-bit elements: in[k] holds 8 consecutive rows at one k; out[r] holds 8
-// consecutive k of one row.
-__device__ __forceinline__ void transpose8x8(const u32x4 (&in)[8], u32x4 (&out)[8]) {
-#pragma unroll
-  for (int r = 0; r < 8; ++r) {
-    const int w = r >> 1;
-    const bool hi = r & 1;
-#pragma unroll
-    for (int d = 0; d < 4; ++d) {
-      const u32_t lo_src = in[2 * d][w], hi_src = in[2 * d + 1][w];
-      out[r][d] = hi ? ((lo_src >> 16) | (hi_src & 0xffff0000u)) : ((lo_src & 0xffffu) | (hi_src << 16));
-    }
   }
 }
 
@@ -78,167 +55,8 @@ __device__ __forceinline__ void tile_of(long bid, long& tm, long& tn) {
   tile_in_groups<TILES_M, TILES_N, GROUP_M>(xcd_contiguous<TILES_M * TILES_N>(bid), tm, tn);
 }
 
-// Loads one operand tile (ROWS rows of the operand's M or N, BK values of K) into registers.
-// KC: K stride is 1 (vectors along K); otherwise the row stride is 1 (8 x 8 blocks, transposed).
-template <int ROWS, int BK, int THREADS, bool KC, long RT, long KT, long SR, long SK>
-struct TileLoader {
-  static constexpr int VEC_PER_ROW = BK / 8;
-  static constexpr int VECS = ROWS * BK / 8;
-  static constexpr int PER_THREAD = VECS / THREADS;
-  static_assert(VECS % THREADS == 0, "tile vectors must divide evenly among loader threads");
-  static_assert(KC || PER_THREAD % 8 == 0, "transposing loader handles whole 8 x 8 blocks");
-  u32x4 v[PER_THREAD];
-
-  __device__ __forceinline__ void load(const u16_t* __restrict__ base, long r0, long k0, int t) {
-    if constexpr (KC) {
-#pragma unroll
-      for (int i = 0; i < PER_THREAD; ++i) {
-        const int idx = t + i * THREADS;
-        const int row = idx / VEC_PER_ROW, kc = idx % VEC_PER_ROW;
-        const long r = r0 + row, k = k0 + kc * 8;
-        if ((RT % 256 == 0 || r < RT) && (KT % 64 == 0 || k < KT))
-          v[i] = *(const u32x4*)(base + r * SR + k);
-        else
-          v[i] = u32x4{0, 0, 0, 0};
-      }
-    } else {
-      constexpr int RG = ROWS / 8;
-      (void)RG;
-#pragma unroll
-      for (int b = 0; b < PER_THREAD / 8; ++b) {
-        const int bidx = t + b * THREADS;
-        const int kg = bidx % (BK / 8), rg = bidx / (BK / 8);
-        const long r = r0 + rg * 8;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const long k = k0 + kg * 8 + i;
-          if ((RT % 256 == 0 || r < RT) && (KT % 64 == 0 || k < KT))
-            v[b * 8 + i] = *(const u32x4*)(base + k * SK + r);
-          else
-            v[b * 8 + i] = u32x4{0, 0, 0, 0};
-        }
-      }
-    }
-  }
-
-  // Writes the staged tile into LDS as [row][k] with row stride LDK.
-  template <int LDK>
-  __device__ __forceinline__ void store(u16_t* __restrict__ lds, int t) {
-    if constexpr (KC) {
-#pragma unroll
-      for (int i = 0; i < PER_THREAD; ++i) {
-        const int idx = t + i * THREADS;
-        const int row = idx / VEC_PER_ROW, kc = idx % VEC_PER_ROW;
-        *(u32x4*)(lds + row * LDK + kc * 8) = v[i];
-      }
-    } else {
-      constexpr int RG = ROWS / 8;
-      (void)RG;
-#pragma unroll
-      for (int b = 0; b < PER_THREAD / 8; ++b) {
-        const int bidx = t + b * THREADS;
-        const int kg = bidx % (BK / 8), rg = bidx / (BK / 8);
-        u32x4 in[8], out[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) in[i] = v[b * 8 + i];
-        transpose8x8(in, out);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) *(u32x4*)(lds + (rg * 8 + j) * LDK + kg * 8) = out[j];
-      }
-    }
-  }
-};
-
-// One workgroup computes one BM x BN tile of one batch element. Needs BM*BN... LDS of
-// 2 * (BM + BN) * (BK + 8) 16-bit elements, passed as dynamic shared memory.
-template <class C, class Epi>
-__device__ __forceinline__ void mma16(const u16_t* __restrict__ A, const u16_t* __restrict__ B, const Epi& epi) {
-  constexpr int BM = C::BM, BN = C::BN, BK = C::BK, LDK = BK + 8;
-  constexpr int WAVES = C::WAVES_M * C::WAVES_N, THREADS = WAVES * 64, HALF = THREADS / 2;
-  constexpr int WTM = BM / C::WAVES_M, WTN = BN / C::WAVES_N;
-  constexpr int TM = WTM / 32, TN = WTN / 32;
-  constexpr long TILES_M = (C::M + BM - 1) / BM, TILES_N = (C::N + BN - 1) / BN;
-  constexpr long KTILES = (C::K + BK - 1) / BK;
-  constexpr int STAGE = (BM + BN) * LDK;
-  extern __shared__ u16_t lds[];
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave / C::WAVES_N, wn = wave % C::WAVES_N;
-  long tm, tn;
-  tile_of<TILES_M, TILES_N, 8>((long)blockIdx.x, tm, tn);
-  const long m0 = tm * BM, n0 = tn * BN, batch = blockIdx.y;
-  const u16_t* __restrict__ Ab = A + batch * C::A_B;
-  const u16_t* __restrict__ Bb = B + batch * C::B_B;
-
-  // The first half of the workgroup stages A, the second half B (whole wavefronts each).
-  const bool loads_a = tid < HALF;
-  const int lt = loads_a ? tid : tid - HALF;
-  TileLoader<BM, BK, HALF, C::A_KC, C::M, C::K, C::A_M, C::A_K> la;
-  TileLoader<BN, BK, HALF, C::B_KC, C::N, C::K, C::B_N, C::B_K> lb;
-
-  f32x16 acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = f32x16{};
-
-  if (loads_a) {
-    la.load(Ab, m0, 0, lt);
-    la.template store<LDK>(lds, lt);
-  } else {
-    lb.load(Bb, n0, 0, lt);
-    lb.template store<LDK>(lds + BM * LDK, lt);
-  }
-  __syncthreads();
-
-  const int frag_row = lane & 31, frag_k = (lane >> 5) * 8;
-  for (long kt = 0; kt < KTILES; ++kt) {
-    const bool more = kt + 1 < KTILES;
-    if (more) {
-      if (loads_a) la.load(Ab, m0, (kt + 1) * BK, lt);
-      else lb.load(Bb, n0, (kt + 1) * BK, lt);
-    }
-    const u16_t* __restrict__ sa = lds + (kt & 1) * STAGE + (wm * WTM + frag_row) * LDK + frag_k;
-    const u16_t* __restrict__ sb = lds + (kt & 1) * STAGE + BM * LDK + (wn * WTN + frag_row) * LDK + frag_k;
-#pragma unroll
-    for (int s = 0; s < BK / 16; ++s) {
-      u32x4 a[TM], b[TN];
-#pragma unroll
-      for (int i = 0; i < TM; ++i) a[i] = *(const u32x4*)(sa + i * 32 * LDK + s * 16);
-#pragma unroll
-      for (int j = 0; j < TN; ++j) b[j] = *(const u32x4*)(sb + j * 32 * LDK + s * 16);
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = mfma32x32x16<C::DT>(a[i], b[j], acc[i][j]);
-    }
-    if (more) {
-      u16_t* dst = lds + ((kt + 1) & 1) * STAGE;
-      if (loads_a) la.template store<LDK>(dst, lt);
-      else lb.template store<LDK>(dst + BM * LDK, lt);
-    }
-    __syncthreads();
-  }
-
-  // Accumulator layout of a 32x32 MFMA: lane l holds column l % 32, rows 8g + 4(l / 32) + j in
-  // register 4g + j.
-  const long col_base = n0 + wn * WTN + (lane & 31);
-  const long row_base = m0 + wm * WTM + (lane >> 5) * 4;
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int g = 0; g < 4; ++g)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const long m = row_base + i * 32 + g * 8 + r, n = col_base + j * 32;
-          if ((C::M % BM == 0 || m < C::M) && (C::N % BN == 0 || n < C::N)) epi(batch, m, n, acc[i][j][g * 4 + r]);
-        }
-}
-
 // ---------------------------------------------------------------------------------------------
-// Direct-to-LDS pipeline (tiles that divide the problem exactly).
+// Direct-to-LDS pipeline.
 //
 // Each K step (BK = 32) stages a BM x 32 tile of A and a 32 x BN tile of B straight from global
 // memory into LDS with global_load_lds_dwordx4 (lane l of an instruction writes bytes [16 l, 16 l + 16)
@@ -784,6 +602,152 @@ __device__ __forceinline__ void mma16_dma_group(const u16_t* __restrict__ A, con
     if (g == i) Bg = B[i];
   u16_t* __restrict__ const out = epi.out(g);
   mma16_dma_tile<C>(A, Bg, [&](long b, long m, long n, float v) { epi(out, b, m, n, v); }, tm, tn);
+}
+
+// ---------------------------------------------------------------------------------------------
+// 16-bit contraction staged through registers: any extents and alignment, operands whose K or row axis
+// has stride 1 (rows that are not 16-byte aligned, extents that are no multiple of 8, K below 128).
+//
+// 128 x 128 tiles of four waves in K steps of 64, laid out in LDS as two stages of the direct-to-LDS kernel
+// (whose fragment reads these are), two buffers, so that two workgroups share a CU and one's loads and
+// barrier pass under the other's MFMAs. 16 bytes per load at any alignment. A vector that reaches past the
+// operand's rows (or past K in the last step) starts at the last whole one and is shifted down, zeros
+// following: no load leaves the operand, none is behind a divergent branch, and k past the end adds
+// nothing. What bounds it is the loads' latency: 3000 x 2047 x 2045 reaches 448 TFLOP/s (56 us), where one
+// thread per output folding k, as before, reached 7.3 (3426 us).
+// ---------------------------------------------------------------------------------------------
+
+struct __attribute__((packed, aligned(2))) U16x8Any { u32_t v[4]; };
+
+// The eight 16-bit elements of v moved down by d (all zero from d = 8 on).
+__device__ __forceinline__ u32x4 shift_down(u32x4 v, long d) {
+  u64_t lo = (u64_t)v[0] | ((u64_t)v[1] << 32), hi = (u64_t)v[2] | ((u64_t)v[3] << 32);
+  if (d >= 4) {
+    lo = hi;
+    hi = 0;
+  }
+  const int b = 16 * (int)(d & 3);
+  const u64_t down = (lo >> b) | ((hi << 1) << (63 - b));
+  lo = d >= 8 ? 0 : down;
+  hi = d >= 8 ? 0 : hi >> b;
+  return u32x4{(u32_t)lo, (u32_t)(lo >> 32), (u32_t)hi, (u32_t)(hi >> 32)};
+}
+
+// One operand's step of ROWS x 64: O its offset functions, R its row extent, two direct-to-LDS stages in LDS.
+template <int ROWS, bool KC, class O, long R, long K>
+struct StageAny {
+  static constexpr int PER = ROWS * 64 / 8 / 256;
+  u32x4 v[PER];
+
+  template <bool TAIL>
+  __device__ __forceinline__ void load(const u16_t* __restrict__ base, long r0, long k0, int t) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int idx = t + i * 256;
+      // the vector's first element along the contiguous axis, and that axis's extent
+      const long row = r0 + (KC ? idx / 8 : idx % (ROWS / 8) * 8), k = k0 + (KC ? idx % 8 * 8 : idx / (ROWS / 8));
+      const long x = KC ? k : row;
+      constexpr long L = KC ? K : R;
+      const u16_t* __restrict__ p = base + (KC ? O::row(row < R ? row : R - 1) : O::k(!TAIL || k < K ? k : K - 1));
+      constexpr bool MAY_PASS = KC ? TAIL : R % ROWS != 0;
+      if constexpr (L >= 8) {
+        const long from = MAY_PASS && x > L - 8 ? L - 8 : x;
+        const U16x8Any w = *(const U16x8Any*)(p + (KC ? O::k(from) : O::row(from)));
+        v[i] = u32x4{w.v[0], w.v[1], w.v[2], w.v[3]};
+        if constexpr (MAY_PASS && (KC || R % 8 != 0)) v[i] = shift_down(v[i], x - from);
+      } else {
+        u32_t e[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const long at = x + j < L ? x + j : L - 1;
+          const u32_t h = p[KC ? O::k(at) : O::row(at)];
+          e[j] = x + j < L ? h : 0;
+        }
+        v[i] = u32x4{e[0] | e[1] << 16, e[2] | e[3] << 16, e[4] | e[5] << 16, e[6] | e[7] << 16};
+      }
+      if constexpr (!KC && TAIL) v[i] = k < K ? v[i] : u32x4{0, 0, 0, 0};
+    }
+  }
+
+  __device__ __forceinline__ void store(u16_t* lds, int t) const {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int idx = t + i * 256;
+      if constexpr (KC) {
+        const int row = idx / 8, c = idx % 8, line = row >> 2, slot = ((row & 3) << 2) | (c & 3);
+        *(u32x4*)(lds + (c >> 2) * (ROWS * 32) + line * 128 + ((slot ^ (line & 3)) << 3)) = v[i];
+      } else {
+        const int k = idx / (ROWS / 8), c = idx % (ROWS / 8), kk = k & 31;
+        *(u32x4*)(lds + (k >> 5) * (ROWS * 32) + kk * ROWS + ((c >> 1) ^ tr_swizzle(kk)) * 16 + 8 * (c & 1)) = v[i];
+      }
+    }
+  }
+};
+
+template <class C, class Epi>
+__device__ __forceinline__ void mma16_staged(const u16_t* __restrict__ A, const u16_t* __restrict__ B, const Epi& epi) {
+  constexpr int BM = C::BM, BN = C::BN, TM = BM / 64, TN = BN / 64, SA = BM * 64, SB = BN * 64;
+  constexpr long TILES_M = (C::M + BM - 1) / BM, TILES_N = (C::N + BN - 1) / BN;
+  constexpr long STEPS = (C::K + 63) / 64, SPLIT_STEPS = (STEPS + C::SPLITS - 1) / C::SPLITS;
+  __shared__ __attribute__((aligned(1024))) u16_t lds[2 * (SA + SB)];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave >> 1, wn = wave & 1;
+  long tm, tn;
+  tile_of<TILES_M, TILES_N, 8>((long)blockIdx.x, tm, tn);
+  const long m0 = tm * BM, n0 = tn * BN, batch = blockIdx.y;
+  const u16_t* __restrict__ Ab = A + C::a_b(batch);
+  const u16_t* __restrict__ Bb = B + C::b_b(batch);
+  const long first = (long)blockIdx.z * SPLIT_STEPS, end = first + SPLIT_STEPS < STEPS ? first + SPLIT_STEPS : STEPS;
+
+  f32x16 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = f32x16{};
+  StageAny<BM, C::A_KC, AOff<C>, C::M, C::K> sa;
+  StageAny<BN, C::B_KC, BOff<C>, C::N, C::K> sb;
+  auto load = [&](long s) {
+    if (C::K % 64 == 0 || s + 1 < STEPS) {
+      sa.template load<false>(Ab, m0, s * 64, tid);
+      sb.template load<false>(Bb, n0, s * 64, tid);
+    } else {
+      sa.template load<true>(Ab, m0, s * 64, tid);
+      sb.template load<true>(Bb, n0, s * 64, tid);
+    }
+  };
+  load(first);
+  sa.store(lds, tid);
+  sb.store(lds + SA, tid);
+  __syncthreads();
+  for (long s = first; s < end; ++s) {
+    const u16_t* const as = lds + (s - first & 1) * (SA + SB);
+    const bool more = s + 1 < end;
+    if (more) load(s + 1);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      Frags<C> f;
+#pragma unroll
+      for (int i = 0; i < Frags<C>::COUNT; ++i)
+        f.load_one(i, as + (q >> 1) * (BM * 32), as + SA + (q >> 1) * (BN * 32), q & 1, lane, wm, wn);
+#pragma unroll
+      for (int i = 0; i < TM * TN; ++i) f.mma_one(i, acc);
+    }
+    if (more) {
+      u16_t* const next = lds + (s + 1 - first & 1) * (SA + SB);
+      sa.store(next, tid);
+      sb.store(next + SA, tid);
+    }
+    __syncthreads();
+  }
+  const long col_base = n0 + wn * (BN / 2) + (lane & 31), row_base = m0 + wm * (BM / 2) + (lane >> 5) * 4;
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const long m = row_base + i * 32 + (e >> 2) * 8 + (e & 3), n = col_base + j * 32;
+        if ((C::M % BM == 0 || m < C::M) && (C::N % BN == 0 || n < C::N)) epi(batch, m, n, acc[i][j][e]);
+      }
 }
 
 // ---------------------------------------------------------------------------------------------

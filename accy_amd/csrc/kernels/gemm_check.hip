@@ -4,35 +4,11 @@
 #include "common.h"
 #include "gemm.h"
 
-struct CheckNN {
-  static constexpr int DT = 0;
-  static constexpr long M = 8192, N = 8192, K = 8192;
-  static constexpr long A_B = 0, A_M = 8192, A_K = 1, B_B = 0, B_K = 8192, B_N = 1;
-  static constexpr bool A_KC = true, B_KC = false;
-  static constexpr int BM = 256, BN = 256, BK = 64, WAVES_M = 4, WAVES_N = 2;
-};
-
-struct CheckNT {
-  static constexpr int DT = 1;
-  static constexpr long M = 4100, N = 1000, K = 136;
-  static constexpr long A_B = 4100 * 136, A_M = 136, A_K = 1, B_B = 1000 * 136, B_K = 1, B_N = 136;
-  static constexpr bool A_KC = true, B_KC = true;
-  static constexpr int BM = 256, BN = 256, BK = 64, WAVES_M = 4, WAVES_N = 2;
-};
-
 struct CheckEpi {
   u16_t* c;
   long ld;
   __device__ __forceinline__ void operator()(long b, long m, long n, float v) const { c[m * ld + n] = accy::f32_to_bf16(v); }
 };
-
-extern "C" __global__ void __launch_bounds__(512) accy_check_gemm_nn(const u16_t* a, const u16_t* b, u16_t* c) {
-  accy::gemm::mma16<CheckNN>(a, b, CheckEpi{c, 8192});
-}
-
-extern "C" __global__ void __launch_bounds__(512) accy_check_gemm_nt(const u16_t* a, const u16_t* b, u16_t* c) {
-  accy::gemm::mma16<CheckNT>(a, b, CheckEpi{c, 1000});
-}
 
 extern "C" __global__ void __launch_bounds__(256) accy_check_common(const float* x, float* y) {
   __shared__ float lds[4];
@@ -107,4 +83,15 @@ struct CheckDmaMultiAxis {
 
 extern "C" __global__ void __launch_bounds__(256) accy_check_gemm_dma_multi(const u16_t* a, const u16_t* b, u16_t* c) {
   accy::gemm::mma16_dma<CheckDmaMultiAxis>(a, b, CheckEpi{c, 2048});
+}
+
+// Rows of any alignment and extents of no multiple, split along K.
+struct CheckStagedNT : accy::gemm::Strided<0, 137, 1, 0, 1, 137> {
+  static constexpr int DT = 1;
+  static constexpr long BATCH = 1, M = 4101, N = 1003, K = 137;
+  static constexpr bool A_KC = true, B_KC = true;
+  static constexpr int BM = 128, BN = 128, SPLITS = 2;
+};
+extern "C" __global__ void __launch_bounds__(256) accy_check_gemm_staged(const u16_t* a, const u16_t* b, u16_t* c) {
+  accy::gemm::mma16_staged<CheckStagedNT>(a, b, CheckEpi{c, 1003});
 }

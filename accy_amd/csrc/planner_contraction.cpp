@@ -188,9 +188,9 @@ bool Planner::f32_direct(const GemmShape& gs) {
   return f32_layout_ok(gs) || large;
 }
 
-bool Planner::f32_staged_layout(const GemmShape& gs, bool& a_kc, bool& b_kc) {
-  auto operand = [](const Group& rows, const Group& k, bool& kc) {
-    auto whole = [](const Group& g) { return g.inner_str() == 1 && (g.single() || g.inner_ext() % 4 == 0); };
+bool Planner::staged_layout(const GemmShape& gs, int64_t vector, bool& a_kc, bool& b_kc) {
+  auto operand = [vector](const Group& rows, const Group& k, bool& kc) {
+    auto whole = [vector](const Group& g) { return g.inner_str() == 1 && (g.single() || g.inner_ext() % vector == 0); };
     kc = whole(k);
     return kc || whole(rows);
   };
@@ -209,7 +209,7 @@ bool Planner::f32_staged_layout(const GemmShape& gs, bool& a_kc, bool& b_kc) {
 Planner::Tile Planner::f32_tile(const GemmShape& gs) {
   bool a_kc, b_kc;
   Tile best;
-  if (!f32_staged_layout(gs, a_kc, b_kc)) return best;
+  if (!staged_layout(gs, 4, a_kc, b_kc)) return best;
   auto up = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
   const int64_t direct = up(gs.m, 256) * up(gs.n, 256) * gs.batch;
   if (f32_direct(gs) && (double)direct >= 0.8 * 256.0 * (double)up(direct, 256)) return best;
@@ -276,6 +276,18 @@ Planner::Tile Planner::dma_tile(const GemmShape& gs) {
   return best;
 }
 
+// The staged 16-bit kernel: 128 x 128 tiles, K split until two workgroups share every CU (each split keeps four
+// steps of 64 at least).
+Planner::Tile Planner::staged16_tile(const GemmShape& gs) {
+  auto up = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+  Tile t;
+  t.bm = t.bn = 128;
+  const int64_t groups = up(gs.m, 128) * up(gs.n, 128) * gs.batch, steps = up(gs.k, 64);
+  const int64_t want = std::max<int64_t>(1, std::min<int64_t>({512 / groups, steps / 4, 16}));
+  t.splits = (int)up(steps, up(steps, want));
+  return t;
+}
+
 bool Planner::gemm_eligible(const Op& op, GemmShape& gs) const {
   if (!opt_.allow_gemm) return false;
   DType d = op.result.dtype;
@@ -287,21 +299,17 @@ bool Planner::gemm_eligible(const Op& op, GemmShape& gs) const {
     bool akc, bkc;
     // Small and shallow contractions keep runCpu's serial k order: 962 x 67 x 130 takes 5.5 us there, a
     // launch's time, but a fold of k = 1000 on few threads hundreds (1000^3: 262 us).
-    return f32_direct(gs) || ((gs.k >= 128 || macs(gs) >= (double)(1ull << 23)) && f32_staged_layout(gs, akc, bkc));
+    return f32_direct(gs) || ((gs.k >= 128 || macs(gs) >= (double)(1ull << 23)) && staged_layout(gs, 4, akc, bkc));
   }
-  if (gs.multi) {
-    int dm, dn;
-    bool akc, bkc;
-    return dma_eligible(gs, dm, dn, akc, bkc);
-  }
-  auto ok8 = [](int64_t v) { return v % 8 == 0; };
-  bool a_kc = gs.a_k == 1 && ok8(gs.k) && (gs.m == 1 || ok8(gs.a_m));
-  bool a_mc = gs.a_m == 1 && ok8(gs.m) && (gs.k == 1 || ok8(gs.a_k));
-  bool b_kc = gs.b_k == 1 && ok8(gs.k) && (gs.n == 1 || ok8(gs.b_n));
-  bool b_nc = gs.b_n == 1 && ok8(gs.n) && (gs.k == 1 || ok8(gs.b_k));
-  if (!(a_kc || a_mc) || !(b_kc || b_nc)) return false;
-  if (!ok8(gs.a_b) || !ok8(gs.b_b) || !ok8(gs.a.offset) || !ok8(gs.b.offset)) return false;
-  return true;
+  int dm, dn;
+  bool akc, bkc;
+  if (dma_eligible(gs, dm, dn, akc, bkc)) return true;
+  // Through registers at any alignment; a shallow contraction of rows that are not 16-byte aligned keeps
+  // runCpu's serial k order, as small f32 ones do.
+  if (!staged_layout(gs, 8, akc, bkc)) return false;
+  auto ok8 = [](int64_t x) { return x % 8 == 0; };
+  const bool aligned = ok8(akc ? gs.k : gs.m) && ok8(bkc ? gs.k : gs.n);
+  return aligned || gs.k >= 32 || macs(gs) >= (double)(1ull << 20);
 }
 
 void Planner::mark_gemm_operands() {
@@ -549,8 +557,9 @@ void Planner::gemm(uint32_t v, const GemmShape& gs, const OutStrides& os) {
   int dm = 0, dn = 0;
   bool akc = gs.a_k == 1, bkc = gs.b_k == 1;
   const bool dma = d != DType::f32 && dma_eligible(gs, dm, dn, akc, bkc);
-  const Tile tile = d == DType::f32 ? f32_tile(gs) : dma ? dma_tile(gs) : Tile();
-  if (dma && tile.bm) {
+  const Tile tile = d == DType::f32 ? f32_tile(gs) : dma ? dma_tile(gs) : staged16_tile(gs);
+  if (d != DType::f32) {
+    if (!dma) staged_layout(gs, 8, akc, bkc);
     dm = tile.bm;
     dn = tile.bn;
   }
@@ -687,7 +696,7 @@ void Planner::gemm(uint32_t v, const GemmShape& gs, const OutStrides& os) {
         << gs.gb_n.fn("b_n");
     if (tile.bm) {
       bool a_kc = false, b_kc = false;
-      f32_staged_layout(gs, a_kc, b_kc);
+      staged_layout(gs, 4, a_kc, b_kc);
       src << "  static constexpr bool A_KC = " << (a_kc ? "true" : "false") << ", B_KC = " << (b_kc ? "true" : "false")
           << ";\n  static constexpr int BM = " << tile.bm << ", BN = " << tile.bn << ", WAVES_M = " << tile.wm
           << ", WAVES_N = " << tile.wn << ", WAVES_K = " << tile.wk << ", SPLITS = " << tile.splits << ";\n";
@@ -702,19 +711,8 @@ void Planner::gemm(uint32_t v, const GemmShape& gs, const OutStrides& os) {
         << "  accy::gemm::mma32f<Cfg_" << nm << ">(" << a << " + " << gs.a.offset << "L, " << b << " + "
         << gs.b.offset << "L, " << functor << ");\n}\n";
   } else {
-    // 256 x 256 x 64 tiles; the wave grid (4 x 2 waves of 64 x 128, or 2 x 2 waves of 128 x 128)
-    // can be overridden with ACCY_GEMM_WAVES=MxN for tuning.
-    const int BM = 256, BN = 256, BK = 64;
-    int WM = 2, WN = 2;
-    if (const char* e = std::getenv("ACCY_GEMM_WAVES")) {
-      int mm = 0, nn = 0;
-      if (std::sscanf(e, "%dx%d", &mm, &nn) == 2 && (mm == 2 || mm == 4) && (nn == 2 || nn == 4) && mm * nn <= 8) {
-        WM = mm;
-        WN = nn;
-      }
-    }
-    // Direct-to-LDS pipeline (dma_eligible: every row start 16-byte aligned); otherwise the
-    // register-staged kernel, which guards edges (single strides only).
+    // Direct-to-LDS pipeline (dma_eligible: every row start 16-byte aligned); otherwise the kernel that
+    // stages through registers.
     src << "struct Cfg_" << nm << " {\n"
         << "  static constexpr int DT = " << (d == DType::bf16 ? 0 : 1) << ";\n"
         << "  static constexpr long BATCH = " << gs.batch << ", M = " << gs.m << ", N = " << gs.n << ", K = " << gs.k << ";\n"
@@ -738,17 +736,12 @@ void Planner::gemm(uint32_t v, const GemmShape& gs, const OutStrides& os) {
         n_tiles.push_back(other);
     }
     const bool placeholder = n_tiles.size() > 1;
-    if (dma) {
-      src << "  static constexpr int BM = " << dm << ", BN = " << (placeholder ? "ACCY_N_TILE" : std::to_string(dn))
-          << ", STAGES = 4, GROUP_M = " << tile_group_m(gs.m, gs.n) << (split ? ", SPLITS = " + std::to_string(tile.splits) : "")
-          << ";\n};\n";
-    } else {
-      src << "  static constexpr int BM = " << BM << ", BN = " << BN << ", BK = " << BK << ", WAVES_M = " << WM
-          << ", WAVES_N = " << WN << ";\n};\n";
-    }
-    int threads = dma ? 256 : WM * WN * 64;
-    src << part_struct << "extern \"C\" __global__ void __launch_bounds__(" << threads << ") " << nm << "(" << kw.params()
-        << ") {\n  accy::gemm::" << (dma ? "mma16_dma" : "mma16") << "<Cfg_" << nm << ">(" << a << " + " << gs.a.offset
+    src << "  static constexpr int BM = " << dm << ", BN = " << (placeholder ? "ACCY_N_TILE" : std::to_string(dn));
+    if (dma) src << ", STAGES = 4, GROUP_M = " << tile_group_m(gs.m, gs.n);
+    if (!dma || split) src << ", SPLITS = " << tile.splits;
+    src << ";\n};\n";
+    src << part_struct << "extern \"C\" __global__ void __launch_bounds__(256) " << nm << "(" << kw.params()
+        << ") {\n  accy::gemm::" << (dma ? "mma16_dma" : "mma16_staged") << "<Cfg_" << nm << ">(" << a << " + " << gs.a.offset
         << "L, " << b << " + " << gs.b.offset << "L, " << functor << ");\n}\n";
     k.grid[2] = (uint32_t)tile.splits;
     k.source = src.str();
@@ -761,10 +754,8 @@ void Planner::gemm(uint32_t v, const GemmShape& gs, const OutStrides& os) {
       const std::string mark = "ACCY_N_TILE";
       k.source.replace(k.source.find(mark), mark.size(), std::to_string(dn));
     }
-    int64_t tiles = dma ? ((gs.m + dm - 1) / dm) * ((gs.n + dn - 1) / dn) : ((gs.m + BM - 1) / BM) * ((gs.n + BN - 1) / BN);
-    k.grid[0] = (uint32_t)tiles;
-    k.block[0] = threads;
-    k.shared_bytes = dma ? 0u : 2u * (BM + BN) * (BK + 8) * 2u;
+    k.grid[0] = (uint32_t)(((gs.m + dm - 1) / dm) * ((gs.n + dn - 1) / dn));
+    k.block[0] = 256;
   }
   if (k.source.empty()) k.source = src.str();
   k.name = nm;

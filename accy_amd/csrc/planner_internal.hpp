@@ -423,9 +423,12 @@ class Planner {
   // The f32 MFMA kernel's operand layouts: A K-contiguous, B N-contiguous, rows 16-byte aligned.
   static bool f32_layout_ok(const GemmShape& gs);
 
-  // Whether the staged f32 kernel can read the operands: K or the row axis of each has stride 1 (in whole
-  // vectors of four, where several axes make up the group).
-  static bool f32_staged_layout(const GemmShape& gs, bool& a_kc, bool& b_kc);
+  // Whether the kernels that stage through registers can read the operands: K or the row axis of each has
+  // stride 1 (in whole vectors, where several axes make up the group).
+  static bool staged_layout(const GemmShape& gs, int64_t vector, bool& a_kc, bool& b_kc);
+
+  // Tile and K split of the staged 16-bit kernel.
+  static Tile staged16_tile(const GemmShape& gs);
 
   // Tile and split of the staged f32 kernel; none (bm = 0) where the 256 x 256 direct-to-LDS kernel
   // applies and spreads its tiles over the CUs.
@@ -443,8 +446,7 @@ class Planner {
   // Repacks the operands of a large f32 contraction whose layout the MFMA kernel does not take.
   void pack_f32_operands(GemmShape& gs);
 
-  // The MFMA templates take 16-bit operands whose K or M/N stride is 1, with 8-element aligned rows
-  // (or, for operands whose groups span several axes, the direct-to-LDS kernel's layouts).
+  // The MFMA templates take operands whose K or M/N stride is 1.
   bool gemm_eligible(const Op& op, GemmShape& gs) const;
 
   // Marks dot operands that are not plain views of a buffer: they are materialised first (by the

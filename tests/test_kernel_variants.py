@@ -270,18 +270,43 @@ def test_direct_to_lds_contractions_within_the_summation_bound(shape, dtype):
         assert np.all(np.abs(got - ref) <= bound + 2.0 ** -24)
 
 
+# extents of no multiple of 8, K below one step and below a vector, shallow aligned rows, splits, batches
+STAGED_SHAPES = [(1, 33, 1), (7, 65, 9), (130, 67, 131), (129, 1001, 255), (200, 64, 264), (33, 2049, 7), (1, 40, 1000),
+                 (1100, 5, 1003), (16, 4097, 300), (3, 1030, 1887)]
+
+
 @pytest.mark.gpu
-def test_contraction_tail_ignores_what_lies_past_k():
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("layout", ["NN", "NT", "TN", "TT"])
+@pytest.mark.parametrize("shape", STAGED_SHAPES, ids=str)
+def test_staged_16bit_contractions_within_the_summation_bound(shape, layout, dtype):
+    """The bound of the direct-to-LDS contractions, for a plain and a batched contraction."""
+    m, k, n = shape
+    for batch in (0, 3):
+        prog = contraction(dtype, m, k, n, layout, batch)
+        src = hip.plan_source(prog)
+        assert "mma16_staged<" in src or "mma16_dma<" in src
+        ins, a, b, _ = contraction_inputs(dtype, m, k, n, layout, batch, False, m + k)
+        got = to_f32(hip_run(prog, ins)[0], dtype).astype(np.float64)
+        ref, r = a @ b, {"bf16": 2.0 ** -7, "f16": 2.0 ** -11}[dtype]
+        assert np.all(np.abs(got - ref) <= (k + 2) * 2.0 ** -24 * (np.abs(a) @ np.abs(b)) + r * np.abs(ref) + 2.0 ** -24)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,k,n,layout", [(130, 1005, 136, "TN"), (131, 1005, 137, "NN"), (131, 1005, 137, "TT"), (9, 70, 11, "NT")])
+def test_contraction_tail_ignores_what_lies_past_k(m, k, n, layout):
     """Infinities and NaN in the rows and columns that follow K in memory, or that the clamped loads
-    repeat, do not reach other outputs: row 0 of A and column 0 of B are not finite, everything else is."""
-    m, k, n = 130, 1005, 136
-    prog = contraction("bf16", m, k, n, "TN")
-    ins, a, b, _ = contraction_inputs("bf16", m, k, n, "TN", 0, False, 4)
+    repeat, do not reach other outputs: rows 0 and m - 1 of A and columns 0 and n - 1 of B are not finite,
+    everything else is."""
+    prog = contraction("bf16", m, k, n, layout)
+    ins, a, b, _ = contraction_inputs("bf16", m, k, n, layout, 0, False, 4)
     clean = hip_run(prog, ins)[0]
-    ins[0][:, 0] = 0x7f80      # +inf in row 0
-    ins[1][:, 0] = 0x7fc0      # NaN in column 0
+    rows = ins[0] if layout[0] == "N" else ins[0].T
+    cols = ins[1].T if layout[1] == "N" else ins[1]
+    rows[0] = rows[-1] = 0x7f80      # +inf
+    cols[0] = cols[-1] = 0x7fc0      # NaN
     got = hip_run(prog, ins)[0]
-    assert np.array_equal(got[1:, 1:], clean[1:, 1:])
+    assert np.array_equal(got[1:-1, 1:-1], clean[1:-1, 1:-1])
 
 
 def test_contractions_choose_their_tile_by_size():
