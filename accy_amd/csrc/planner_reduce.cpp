@@ -7,6 +7,13 @@ namespace planning {
 
 // ---- fold: one output per thread, serial left-to-right over the reduced index ----
 
+namespace {
+
+// A fold in chunks: a long range of few outputs, where a thread per output leaves most of the GPU idle.
+bool long_fold(uint64_t nred, uint64_t nout) { return nred >= 256 && nout * nred >= (1ull << 17) && nout < (1ull << 18); }
+
+}  // namespace
+
 void Planner::fold(uint32_t v) {
   const Op& op = g_.ops[v];
   const Type& in = g_.type(op.args[0]);
@@ -29,7 +36,7 @@ void Planner::fold(uint32_t v) {
   // Few outputs over a long reduced range: one serial fold per output cannot fill the GPU (and keeps
   // too few loads in flight), so the range is folded in chunks and the chunks' partials folded in
   // order (fold_chunked).
-  if (nred >= 1024 && nout * nred >= (1ull << 22) && nout < (1ull << 18) && chunk_identity(d, r)) {
+  if (long_fold(nred, nout) && chunk_identity(d, r)) {
     const int out = temp_slot(v);
     fold_chunked(v, out, in, red, keep, rdims, kdims, nout, nred, r, d);
     finish(v);
@@ -41,7 +48,7 @@ void Planner::fold(uint32_t v) {
   // pass in two launches, 7.5 us in one.)
   std::vector<uint32_t> group{v};
   const std::set<int64_t> axes(op.ints.begin(), op.ints.end());
-  const bool long_range = nred >= 1024 && nout * nred >= (1ull << 22) && nout < (1ull << 18);
+  const bool long_range = long_fold(nred, nout);
   constexpr size_t kMaxFolds = 4;
   for (uint32_t u = v + 1; !long_range && u < (uint32_t)g_.ops.size() && group.size() < kMaxFolds; ++u) {
     const Op& uo = g_.ops[u];
@@ -105,7 +112,7 @@ std::string Planner::fold_body(KernelWriter& w, const std::vector<uint32_t>& gro
     const std::string res = is_int(d) ? "(" + std::string(compute_type(d)) + ")" + acc : round_to(d, acc);
     stores << "    " << w.store(out, "o", d, res) << "\n";
   }
-  body << "    for (I r = 0; r < (I)" << nred << "; ++r) {\n" << steps.str() << "    }\n" << stores.str();
+  body << "#pragma unroll 8\n    for (I r = 0; r < (I)" << nred << "; ++r) {\n" << steps.str() << "    }\n" << stores.str();
   return body.str();
 }
 
@@ -136,51 +143,88 @@ void Planner::fold_chunked(uint32_t v, int out, const Type& in, const std::vecto
                            DType d) {
   const Op& op = g_.ops[v];
   const uint32_t B = 256;
-  uint64_t S = std::max<uint64_t>(2, ((1ull << 20) + nout - 1) / nout);
-  S = std::min<uint64_t>(S, std::min<uint64_t>(nred / 256, 65535));
-  const uint64_t chunk = (nred + S - 1) / S;
+  // Four adjacent outputs per lane where they are adjacent in the input too; 64 lanes x 4 waves per workgroup,
+  // each wave a quarter of the workgroup's chunk, put together in order in LDS.
+  const bool flat = kdims.size() == 1 && keep.back() + 1 == in.rank() && nout % 4 == 0;
+  const uint64_t VEC = flat ? 4 : 1, tiles = (nout + 64 * VEC - 1) / (64 * VEC);
+  // Two workgroups for every CU, of 32 reduced elements each at least. (3000 x 2048 bf16 summed over 3000:
+  // one output per lane and chunks of 256 and more took 24 us in two launches, now 13; 1142 x 1110, one thread per
+  // output before, 160 us, now 9.)
+  uint64_t S = std::min<uint64_t>({(512 + tiles - 1) / tiles, nred / 32, 65535});
+  S = std::max<uint64_t>(S, 1);
+  const uint64_t chunk = (nred + S - 1) / S, quarter = (chunk + 3) / 4;
   S = (nred + chunk - 1) / chunk;
   const DType pd = partial_dtype(d, r);
   const std::string at = acc_type(d, r);
-  const int part = slots_.add(SlotInfo::Temp, -1, pd, S * nout * dtype_size(pd));
+  const int part = S > 1 ? slots_.add(SlotInfo::Temp, -1, pd, S * nout * dtype_size(pd)) : -1;
   {
     KernelWriter w(g_, slots_, itype());
-    std::ostringstream body;
-    std::vector<std::string> kc = delinearize("o", kdims), rc = delinearize("r", rdims);
+    std::ostringstream body, pre;
+    std::vector<std::string> kc = flat ? std::vector<std::string>{"c"} : delinearize("c", kdims), rc = delinearize("r", rdims);
     std::vector<std::string> full(in.rank());
     for (size_t i = 0; i < red.size(); ++i) full[red[i]] = rc[i];
     for (size_t i = 0; i < keep.size(); ++i) full[keep[i]] = kc[i];
-    body << "    " << at << " acc = " << *chunk_identity(d, r) << ";\n"
-         << "    const I r0 = s * (I)" << chunk << ";\n"
-         << "    const I r1 = r0 + (I)" << chunk << " < (I)" << nred << " ? r0 + (I)" << chunk << " : (I)" << nred << ";\n"
-         << "#pragma unroll 8\n    for (I r = r0; r < r1; ++r) {\n";
-    Scope inner(body, "      ");
-    std::string x = w.value(op.args[0], full, inner);
-    body << "      acc = " << serial_fold_step(d, r, "acc", x) << ";\n    }\n"
-         << "    " << w.store(part, "s * (I)" + std::to_string(nout) + " + o", pd, "acc") << "\n";
-    std::string nm = name("fold_chunks", v);
+    std::string hoisted;
+    std::map<std::string, std::string> hoisted_var;
+    if (flat)
+      w.leaf_hook = [&](int slot, const std::string& off, DType ld, Scope& sc, std::string& res) -> bool {
+        const std::optional<std::string> base = quad_base(off);
+        if (!base) return false;
+        const std::string key = std::to_string(slot) + "|" + off;
+        auto hv = hoisted_var.find(key);
+        if (hv == hoisted_var.end()) {
+          const std::string q = "q" + std::to_string(hoisted_var.size());
+          hoisted += "      " + w.quad_load(slot, q, *base, ld) + "\n";
+          hv = hoisted_var.emplace(key, q).first;
+        }
+        res = w.tmp();
+        sc.out << sc.indent << "const " << compute_type(ld) << " " << res << " = " << KernelWriter::quad_elem(hv->second, "u", ld) << ";\n";
+        return true;
+      };
+    Scope inner(body, "        ");
+    const std::string x = w.value(op.args[0], full, inner);
+    body << "        mine[u] = " << serial_fold_step(d, r, "mine[u]", x) << ";\n";
+    w.leaf_hook = nullptr;
+    Scope outer(pre, "  ");
+    const std::string start = S > 1 ? *chunk_identity(d, r) : "(" + at + ")" + w.value(op.args[1], {}, outer);
+    const std::string res = is_int(d) ? "(" + std::string(compute_type(d)) + ")acc" : round_to(d, "acc");
+    const std::string store = S > 1 ? w.store(part, "s * (I)" + std::to_string(nout) + " + c", pd, "acc") : w.store(out, "c", d, res);
+    std::string nm = name(S > 1 ? "fold_chunks" : "fold", v);
     std::ostringstream src;
     src << "extern \"C\" __global__ void __launch_bounds__(" << B << ") " << nm << "(" << w.params() << ") {\n"
-        << "  typedef " << w.itype << " I;\n  const I s = (I)blockIdx.y;\n"
-        << "  for (I o = (I)blockIdx.x * " << B << " + threadIdx.x; o < (I)" << nout << "; o += (I)gridDim.x * " << B
-        << ") {\n" << body.str() << "  }\n}\n";
+        << "  typedef " << w.itype << " I;\n" << w.align_hints() << "  __shared__ " << at << " parts[4][" << 64 * VEC << "];\n"
+        << "  const I lane = (I)(threadIdx.x & 63), wave = (I)(threadIdx.x >> 6), s = (I)blockIdx.y;\n"
+        << "  const I c0 = ((I)blockIdx.x * 64 + lane) * " << VEC << ";\n"
+        << "  const I last = s * (I)" << chunk << " + (I)" << chunk << " < (I)" << nred << " ? s * (I)" << chunk << " + (I)" << chunk
+        << " : (I)" << nred << ";\n"
+        << "  const I r0 = s * (I)" << chunk << " + wave * (I)" << quarter << ";\n"
+        << "  const I r1 = r0 + (I)" << quarter << " < last ? r0 + (I)" << quarter << " : last;\n"
+        << "  " << at << " mine[" << VEC << "];\n#pragma unroll\n  for (int u = 0; u < " << VEC << "; ++u) {\n    const " << at
+        << " empty = " << *chunk_identity(d, r) << ";\n    mine[u] = empty;\n  }\n"
+        << "  if (c0 < (I)" << nout << ") {\n#pragma unroll 8\n    for (I r = r0; r < r1; ++r) {\n" << hoisted
+        << "#pragma unroll\n      for (int u = 0; u < " << VEC << "; ++u) {\n        const I c = c0 + u;\n" << body.str() << "      }\n    }\n  }\n"
+        << "#pragma unroll\n  for (int u = 0; u < " << VEC << "; ++u) parts[wave][lane * " << VEC << " + u] = mine[u];\n  __syncthreads();\n"
+        << pre.str() << "  for (I i = (I)threadIdx.x; i < " << 64 * VEC << "; i += " << B << ") {\n"
+        << "    const I c = (I)blockIdx.x * " << 64 * VEC << " + i;\n    if (c >= (I)" << nout << ") continue;\n    " << at << " acc = " << start
+        << ";\n#pragma unroll\n    for (int k = 0; k < 4; ++k) acc = " << serial_fold_step(d, r, "acc", "parts[k][i]") << ";\n    " << store << "\n  }\n}\n";
     KernelStep k;
     k.source = src.str();
     k.name = nm;
-    k.grid[0] = grid_for(nout, B, 65536);
+    k.grid[0] = (uint32_t)tiles;
     k.grid[1] = (uint32_t)S;
     k.block[0] = B;
     k.klass = "fold";
-    k.label = "fold:%" + std::to_string(v) + " chunks";
+    k.label = "fold:%" + std::to_string(v) + (S > 1 ? " chunks" : "");
     push(std::move(k), w);
   }
+  if (S == 1) return;
   {
     KernelWriter w(g_, slots_, itype());
     std::ostringstream body;
     Scope outer(body, "    ");
     std::string init = w.value(op.args[1], {}, outer);
     body << "    " << at << " acc = (" << at << ")" << init << ";\n"
-         << "    for (I s = 0; s < (I)" << S << "; ++s) acc = "
+         << "#pragma unroll 8\n    for (I s = 0; s < (I)" << S << "; ++s) acc = "
          << serial_fold_step(d, r, "acc", w.load(part, "s * (I)" + std::to_string(nout) + " + o", pd)) << ";\n";
     std::string res = is_int(d) ? "(" + std::string(compute_type(d)) + ")acc" : round_to(d, "acc");
     body << "    " << w.store(out, "o", d, res) << "\n";

@@ -345,3 +345,35 @@ def test_f32_attention_key_groups(case):
     ins = [rng.standard_normal((heads, n, 64)).astype(np.float32) for n in (queries, keys, keys)]
     exact = exact_attention(*ins, 0.125, causal, "f32")
     assert np.abs(hip_run(prog, ins)[0] - exact).max() <= 1e-4 * np.abs(exact).max()
+
+
+# ---- folds of a long leading range: chunks over workgroups and waves ----
+
+# (reduced, kept, and a kept axis before the reduced one): vectors of four outputs and single ones, one chunk,
+# quarters that the chunk does not fill, a last chunk shorter than a quarter, one output
+FOLDS = [(256, 512, 0), (257, 1110, 0), (1142, 1110, 0), (3000, 2048, 0), (131072, 1, 0), (40000, 4, 0), (300, 128, 5),
+         (16387, 12, 2), (999, 6, 30)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", FOLDS, ids=str)
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "i32"])
+def test_chunked_folds_of_a_leading_axis(shape, dtype):
+    """A computed operand. Integers, max and min bit for bit; a float sum within (n - 1) u sum|x| of float64
+    and the result's rounding (bf16 truncates: 2^-7)."""
+    r, c, p = shape
+    dims = ([("p", p)] if p else []) + [("r", r), ("c", c)]
+    prog = T.define("folds", [T.spec(dtype, *dims)], lambda b, a: [a[0].neg().sum("r"), a[0].max("r"), a[0].neg().min("r")])
+    assert "parts[4]" in hip.plan_source(prog)
+    rng = np.random.default_rng(r)
+    x = rng.standard_normal([e for _, e in dims]) * 100
+    x = x.astype(np.int32) if dtype == "i32" else W.to_dtype(x, dtype)
+    got, ref = hip_run(prog, [x]), oracle_run(prog, [x])
+    assert np.array_equal(got[1], ref[1]) and np.array_equal(got[2], ref[2])
+    if dtype == "i32":
+        assert np.array_equal(got[0], ref[0])
+        return
+    x64 = to_f32(x, dtype).astype(np.float64)
+    exact, size = -x64.sum(-2), np.abs(x64).sum(-2)
+    bound = (r - 1) * 2.0 ** -24 * size
+    assert np.all(np.abs(to_f32(got[0], dtype) - exact) <= bound + (2.0 ** -7 * (np.abs(exact) + bound) if dtype == "bf16" else 2.0 ** -24 * np.abs(exact)))
