@@ -28,7 +28,8 @@ HOST_SOURCES = ["ir.cpp", "wire.cpp", "lower.cpp", "planner.cpp", "planner_reduc
                 "planner_contraction.cpp", "planner_attention.cpp", "runtime.cpp", "tuning.cpp", "tune.cpp", "capi.cpp"]
 # Device sources embedded as text: (C++ symbol, file under csrc/kernels).
 EMBEDDED = [("kCommonDeviceSource", "common.h"), ("kGemmDeviceSource", "gemm.h"),
-            ("kAttentionDeviceSource", "attention.h"), ("kScatterDeviceSource", "scatter.h")]
+            ("kAttentionDeviceSource", "attention.h"), ("kScatterDeviceSource", "scatter.h"),
+            ("kDecodeDeviceSource", "decode.h")]
 # Packed-f32 instructions stay off in every device build; loops marked `#pragma unroll` unroll
 # whatever their size (as for the kernels compiled at run time).
 NO_PACKED_F32 = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-mllvm", "-pragma-unroll-threshold=65536"]

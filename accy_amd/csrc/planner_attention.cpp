@@ -79,8 +79,10 @@ bool Planner::match_attention(uint32_t pv, Attn& at) const {
   const Op& dv = g_.ops[pdiv];
   const size_t R = dv.result.rank();
   if (R < 2 || dv.result.dtype != dt) return false;
-  if (d.lhs_contract.size() != 1 || d.lhs_contract[0] != (int64_t)R - 1 || d.lhs_batch.size() != R - 2) return false;
-  for (size_t i = 0; i + 2 < R; ++i)
+  // [batch, query, key], or [batch, key] of one query per batch index
+  const size_t nb = d.lhs_batch.size();
+  if (d.lhs_contract.size() != 1 || d.lhs_contract[0] != (int64_t)R - 1 || (nb != R - 2 && nb != R - 1)) return false;
+  for (size_t i = 0; i < nb; ++i)
     if (d.lhs_batch[i] != (int64_t)i) return false;
   if (dv.kind != Kind::binary || (Binary)dv.code != Binary::div) return false;
   const uint32_t e = dv.args[0];
@@ -107,7 +109,7 @@ bool Planner::match_attention(uint32_t pv, Attn& at) const {
   if (g_.ops[x].kind == Kind::select) {
     const Op& sel = g_.ops[x];
     double f;
-    if (!splat_float(sel.args[2], f) || !(std::isinf(f) && f < 0) || !causal_mask(sel.args[0], R)) return false;
+    if (nb != R - 2 || !splat_float(sel.args[2], f) || !(std::isinf(f) && f < 0) || !causal_mask(sel.args[0], R)) return false;
     at.causal = true;
     inner.push_back(x);
     x = sel.args[1];
@@ -133,7 +135,7 @@ bool Planner::match_attention(uint32_t pv, Attn& at) const {
   if (!(at.scale > 0) || !std::isfinite(at.scale)) return false;
   const Op& qk = g_.ops[x];
   if (qk.kind != Kind::dot_general || qk.result.dtype != dt || qk.result.dims != dv.result.dims) return false;
-  if (qk.lhs_contract.size() != 1 || qk.rhs_contract.size() != 1 || qk.lhs_batch.size() != R - 2) return false;
+  if (qk.lhs_contract.size() != 1 || qk.rhs_contract.size() != 1 || qk.lhs_batch.size() != nb) return false;
   inner.push_back(x);
   std::sort(inner.begin(), inner.end());
   inner.erase(std::unique(inner.begin(), inner.end()), inner.end());
@@ -170,6 +172,96 @@ int Planner::free_axis(size_t rank, const std::vector<int64_t>& batch, const std
     f = (int)i;
   }
   return f;
+}
+
+bool Planner::decode_layout(uint32_t pv, const Attn& at, AttnLayout& L) const {
+  const Op& d = g_.ops[pv];
+  const Op& qk = g_.ops[at.qk];
+  if (at.causal || !resolve_view(qk.args[0], L.q) || !resolve_view(qk.args[1], L.k) || !resolve_view(d.args[1], L.v)) return false;
+  const Type& qt = g_.type(qk.args[0]);
+  const Type& kt = g_.type(qk.args[1]);
+  const Type& vt = g_.type(d.args[1]);
+  const int qf = free_axis(qt.rank(), qk.lhs_batch, qk.lhs_contract);
+  const int kf = free_axis(kt.rank(), qk.rhs_batch, qk.rhs_contract);
+  const int vf = free_axis(vt.rank(), d.rhs_batch, d.rhs_contract);
+  // one query: no query axis, or one of extent 1
+  if (qf == -2 || (qf >= 0 && qt.dims[(size_t)qf].extent != 1) || kf < 0 || vf < 0 || d.rhs_contract.size() != 1) return false;
+  const size_t qc = (size_t)qk.lhs_contract[0], kc = (size_t)qk.rhs_contract[0], vc = (size_t)d.rhs_contract[0];
+  const int64_t size = (int64_t)dtype_size(d.result.dtype), vec = 16 / size;
+  L.hd = qt.dims[qc].extent;
+  const int64_t lanes = L.hd / vec;  // per key row, 16 bytes each: a power of two
+  if (L.hd % vec != 0 || lanes < 1 || lanes > 64 || (lanes & (lanes - 1)) != 0) return false;
+  if (kt.dims[kc].extent != L.hd || vt.dims[(size_t)vf].extent != L.hd) return false;
+  if (L.q.strides[qc] != 1 || L.k.strides[kc] != 1 || L.v.strides[(size_t)vf] != 1) return false;
+  L.sq = 1;
+  L.sk = kt.dims[(size_t)kf].extent;
+  if (vt.dims[vc].extent != L.sk || L.sk == 0) return false;
+  L.k_s = L.k.strides[(size_t)kf];
+  L.v_s = L.v.strides[vc];
+  auto aligned = [vec](int64_t x) { return x % vec == 0; };
+  if (!aligned(L.k_s) || !aligned(L.v_s) || !aligned(L.q.offset) || !aligned(L.k.offset) || !aligned(L.v.offset)) return false;
+  L.nb = 1;
+  for (size_t i = 0; i < qk.lhs_batch.size(); ++i) {
+    const int64_t e = qt.dims[(size_t)qk.lhs_batch[i]].extent;
+    if (kt.dims[(size_t)qk.rhs_batch[i]].extent != e || vt.dims[(size_t)d.rhs_batch[i]].extent != e) return false;
+    L.extents.push_back(e);
+    L.q_b.push_back(L.q.strides[(size_t)qk.lhs_batch[i]]);
+    L.k_b.push_back(L.k.strides[(size_t)qk.rhs_batch[i]]);
+    L.v_b.push_back(L.v.strides[(size_t)d.rhs_batch[i]]);
+    if (!aligned(L.q_b.back()) || !aligned(L.k_b.back()) || !aligned(L.v_b.back())) return false;
+    L.nb *= e;
+  }
+  return L.nb > 0 && L.nb < (int64_t(1) << 31);
+}
+
+void Planner::attention_decode(uint32_t pv, const Attn& at, const AttnLayout& L) {
+  const DType d = g_.ops[pv].result.dtype;
+  const bool f32 = d == DType::f32;
+  const int64_t lanes = L.hd * (int64_t)dtype_size(d) / 16, step = 4 * 8 * (64 / lanes);  // decode.h step_keys
+  // Keys of a batch index over several workgroups until four share every CU, a step of keys each at least.
+  const int64_t steps = (L.sk + step - 1) / step;
+  const int64_t want = std::max<int64_t>(1, std::min<int64_t>({(1024 + L.nb - 1) / L.nb, steps, 64}));
+  const int64_t per = (steps + want - 1) / want, splits = (steps + per - 1) / per;
+  const int out = slots_.slot_of[pv] >= 0 ? slots_.slot_of[pv] : temp_slot(pv);
+  const std::string nm = name("decode", pv), elem = f32 ? "float" : "u16_t";
+  char sl[64];
+  std::snprintf(sl, sizeof sl, "%af", (double)(float)(at.scale * 1.4426950408889634));
+  std::ostringstream head;
+  head << "#include \"decode\"\nstruct Cfg_" << nm << " {\n  static constexpr int DT = " << (f32 ? 2 : d == DType::bf16 ? 0 : 1)
+       << ", HD = " << L.hd << ", SPLITS = " << splits << ";\n  static constexpr long SK = " << L.sk << ", NB = " << L.nb
+       << ", PER = " << per * step << ", K_S = " << L.k_s << ", V_S = " << L.v_s << ";\n  static constexpr float SL = " << sl << ";\n"
+       << "  static __device__ __forceinline__ long q_off(long b) { return " << batch_offset(L.extents, L.q_b, L.q.offset) << "; }\n"
+       << "  static __device__ __forceinline__ long k_off(long b) { return " << batch_offset(L.extents, L.k_b, L.k.offset) << "; }\n"
+       << "  static __device__ __forceinline__ long v_off(long b) { return " << batch_offset(L.extents, L.v_b, L.v.offset) << "; }\n};\n";
+  KernelWriter w(g_, slots_, "i64_t");
+  const std::string q = w.arg(L.q.slot, false), k = w.arg(L.k.slot, false), v = w.arg(L.v.slot, false);
+  const int part = splits > 1 ? slots_.add(SlotInfo::Temp, -1, DType::f32, (uint64_t)(L.nb * splits * (L.hd + 2)) * 4) : -1;
+  const std::string o = w.arg(splits > 1 ? part : out, true);
+  KernelStep ks;
+  ks.source = head.str() + "extern \"C\" __global__ void __launch_bounds__(256) " + nm + "(" + w.params() + ") {\n  accy::decode::attend<Cfg_" +
+              nm + ">(" + q + ", " + k + ", " + v + ", " + (splits > 1 ? "(" + elem + "*)nullptr, " + o : o + ", (float*)nullptr") + ");\n}\n";
+  ks.name = nm;
+  ks.grid[0] = (uint32_t)L.nb;
+  ks.grid[1] = (uint32_t)splits;
+  ks.block[0] = 256;
+  ks.klass = "attention";
+  ks.label = "decode:%" + std::to_string(pv);
+  ks.algorithmic_flops = 4.0 * (double)L.nb * (double)L.sk * (double)L.hd;
+  push(std::move(ks), w);
+  if (splits > 1) {
+    KernelWriter jw(g_, slots_, "i64_t");
+    const std::string p = jw.arg(part, false), r = jw.arg(out, true);
+    KernelStep js;
+    js.name = name("decode_join", pv);
+    js.source = head.str() + "extern \"C\" __global__ void __launch_bounds__(256) " + js.name + "(" + jw.params() +
+                ") {\n  accy::decode::join<Cfg_" + nm + ">(" + p + ", " + r + ");\n}\n";
+    js.grid[0] = (uint32_t)((L.nb * L.hd + 255) / 256);
+    js.block[0] = 256;
+    js.klass = "attention";
+    js.label = "join:%" + std::to_string(pv);
+    push(std::move(js), jw);
+  }
+  finish(pv);
 }
 
 bool Planner::attention_layout(uint32_t pv, const Attn& at, AttnLayout& L) const {

@@ -350,6 +350,11 @@ void Planner::dot(uint32_t v) {
       attention(v, fused->second, L);
       return;
     }
+    AttnLayout one;
+    if (decode_layout(v, fused->second, one)) {
+      attention_decode(v, fused->second, one);
+      return;
+    }
     // Operands the kernel cannot address: compute the absorbed values after all, in order.
     needed_[op.args[0]] = true;
     std::vector<uint32_t> inner = fused->second.inner;

@@ -500,6 +500,12 @@ class Planner {
 
   bool attention_layout(uint32_t pv, const Attn& at, AttnLayout& L) const;
 
+  // One query per batch index (kernels/decode.h): operands whose rows are whole 16-byte vectors, a power of
+  // two of them.
+  bool decode_layout(uint32_t pv, const Attn& at, AttnLayout& L) const;
+
+  void attention_decode(uint32_t pv, const Attn& at, const AttnLayout& L);
+
   // Element offset of flattened (row-major) batch index b for one operand.
   static std::string batch_offset(const std::vector<int64_t>& extents, const std::vector<int64_t>& strides,
                                   int64_t offset);

@@ -16,6 +16,7 @@ extern const char* const kCommonDeviceSource;
 extern const char* const kGemmDeviceSource;
 extern const char* const kAttentionDeviceSource;
 extern const char* const kScatterDeviceSource;
+extern const char* const kDecodeDeviceSource;
 
 namespace {
 
@@ -60,7 +61,8 @@ std::string full_kernel_source(const std::string& body) {
   std::string out = std::string(kCommonDeviceSource) + "\n";
   const std::pair<const char*, const char*> templates[] = {{"#include \"gemm\"\n", kGemmDeviceSource},
                                                            {"#include \"attention\"\n", kAttentionDeviceSource},
-                                                           {"#include \"scatter\"\n", kScatterDeviceSource}};
+                                                           {"#include \"scatter\"\n", kScatterDeviceSource},
+                                                           {"#include \"decode\"\n", kDecodeDeviceSource}};
   std::string rest = body;
   for (const auto& t : templates) {
     size_t p = rest.find(t.first);

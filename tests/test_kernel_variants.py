@@ -377,3 +377,59 @@ def test_chunked_folds_of_a_leading_axis(shape, dtype):
     exact, size = -x64.sum(-2), np.abs(x64).sum(-2)
     bound = (r - 1) * 2.0 ** -24 * size
     assert np.all(np.abs(to_f32(got[0], dtype) - exact) <= bound + (2.0 ** -7 * (np.abs(exact) + bound) if dtype == "bf16" else 2.0 ** -24 * np.abs(exact)))
+
+
+# ---- attention of one query per batch index ----
+
+# (heads, keys, dim, dtype): fewer keys than a step and than a lane group's rows, steps that the keys do not fill,
+# one workgroup per head and several, every number of lanes per row
+DECODES = [(3, 1, 128, "bf16"), (2, 37, 64, "f16"), (5, 128, 128, "bf16"), (600, 300, 64, "bf16"), (2, 5000, 128, "f16"),
+           (3, 1029, 64, "f32"), (2, 700, 128, "f32"), (2, 300, 256, "f32"), (4, 513, 256, "bf16"), (2, 999, 8, "f16"),
+           (1, 20000, 16, "bf16")]
+
+
+def decode(heads, keys, dim, dtype, query_axis):
+    def body(b, a):
+        q, k, v = a
+        s = q.contract(k, "dim").mul(b.full_float(T.Type(dtype, ()), 0.125))
+        e = s.sub(s.max("key")).exp()
+        return e.div(e.sum("key")).contract(v, "key")
+    one = [("query", 1)] if query_axis else []
+    return T.define("decode", [T.spec(dtype, ("head", heads), *one, ("dim", dim))]
+                    + [T.spec(dtype, head=heads, key=keys, dim=dim)] * 2, body)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("query_axis", [False, True])
+@pytest.mark.parametrize("case", DECODES, ids=str)
+def test_single_query_attention(case, query_axis):
+    """Against float64: f32 scores and sums (1e-5 of the largest magnitude), then the result's rounding (bf16
+    truncates: 2^-7; f16: 2^-11)."""
+    heads, keys, dim, dtype = case
+    prog = decode(heads, keys, dim, dtype, query_axis)
+    assert "accy::decode::attend<" in hip.plan_source(prog)
+    rng = np.random.default_rng(keys)
+    shapes = [(heads, 1, dim) if query_axis else (heads, dim), (heads, keys, dim), (heads, keys, dim)]
+    ins = [W.to_dtype(rng.standard_normal(sh), dtype) for sh in shapes]
+    exact = exact_attention(ins[0].reshape(heads, 1, dim), ins[1], ins[2], 0.125, False, dtype).reshape(shapes[0])
+    got = to_f32(hip_run(prog, ins)[0], dtype).astype(np.float64)
+    r = {"bf16": 2.0 ** -7, "f16": 2.0 ** -11, "f32": 2.0 ** -24}[dtype]
+    assert np.all(np.abs(got - exact) <= 1e-5 * np.abs(exact).max() + r * np.abs(exact))
+
+
+@pytest.mark.gpu
+def test_single_query_attention_special_values():
+    """The row past the last key in memory (the next head's first) and the last row, which clamped loads
+    repeat, are not finite: heads 0 and 2 stay exact, as does head 1 with a score of -inf."""
+    heads, keys, dim = 4, 131, 64
+    prog = decode(heads, keys, dim, "f32", False)
+    rng = np.random.default_rng(5)
+    q, k, v = (rng.standard_normal(s).astype(np.float32) for s in ((heads, dim), (heads, keys, dim), (heads, keys, dim)))
+    clean = hip_run(prog, [q, k, v])[0]
+    k[3, 0], v[3, 0] = np.nan, np.inf
+    q[1], k[1, 7] = np.abs(q[1]), -np.inf
+    got, ref = hip_run(prog, [q, k, v])[0], oracle_run(prog, [q, k, v])[0]
+    assert np.array_equal(got[0], clean[0]) and np.array_equal(got[2], clean[2])
+    assert np.allclose(got[1], ref[1], rtol=1e-4, atol=1e-5) and np.isnan(got[3]).all() and np.isnan(ref[3]).all()
+    v[2, -1] = np.inf              # the last key's own value: inf in the sum, in every dimension
+    assert np.array_equal(np.isinf(hip_run(prog, [q, k, v])[0][2]), np.isinf(oracle_run(prog, [q, k, v])[0][2]))
