@@ -5,14 +5,14 @@
 //
 // What bounds it is the table's copy (read and write of every row) and the updates read once; the
 // rows that many updates hit (a frequent token) are the serial part, so their updates are loaded
-// sixteen at a time ahead of the dependent additions. One thread per (p, q) walking all j, as before,
+// eight to 32 at a time (32 registers' worth) ahead of the dependent additions. One thread per (p, q) walking all j, as before,
 // took 989 us for 4096 updates of a 32000 x 1024 f32 table after a 43 us copy: one dependent load, add
 // and store per update and only 1024 threads in flight.
 //
 // A workgroup owns ROWS = LOOP x 4 x GROUPS rows of one p and one tile of q: LOOP x 4 blocks of GROUPS
 // consecutive rows, ROW_TILES blocks apart, so that the frequent tokens, whose ids are small in most
 // vocabularies, fall to different workgroups (four consecutive rows per workgroup took 194 us
-// instead of 87 us for the table above, with ids whose frequency falls as 1 / rank). It
+// instead of 87 us for the table above, now 66-77, with ids whose frequency falls as 1 / rank). It
 // reads the whole index list (from L2) and keeps the entries of its rows: (row, j) pairs in LDS, in
 // the order of j (ballot ranks). A batch of up to CAP of them is sorted stably by row (the rank of every key among
 // the batch: keys are row * CAP + position, all distinct), and each group of TC threads (along a row) then adds
@@ -26,6 +26,8 @@
 
 namespace accy {
 namespace scatter {
+
+struct alignas(16) Int4 { int v[4]; };
 
 constexpr int BLOCK = 256, RR = 4, CAP = 1024, STEP = 512;  // STEP indices per scan round (two per thread)
 
@@ -49,10 +51,12 @@ __device__ __forceinline__ void rows(const S& s) {
   constexpr int VEC = S::VEC, LOOP = S::LOOP;
   constexpr long VECS = S::POST / VEC;
   constexpr int TC = S::TC, GROUPS = BLOCK / TC, ROWS = LOOP * GROUPS * RR;
+  constexpr int DEPTH = TC <= 64 ? 16 : 32 / VEC;
   constexpr long COL_TILES = (VECS + TC - 1) / TC, ROW_TILES = (S::EXT + ROWS - 1) / ROWS;  // blocks of GROUPS rows a tile apart
   constexpr long TILES = ROW_TILES * COL_TILES * S::PRE;
   static_assert((long)ROWS * CAP < (1l << 31), "keys fit an int");
-  __shared__ int key[CAP], row_of[CAP];
+  __shared__ __attribute__((aligned(16))) int key[CAP];
+  __shared__ int row_of[CAP];
   __shared__ I pos[CAP], sorted[CAP];
   __shared__ int first[ROWS], last[ROWS];
   __shared__ int wave_count[BLOCK / 64];
@@ -113,14 +117,31 @@ __device__ __forceinline__ void rows(const S& s) {
       }
       if (n) {
         for (int i = tid; i < ROWS; i += BLOCK) first[i] = last[i] = 0;
+        if (tid < 4 && n + tid < CAP) key[n + tid] = 0x7fffffff;  // fills the last vector of four
         __syncthreads();
-        for (int e = tid; e < n; e += BLOCK) {
-          const int own = key[e];
-          int rank = 0;
-          for (int i = 0; i < n; ++i) rank += key[i] < own ? 1 : 0;
-          sorted[rank] = pos[e];
-          row_of[rank] = own / CAP;
+        // Every key's rank, CAP / BLOCK keys per thread against four at a time. (One at a time, each read waited
+        // for: 190 us for 8000 updates of a 50000 x 256 table,
+        // whose frequent rows one workgroup takes, now 76.)
+        int own[CAP / BLOCK], rank[CAP / BLOCK];
+#pragma unroll
+        for (int h = 0; h < CAP / BLOCK; ++h) {
+          own[h] = tid + h * BLOCK < n ? key[tid + h * BLOCK] : 0;
+          rank[h] = 0;
         }
+#pragma unroll 2
+        for (int i = 0; i < n; i += 4) {
+          const Int4 other = *(const Int4*)(key + i);
+#pragma unroll
+          for (int h = 0; h < CAP / BLOCK; ++h)
+#pragma unroll
+            for (int w = 0; w < 4; ++w) rank[h] += other.v[w] < own[h] ? 1 : 0;
+        }
+#pragma unroll
+        for (int h = 0; h < CAP / BLOCK; ++h)
+          if (tid + h * BLOCK < n) {
+            sorted[rank[h]] = pos[tid + h * BLOCK];
+            row_of[rank[h]] = own[h] / CAP;
+          }
         __syncthreads();
         for (int x = tid; x < n; x += BLOCK) {
           const int r = row_of[x];
@@ -143,7 +164,7 @@ __device__ __forceinline__ void rows(const S& s) {
           } else if (t > 0) {
             s.init(p, k, c0, v[i]);
           }
-          for (; e - x > 4; x += 16) add_run<16>(s, sorted, x, e, p, c0, v[i]);
+          for (; e - x > 4; x += DEPTH) add_run<DEPTH>(s, sorted, x, e, p, c0, v[i]);
           if (x < e) add_run<4>(s, sorted, x, e, p, c0, v[i]);
           s.store(p, k, c0, v[i]);
         }
