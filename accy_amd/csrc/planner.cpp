@@ -3,6 +3,7 @@
 // contractions and scatter_add; the other parts are in planner_*.cpp). See lower.cpp for the fusion
 // rules and the references.
 #include "planner_internal.hpp"
+#include "scratch.hpp"
 
 namespace accy {
 namespace planning {
@@ -578,13 +579,40 @@ Graph expand_sparse_cross_entropy(const Graph& g) {
 
 }  // namespace
 
+namespace {
+
+// Device scratch of one invocation: every temporary, a loop's two sets of carries and its body's scratch, each
+// 256-byte aligned (the executor's layout for accy_hip_invoke_device_scratch).
+uint64_t scratch_need(const Plan& plan) {
+  auto aligned = [](uint64_t bytes) { return (bytes + 255) & ~uint64_t(255); };
+  uint64_t n = 0;
+  for (const SlotInfo& s : plan.slots)
+    if (s.role == SlotInfo::Temp) n += aligned(s.bytes);
+  for (const Step& st : plan.steps) {
+    if (st.type != Step::Loop) continue;
+    const Plan& body = *st.loop.plan;
+    for (int s : body.input_slots) n += 2 * aligned(body.slots[(size_t)s].bytes);
+    n += aligned(scratch_need(body));
+  }
+  return n;
+}
+
+Plan lower_expanded(const Graph& g, const LowerOptions& options) {
+  Plan plan = planning::Planner(g, options).run();
+  if (!options.allow_split || scratch_need(plan) <= kScratchBytes) return plan;
+  // The partial sums of splits must not be what keeps a program out of the scratch array.
+  LowerOptions whole = options;
+  whole.allow_split = false;
+  Plan without = planning::Planner(g, whole).run();
+  return scratch_need(without) <= kScratchBytes ? std::move(without) : std::move(plan);
+}
+
+}  // namespace
+
 Plan lower(const Program& program, const LowerOptions& options) {
   for (const Op& op : program.ops)
-    if (op.kind == Kind::sparse_cross_entropy) {
-      const Graph expanded = expand_sparse_cross_entropy(program);
-      return planning::Planner(expanded, options).run();
-    }
-  return planning::Planner(program, options).run();
+    if (op.kind == Kind::sparse_cross_entropy) return lower_expanded(expand_sparse_cross_entropy(program), options);
+  return lower_expanded(program, options);
 }
 
 }  // namespace accy

@@ -220,7 +220,7 @@ void Planner::attention_decode(uint32_t pv, const Attn& at, const AttnLayout& L)
   const int64_t lanes = L.hd * (int64_t)dtype_size(d) / 16, step = 4 * 8 * (64 / lanes);  // decode.h step_keys
   // Keys of a batch index over several workgroups until four share every CU, a step of keys each at least.
   const int64_t steps = (L.sk + step - 1) / step;
-  const int64_t want = std::max<int64_t>(1, std::min<int64_t>({(1024 + L.nb - 1) / L.nb, steps, 64}));
+  const int64_t want = opt_.allow_split ? std::max<int64_t>(1, std::min<int64_t>({(1024 + L.nb - 1) / L.nb, steps, 64})) : 1;
   const int64_t per = (steps + want - 1) / want, splits = (steps + per - 1) / per;
   const int out = slots_.slot_of[pv] >= 0 ? slots_.slot_of[pv] : temp_slot(pv);
   const std::string nm = name("decode", pv), elem = f32 ? "float" : "u16_t";

@@ -206,7 +206,7 @@ bool Planner::staged_layout(const GemmShape& gs, int64_t vector, bool& a_kc, boo
 // 180 / 85 (19 as 32 x 64 tiles in 8 splits). The direct kernel's 256-wide tiles reach 137 TFLOP/s where
 // they fill every round and the staged ones 100-114, so the line between them lies at 0.8 full
 // rounds (2048^3, 64 tiles: 496 us).
-Planner::Tile Planner::f32_tile(const GemmShape& gs) {
+Planner::Tile Planner::f32_tile(const GemmShape& gs) const {
   bool a_kc, b_kc;
   Tile best;
   if (!staged_layout(gs, 4, a_kc, b_kc)) return best;
@@ -217,7 +217,7 @@ Planner::Tile Planner::f32_tile(const GemmShape& gs) {
   double best_cost = 0;
   for (Tile t : kTiles) {
     const int64_t tiles = up(gs.m, t.bm) * up(gs.n, t.bn) * gs.batch, steps = up(gs.k, 32 * t.wk);
-    for (int splits = 1; splits <= 64 && (splits == 1 || steps / splits >= 4); splits *= 2) {
+    for (int splits = 1; splits <= (opt_.allow_split ? 64 : 1) && (splits == 1 || steps / splits >= 4); splits *= 2) {
       const int64_t per = up(steps, splits), used = up(steps, per);  // every split has a step
       const double groups = (double)(tiles * used), rounds = (double)up(tiles * used, 256);
       const double k = (double)per * 32 * t.wk;
@@ -242,7 +242,7 @@ Planner::Tile Planner::f32_tile(const GemmShape& gs) {
 // them starts and drains in about 4 us, and a split costs a launch and the partials' traffic. Measured (one
 // box, us a pass, 256 x 256 against 128 x 128): 2048 x 8192 x 2048 134 / 66, 3000 x 2048 x 2048 45.6 / 34.1 (128 x 256:
 // 31.9), 1024^3 21.4 / 9.7, 512 x 4096 x 4096 69.6 / 30.8, 16 x 2048 x 8192 22.4 / 13.1.
-Planner::Tile Planner::dma_tile(const GemmShape& gs) {
+Planner::Tile Planner::dma_tile(const GemmShape& gs) const {
   auto up = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
   static const struct { int bm, bn; double rate; } kTiles[] = {{256, 256, 5.4}, {128, 256, 4.6}, {256, 128, 3.9}, {128, 128, 4.05}};
   const int64_t steps = up(gs.k, 32);
@@ -254,7 +254,7 @@ Planner::Tile Planner::dma_tile(const GemmShape& gs) {
     if (!dma_operand(gs.ga_m, gs.ga_k, gs.ga_b, gs.a.offset, gs.m % t.bm == 0 ? t.bm : 8, akc) ||
         !dma_operand(gs.gb_n, gs.gb_k, gs.gb_b, gs.b.offset, gs.n % t.bn == 0 ? t.bn : 8, bkc))
       continue;
-    for (int splits = 1; splits <= 8; ++splits) {
+    for (int splits = 1; splits <= (opt_.allow_split ? 8 : 1); ++splits) {
       if (steps % splits != 0 || (splits > 1 && steps / splits < 8)) continue;
       const double groups = (double)(up(gs.m, t.bm) * up(gs.n, t.bn) * gs.batch) * splits;
       const double full = std::floor(groups / 256.0), rest = groups - 256.0 * full;
@@ -278,12 +278,12 @@ Planner::Tile Planner::dma_tile(const GemmShape& gs) {
 
 // The staged 16-bit kernel: 128 x 128 tiles, K split until two workgroups share every CU (each split keeps four
 // steps of 64 at least).
-Planner::Tile Planner::staged16_tile(const GemmShape& gs) {
+Planner::Tile Planner::staged16_tile(const GemmShape& gs) const {
   auto up = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
   Tile t;
   t.bm = t.bn = 128;
   const int64_t groups = up(gs.m, 128) * up(gs.n, 128) * gs.batch, steps = up(gs.k, 64);
-  const int64_t want = std::max<int64_t>(1, std::min<int64_t>({512 / groups, steps / 4, 16}));
+  const int64_t want = opt_.allow_split ? std::max<int64_t>(1, std::min<int64_t>({512 / groups, steps / 4, 16})) : 1;
   t.splits = (int)up(steps, up(steps, want));
   return t;
 }

@@ -418,7 +418,7 @@ class Planner {
   };
 
   // Tile and K split of the direct-to-LDS 16-bit kernel.
-  static Tile dma_tile(const GemmShape& gs);
+  Tile dma_tile(const GemmShape& gs) const;
 
   // The f32 MFMA kernel's operand layouts: A K-contiguous, B N-contiguous, rows 16-byte aligned.
   static bool f32_layout_ok(const GemmShape& gs);
@@ -428,11 +428,11 @@ class Planner {
   static bool staged_layout(const GemmShape& gs, int64_t vector, bool& a_kc, bool& b_kc);
 
   // Tile and K split of the staged 16-bit kernel.
-  static Tile staged16_tile(const GemmShape& gs);
+  Tile staged16_tile(const GemmShape& gs) const;
 
   // Tile and split of the staged f32 kernel; none (bm = 0) where the 256 x 256 direct-to-LDS kernel
   // applies and spreads its tiles over the CUs.
-  static Tile f32_tile(const GemmShape& gs);
+  Tile f32_tile(const GemmShape& gs) const;
 
   // Extents and layout the 256 x 256 direct-to-LDS f32 kernel takes (large problems are repacked for it).
   static bool f32_direct(const GemmShape& gs);

@@ -270,6 +270,17 @@ def test_direct_to_lds_contractions_within_the_summation_bound(shape, dtype):
         assert np.all(np.abs(got - ref) <= bound + 2.0 ** -24)
 
 
+def test_partial_sums_do_not_keep_a_program_out_of_the_scratch_array():
+    """A temporary of 510 MiB and a contraction that would split: 518 MiB with its partial sums, more than the
+    512 MiB of accy_hip_invoke_device_scratch, so it is planned whole; half the rows split."""
+    def prog(rows):
+        def body(b, a):
+            e = a[0].sub(a[0].max("k")).exp()
+            return e.div(e.sum("k")).contract(a[1], "k")
+        return T.define("wide", [T.spec("bf16", m=rows, k=32000), T.spec("bf16", k=32000, n=64)], body)
+    assert "split_sum" in hip.plan_source(prog(4096)) and "split_sum" not in hip.plan_source(prog(8352))
+
+
 # extents of no multiple of 8, K below one step and below a vector, shallow aligned rows, splits, batches
 STAGED_SHAPES = [(1, 33, 1), (7, 65, 9), (130, 67, 131), (129, 1001, 255), (200, 64, 264), (33, 2049, 7), (1, 40, 1000),
                  (1100, 5, 1003), (16, 4097, 300), (3, 1030, 1887)]
