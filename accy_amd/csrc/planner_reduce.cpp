@@ -442,6 +442,16 @@ KernelStep Planner::gen_row(const RowShape& rs, const RowKernel& rk, bool commit
   const bool pairs_ok = commit && VEC == 4 && flat && row_leaves_16bit();
   auto keepable = [&](uint32_t threads) -> uint64_t { return !pairs_ok ? 64 : threads == 1024 ? 128 : 104; };
   size_t passes = (size_t)reduce_passes + (rk.full_vals.empty() ? 0 : 1);
+  // No more rows than CUs: as many threads per row as have a vector each, up to 1024, so that a CU has more than two
+  // waves. (us a pass, 128 threads / now: logsumexp 1 x 100000 f32 61 / 14, tone 200 x 16384 19.2 / 7.7, 1 x 8395 10.1 /
+  // 7.7; rows that 128 threads keep in registers stay at a launch's 7.3.)
+  if (kn <= 256)
+    for (uint32_t wide : {1024u, 512u, 256u})
+      if (lanes >= wide) {
+        B = wide;
+        E = (tn + (uint64_t)B * VEC - 1) / ((uint64_t)B * VEC);
+        break;
+      }
   // A row read by several passes is kept in registers when each thread holds at most 64 (128) of its
   // elements; a row too long for that with 128 threads takes 256, 512 or 1024 threads if that makes it
   // fit (read once instead of once per pass; four waves per SIMD still have 128 registers each).

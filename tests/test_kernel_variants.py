@@ -229,6 +229,24 @@ def test_ragged_rows_match_the_oracle(rows, cols, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows,cols,threads", [(1, 100003, 1024), (3, 80000, 1024), (256, 2050, 512), (9, 1030, 256), (257, 2050, 128)])
+def test_few_rows_take_more_threads(rows, cols, threads):
+    """Against float64. A thread adds at most cols / threads + 4 positive terms in a chain, the tree 10 more and the
+    exponential 2 ulp: 1e-5 relative holds up to 140 roundings."""
+    def body(b, a):
+        x = a[0]
+        m = x.max("c")
+        return [x.mul(x).sum("c"), m.add(x.sub(m).exp().sum("c").log()), m]
+    prog = T.define("few", [T.spec("f32", r=rows, c=cols)], body)
+    assert f" block {threads}\n" in hip.plan_source(prog)
+    x = (1.0 + np.abs(W.normal(cols, rows * cols))).astype(np.float32).reshape(rows, cols)
+    x64 = x.astype(np.float64)
+    ref = [(x64 * x64).sum(1), x64.max(1) + np.log(np.exp(x64 - x64.max(1, keepdims=True)).sum(1)), x64.max(1)]
+    for got, r in zip(hip_run(prog, [x]), ref):
+        assert np.all(np.abs(got - r) <= 1e-5 * r)
+
+
+@pytest.mark.gpu
 def test_ragged_rows_write_only_their_own_elements():
     """Exact integer rows of 67 and 70 next to each other: every element of the full-row output, and the
     sums, bit for bit."""
