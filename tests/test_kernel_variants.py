@@ -462,3 +462,40 @@ def test_single_query_attention_special_values():
     assert np.allclose(got[1], ref[1], rtol=1e-4, atol=1e-5) and np.isnan(got[3]).all() and np.isnan(ref[3]).all()
     v[2, -1] = np.inf              # the last key's own value: inf in the sum, in every dimension
     assert np.array_equal(np.isinf(hip_run(prog, [q, k, v])[0][2]), np.isinf(oracle_run(prog, [q, k, v])[0][2]))
+
+
+@pytest.mark.gpu
+def test_grouped_projections_with_a_k_tail():
+    """Three contractions of one activation in one launch whose K is no multiple of 32, against separate float64
+    products (the direct-to-LDS contractions' bound)."""
+    m, k, n = 256, 1000, 256
+    prog = T.define("qkv", [T.spec("bf16", m=m, k=k)] + [T.spec("bf16", k=k, n=n)] * 3,
+                    lambda b, a: [a[0].contract(w, "k") for w in a[1:]])
+    assert "mma16_dma_group<" in hip.plan_source(prog)
+    rng = np.random.default_rng(6)
+    ins = [W.to_dtype(rng.standard_normal(s), "bf16") for s in ((m, k), (k, n), (k, n), (k, n))]
+    x, *ws = (to_f32(i, "bf16").astype(np.float64) for i in ins)
+    for got, w in zip(hip_run(prog, ins), ws):
+        ref = x @ w
+        assert np.all(np.abs(to_f32(got, "bf16") - ref) <= (k + 2) * 2.0 ** -24 * (np.abs(x) @ np.abs(w)) + 2.0 ** -7 * np.abs(ref))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens,model,ffn", [(130, 264, 520), (3, 67, 131), (257, 1000, 3001)])
+def test_mlp_block_of_odd_sizes(tokens, model, ffn):
+    """RMS norm, two contractions, GELU and a residual at sizes that take every contraction kernel's edges; no
+    further from float64 than 1.5x the oracle's own error and one bf16 rounding of the largest value."""
+    def body(b, a):
+        x, g, w1, w2 = a
+        return x.add(W.gelu(b, W.rms_norm(b, x, g, "model", "bf16").contract(w1, "model"), "bf16").contract(w2, "ffn"))
+    prog = T.define("mlp", [T.spec("bf16", token=tokens, model=model), T.spec("bf16", model=model),
+                            T.spec("bf16", model=model, ffn=ffn), T.spec("bf16", ffn=ffn, model=model)], body)
+    rng = np.random.default_rng(tokens)
+    ins = [W.to_dtype(v, "bf16") for v in (rng.standard_normal((tokens, model)), 0.5 + rng.random(model),
+                                           rng.standard_normal((model, ffn)) / np.sqrt(model),
+                                           rng.standard_normal((ffn, model)) / np.sqrt(ffn))]
+    x, g, w1, w2 = (to_f32(i, "bf16").astype(np.float64) for i in ins)
+    h = x / np.sqrt((x * x).mean(1, keepdims=True) + 1e-5) * g @ w1
+    exact = x + 0.5 * h * (1 + np.tanh(0.7978845608028654 * (h + 0.044715 * h ** 3))) @ w2
+    got, ref = (to_f32(r[0], "bf16").astype(np.float64) for r in (hip_run(prog, ins), oracle_run(prog, ins)))
+    assert np.abs(got - exact).max() <= 1.5 * np.abs(ref - exact).max() + 2.0 ** -7 * np.abs(exact).max()
