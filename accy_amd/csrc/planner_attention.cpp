@@ -211,7 +211,7 @@ bool Planner::decode_layout(uint32_t pv, const Attn& at, AttnLayout& L) const {
     if (!aligned(L.q_b.back()) || !aligned(L.k_b.back()) || !aligned(L.v_b.back())) return false;
     L.nb *= e;
   }
-  return L.nb > 0 && L.nb < (int64_t(1) << 31);
+  return L.nb > 0 && launchable((uint64_t)L.nb, 256);  // a workgroup for every batch index
 }
 
 void Planner::attention_decode(uint32_t pv, const Attn& at, const AttnLayout& L) {

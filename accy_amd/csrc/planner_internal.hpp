@@ -81,6 +81,9 @@ inline uint32_t grid_for(uint64_t work_items, uint32_t block, uint64_t cap = 1u 
   return (uint32_t)std::min<uint64_t>(g, cap);
 }
 
+// HIP takes at most 2^32 - 1 work items along a grid dimension.
+inline bool launchable(uint64_t groups, uint64_t threads) { return groups < (1ull << 32) / threads; }
+
 // The body of a 64 x 64 tile of a transposing copy through LDS, for a kernel that has defined
 // `const long r0, c0` (the tile's first r and c). The source's r axis is contiguous (element (r, c)
 // at src[r + c * sc]), the destination's c axis (element (r, c) at dst[r * ds + c]); extents R and

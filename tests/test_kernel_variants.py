@@ -1,5 +1,7 @@
 """Kernel variants that the planner chooses by size, layout or neighbouring operations, each at the sizes
 where it can go wrong: compared with the CPU oracle, or with the float64 formula where stated."""
+import re
+
 import numpy as np
 import pytest
 
@@ -9,6 +11,11 @@ from accy_amd import workloads as W
 from conftest import exact_attention, hip_run, oracle_run, to_f32
 
 F32 = T.Type("f32", ())
+
+
+def work_items(prog):
+    """Work items along the first grid dimension of every kernel of a plan."""
+    return [int(g) * int(b) for g, b in re.findall(r"^ *// .* grid (\d+) block (\d+)$", hip.plan_source(prog), re.M)]
 
 
 # ---- reductions that share a pass over their row, folds that share a launch ----
@@ -444,6 +451,13 @@ def test_single_query_attention(case, query_axis):
     got = to_f32(hip_run(prog, ins)[0], dtype).astype(np.float64)
     r = {"bf16": 2.0 ** -7, "f16": 2.0 ** -11, "f32": 2.0 ** -24}[dtype]
     assert np.all(np.abs(got - exact) <= 1e-5 * np.abs(exact).max() + r * np.abs(exact))
+
+
+def test_single_query_attention_of_any_number_of_heads_can_be_launched():
+    """HIP refuses a launch of 2^32 work items: 2^24 heads of a workgroup each run as separate kernels."""
+    assert "accy::decode::" in hip.plan_source(decode((1 << 24) - 1, 4096, 8, "f16", False))
+    prog = decode(1 << 24, 4096, 8, "f16", False)
+    assert "accy::decode::" not in hip.plan_source(prog) and max(work_items(prog)) < 1 << 32
 
 
 @pytest.mark.gpu
