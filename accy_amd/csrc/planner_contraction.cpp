@@ -217,6 +217,7 @@ Planner::Tile Planner::f32_tile(const GemmShape& gs) const {
   double best_cost = 0;
   for (Tile t : kTiles) {
     const int64_t tiles = up(gs.m, t.bm) * up(gs.n, t.bn) * gs.batch, steps = up(gs.k, 32 * t.wk);
+    if (!launchable((uint64_t)(tiles / gs.batch), 64 * t.wm * t.wn * t.wk)) continue;
     for (int splits = 1; splits <= (opt_.allow_split ? 64 : 1) && (splits == 1 || steps / splits >= 4); splits *= 2) {
       const int64_t per = up(steps, splits), used = up(steps, per);  // every split has a step
       const double groups = (double)(tiles * used), rounds = (double)up(tiles * used, 256);
@@ -250,6 +251,7 @@ Planner::Tile Planner::dma_tile(const GemmShape& gs) const {
   double best_cost = 0;
   for (const auto& t : kTiles) {
     if (gs.multi && (gs.m % t.bm != 0 || gs.n % t.bn != 0)) continue;
+    if (!launchable((uint64_t)(up(gs.m, t.bm) * up(gs.n, t.bn)), 256)) continue;
     bool akc, bkc;
     if (!dma_operand(gs.ga_m, gs.ga_k, gs.ga_b, gs.a.offset, gs.m % t.bm == 0 ? t.bm : 8, akc) ||
         !dma_operand(gs.gb_n, gs.gb_k, gs.gb_b, gs.b.offset, gs.n % t.bn == 0 ? t.bn : 8, bkc))
@@ -283,6 +285,7 @@ Planner::Tile Planner::staged16_tile(const GemmShape& gs) const {
   Tile t;
   t.bm = t.bn = 128;
   const int64_t groups = up(gs.m, 128) * up(gs.n, 128) * gs.batch, steps = up(gs.k, 64);
+  if (!launchable((uint64_t)(groups / gs.batch), 256)) return Tile();
   const int64_t want = opt_.allow_split ? std::max<int64_t>(1, std::min<int64_t>({512 / groups, steps / 4, 16})) : 1;
   t.splits = (int)up(steps, up(steps, want));
   return t;
@@ -299,14 +302,14 @@ bool Planner::gemm_eligible(const Op& op, GemmShape& gs) const {
     bool akc, bkc;
     // Small and shallow contractions keep runCpu's serial k order: 962 x 67 x 130 takes 5.5 us there, a
     // launch's time, but a fold of k = 1000 on few threads hundreds (1000^3: 262 us).
-    return f32_direct(gs) || ((gs.k >= 128 || macs(gs) >= (double)(1ull << 23)) && staged_layout(gs, 4, akc, bkc));
+    return f32_direct(gs) || ((gs.k >= 128 || macs(gs) >= (double)(1ull << 23)) && staged_layout(gs, 4, akc, bkc) && f32_tile(gs).bm);
   }
   int dm, dn;
   bool akc, bkc;
-  if (dma_eligible(gs, dm, dn, akc, bkc)) return true;
+  if (dma_eligible(gs, dm, dn, akc, bkc)) return dma_tile(gs).bm != 0;
   // Through registers at any alignment; a shallow contraction of rows that are not 16-byte aligned keeps
   // runCpu's serial k order, as small f32 ones do.
-  if (!staged_layout(gs, 8, akc, bkc)) return false;
+  if (!staged_layout(gs, 8, akc, bkc) || !staged16_tile(gs).bm) return false;
   auto ok8 = [](int64_t x) { return x % 8 == 0; };
   const bool aligned = ok8(akc ? gs.k : gs.m) && ok8(bkc ? gs.k : gs.n);
   return aligned || gs.k >= 32 || macs(gs) >= (double)(1ull << 20);

@@ -415,7 +415,7 @@ class Planner {
 
   bool dma_eligible(const GemmShape& gs, int& dm, int& dn, bool& a_kc, bool& b_kc) const;
 
-  // Tile of a contraction kernel and the workgroups along K; bm = 0: none applies.
+  // Tile of a contraction kernel and the workgroups along K; bm = 0: none applies (or none whose grid HIP takes).
   struct Tile {
     int bm = 0, bn = 0, wm = 0, wn = 0, wk = 0, splits = 1;
   };

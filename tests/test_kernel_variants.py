@@ -353,6 +353,14 @@ def test_contractions_choose_their_tile_by_size():
     hip.plan_source(contraction("bf16", 136, 1001, 264, "TN"), compile=True)
 
 
+@pytest.mark.parametrize("dtype,m,k,n", [("f32", 1 << 31, 34, 16), ("f32", 1 << 30, 2, 1), ("bf16", 1 << 31, 40, 16),
+                                         ("bf16", 1 << 31, 8, 8), ("bf16", 1 << 31, 256, 8)])
+def test_contractions_of_any_size_can_be_launched(dtype, m, k, n):
+    """HIP refuses a launch of 2^32 work items: such a contraction runs on larger tiles or a grid-stride kernel."""
+    assert max(work_items(contraction(dtype, m, k, n))) < 1 << 32
+    assert max(work_items(contraction(dtype, n, k, m))) < 1 << 32
+
+
 # ---- f32 attention of head dimension 64: key groups ----
 
 # (heads, queries, keys, causal, waves, groups): fewer key blocks than groups, a last round that not every group
