@@ -318,9 +318,10 @@ bool Planner::gemm_eligible(const Op& op, GemmShape& gs) const {
 void Planner::mark_gemm_operands() {
   for (uint32_t v = 0; v < g_.ops.size(); ++v) {
     const Op& op = g_.ops[v];
-    if (!live_[v] || op.kind != Kind::dot_general || attn_.count(v)) continue;
+    if (!live_[v] || op.kind != Kind::dot_general) continue;
     if (op.result.dtype != DType::bf16 && op.result.dtype != DType::f16 && op.result.dtype != DType::f32) continue;
     for (uint32_t a : op.args) {
+      if (a == op.args[0] && attn_.count(v)) continue;  // the probabilities of a fused attention
       if (!view_chain_to_anchor(a)) needed_[a] = true;
     }
   }
