@@ -230,7 +230,7 @@ Planner::Tile Planner::f32_tile(const GemmShape& gs) const {
       if (!best.bm || cost < best_cost) {
         best = t;
         best.splits = (int)used;
-        best_cost = cost;
+        best.cost = best_cost = cost;
       }
     }
   }
@@ -288,7 +288,26 @@ Planner::Tile Planner::staged16_tile(const GemmShape& gs) const {
   if (!launchable((uint64_t)(groups / gs.batch), 256)) return Tile();
   const int64_t want = opt_.allow_split ? std::max<int64_t>(1, std::min<int64_t>({512 / groups, steps / 4, 16})) : 1;
   t.splits = (int)up(steps, up(steps, want));
+  t.cost = (double)up(groups, 512) * (1000.0 + 2500.0 * (double)steps);
   return t;
+}
+
+// Batches of a few rows and columns, and very many rows of few columns, leave a tile mostly empty; one thread per
+// output folding k in order is then faster. Its time in clocks: k dependent steps (without reuse between
+// lanes where each batch is one output), multiply-adds at what the lanes' loads allow (B read along n in vectors or not,
+// 16-bit rows in whole vectors along k or not), the operands from memory. Measured (us a pass, tiles / folded):
+// f32 65535 x (4 x 128 x 4) 397 / 48, 4194304 x 4 x 4 329 / 30, 1048576 x 16 x 8 87 / 32, 2 x 130 x 3 6.0 / 3.8, but
+// 20000 x 130 x 9 7.8 / 15.8, 10000 x (20 x 130 x 20) 100 / 129; bf16 65535 x (4 x 128 x 4) 348 / 36, 3000000 x 3 x 3
+// 98 / 16, but 1000 x (50 x 130 x 50) 16 / 115. A single round of the 16-bit kernel is as fast as a launch of the fold.
+bool Planner::fold_wins(const GemmShape& gs, const Tile& t, bool f32) {
+  const int64_t tiles = (gs.m + 127) / 128 * ((gs.n + 127) / 128) * gs.batch;
+  if (!f32 && tiles <= 512) return false;
+  const bool along_n = gs.gb_n.inner_str() == 1 && gs.gb_n.inner_ext() % 4 == 0, along_k = gs.k % 4 == 0;
+  const double rate = f32 ? (along_n ? 1300 : 700) : along_n ? (along_k ? 2200 : 1200) : (along_k ? 1800 : 1000);
+  const double step = gs.batch > 1 && gs.m == 1 && gs.n == 1 ? 350 : f32 ? 55 : 80;
+  const double bytes = (double)gs.batch * (double)gs.k * (double)(gs.m + gs.n) * (f32 ? 4 : 2);
+  const double rest = !f32 ? 1000 : gs.k % 64 ? 500 : -1500;  // a launch against the other's, the last K step's edges
+  return std::max({step * (double)gs.k, macs(gs) / rate, bytes / 1400}) < t.cost + rest;
 }
 
 bool Planner::gemm_eligible(const Op& op, GemmShape& gs) const {
@@ -302,17 +321,22 @@ bool Planner::gemm_eligible(const Op& op, GemmShape& gs) const {
     bool akc, bkc;
     // Small and shallow contractions keep runCpu's serial k order: 962 x 67 x 130 takes 5.5 us there, a
     // launch's time, but a fold of k = 1000 on few threads hundreds (1000^3: 262 us).
-    return f32_direct(gs) || ((gs.k >= 128 || macs(gs) >= (double)(1ull << 23)) && staged_layout(gs, 4, akc, bkc) && f32_tile(gs).bm);
+    if (f32_direct(gs)) return true;
+    if ((gs.k < 128 && macs(gs) < (double)(1ull << 23)) || !staged_layout(gs, 4, akc, bkc)) return false;
+    const Tile t = f32_tile(gs);
+    return t.bm && !fold_wins(gs, t, true);
   }
   int dm, dn;
   bool akc, bkc;
   if (dma_eligible(gs, dm, dn, akc, bkc)) return dma_tile(gs).bm != 0;
   // Through registers at any alignment; a shallow contraction of rows that are not 16-byte aligned keeps
   // runCpu's serial k order, as small f32 ones do.
-  if (!staged_layout(gs, 8, akc, bkc) || !staged16_tile(gs).bm) return false;
+  if (!staged_layout(gs, 8, akc, bkc)) return false;
+  const Tile t = staged16_tile(gs);
+  if (!t.bm) return false;
   auto ok8 = [](int64_t x) { return x % 8 == 0; };
   const bool aligned = ok8(akc ? gs.k : gs.m) && ok8(bkc ? gs.k : gs.n);
-  return aligned || gs.k >= 32 || macs(gs) >= (double)(1ull << 20);
+  return aligned || ((gs.k >= 32 || macs(gs) >= (double)(1ull << 20)) && !fold_wins(gs, t, false));
 }
 
 void Planner::mark_gemm_operands() {

@@ -418,7 +418,11 @@ class Planner {
   // Tile of a contraction kernel and the workgroups along K; bm = 0: none applies (or none whose grid HIP takes).
   struct Tile {
     int bm = 0, bn = 0, wm = 0, wn = 0, wk = 0, splits = 1;
+    double cost = 0;  // clocks, of the staged kernels
   };
+
+  // Whether one thread per output that folds k (dot_serial) is faster than the staged kernel with tile t.
+  static bool fold_wins(const GemmShape& gs, const Tile& t, bool f32);
 
   // Tile and K split of the direct-to-LDS 16-bit kernel.
   Tile dma_tile(const GemmShape& gs) const;

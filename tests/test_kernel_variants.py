@@ -178,7 +178,10 @@ def contraction_inputs(dtype, m, k, n, layout, batch, epilogue, seed):
 # one output, one row, few rows (splits), batches
 F32_SHAPES = [(1, 128, 1, 0), (1, 4096, 300, 0), (3, 129, 2, 0), (31, 1023, 66, 0), (33, 130, 65, 0), (127, 131, 129, 0),
               (962, 133, 130, 0), (3000, 3, 1001, 0), (2900, 1, 2899, 0), (64, 5000, 64, 0), (300, 2050, 70, 0),
-              (513, 1030, 770, 0), (5, 200, 37, 7), (130, 256, 66, 3)]
+              (513, 1030, 770, 0), (5, 200, 37, 7), (130, 256, 66, 3), (3, 1129, 2, 0), (33, 1130, 65, 0),
+              (127, 1131, 129, 0), (5, 1200, 37, 7)]
+# of these, folded by one thread per output (serial k order, within the same bound)
+F32_FOLDED = {(3, 129, 2, 0), (33, 130, 65, 0), (127, 131, 129, 0), (2900, 1, 2899, 0), (5, 200, 37, 7)}
 
 
 @pytest.mark.gpu
@@ -190,7 +193,7 @@ def test_staged_f32_contractions_within_the_summation_bound(shape, layout):
     m, k, n, batch = shape
     for epilogue in (False, True):
         prog = contraction("f32", m, k, n, layout, batch, epilogue)
-        assert "WAVES_K" in hip.plan_source(prog)
+        assert ("WAVES_K" in hip.plan_source(prog)) == (shape not in F32_FOLDED)
         ins, a, b, bias = contraction_inputs("f32", m, k, n, layout, batch, epilogue, m + k)
         got = hip_run(prog, ins)[0].astype(np.float64)
         ref, size = a @ b, np.abs(a) @ np.abs(b)
@@ -207,6 +210,17 @@ def test_f32_contractions_choose_their_kernel_by_size():
     assert "BM = 32" in plan(16, 4096, 4096) and "split_sum" in plan(16, 4096, 4096)
     assert "accy::gemm::" not in plan(200, 100, 200)
     hip.plan_source(contraction("f32", 16, 4096, 4096, epilogue=True), compile=True)
+
+
+@pytest.mark.parametrize("dtype,shape,folded", [
+    ("f32", (4, 128, 4, 65535), True), ("f32", (1 << 22, 4, 4, 0), True), ("f32", (1 << 20, 16, 8, 0), True),
+    ("f32", (1, 256, 1, 60000), True), ("f32", (2, 130, 3, 0), True), ("f32", (128, 128, 128, 0), False),
+    ("f32", (20000, 130, 9, 0), False), ("f32", (33, 130, 33, 1000), False), ("f32", (1, 1000000, 1, 0), False),
+    ("bf16", (4, 128, 4, 65535), True), ("bf16", (1 << 22, 4, 4, 0), True), ("bf16", (3000000, 3, 3, 0), True),
+    ("bf16", (2, 130, 3, 0), False), ("bf16", (50, 130, 50, 1000), False), ("bf16", (20000, 130, 9, 0), False)])
+def test_contractions_that_leave_tiles_empty_are_folded(dtype, shape, folded):
+    m, k, n, batch = shape
+    assert ("accy::gemm::" not in hip.plan_source(contraction(dtype, m, k, n, "NN", batch))) == folded
 
 
 # ---- rows whose length is no multiple of four, or that the threads' vectors do not cover exactly ----
