@@ -211,6 +211,12 @@ bool Planner::decode_layout(uint32_t pv, const Attn& at, AttnLayout& L) const {
     if (!aligned(L.q_b.back()) || !aligned(L.k_b.back()) || !aligned(L.v_b.back())) return false;
     L.nb *= e;
   }
+  // Very many heads of a few keys run unfused: a workgroup loads a step of keys whatever their number. (us a pass,
+  // fused / unfused: f32 200000 x 4 x 64 187 / 142, x 16 x 64 365 / 437, 60000 x 64 x 8 93 / 63, x 128 x 8 115 / 127,
+  // 6000 x 32 x 8 10.5 / 13.1; bf16 200000 x 8 x 64 314 / 197, x 32 x 64 473 / 567, x 128 x 16 548 / 378, while up to 65535
+  // heads, whose 16-bit contractions run on tiles, none is slower fused: 20000 x 4 x 64 33 / 100.)
+  const int64_t step = 4 * 8 * (64 / lanes);  // decode.h step_keys
+  if (L.sk < (lanes <= 2 ? step / 4 : step / 8) && L.nb > (d.result.dtype == DType::f32 ? 8192 : 65535)) return false;
   return L.nb > 0 && launchable((uint64_t)L.nb, 256);  // a workgroup for every batch index
 }
 

@@ -490,6 +490,15 @@ def test_single_query_attention_of_computed_operands(heads, keys, dim):
     assert np.abs(got - exact).max() <= 1.5 * np.abs(ref - exact).max() + 2.0 ** -7 * np.abs(exact).max()
 
 
+@pytest.mark.parametrize("heads,keys,dim,dtype,fused", [
+    (200000, 4, 64, "f32", False), (200000, 16, 64, "f32", True), (60000, 64, 8, "f32", False), (60000, 300, 8, "f32", True),
+    (6000, 4, 64, "f32", True), (200000, 8, 64, "bf16", False), (200000, 32, 64, "bf16", True), (60000, 4, 64, "bf16", True),
+    (1 << 20, 2, 8, "bf16", False), (300, 1, 8, "f16", True)])
+def test_single_query_attention_of_a_few_keys(heads, keys, dim, dtype, fused):
+    """A workgroup loads a whole step of keys: very many heads of a small part of one run unfused."""
+    assert ("accy::decode::" in hip.plan_source(decode(heads, keys, dim, dtype, False))) == fused
+
+
 def test_single_query_attention_of_any_number_of_heads_can_be_launched():
     """HIP refuses a launch of 2^32 work items: 2^24 heads of a workgroup each run as separate kernels."""
     assert "accy::decode::" in hip.plan_source(decode((1 << 24) - 1, 4096, 8, "f16", False))
