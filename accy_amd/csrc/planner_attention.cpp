@@ -211,12 +211,13 @@ bool Planner::decode_layout(uint32_t pv, const Attn& at, AttnLayout& L) const {
     if (!aligned(L.q_b.back()) || !aligned(L.k_b.back()) || !aligned(L.v_b.back())) return false;
     L.nb *= e;
   }
-  // Very many heads of a few keys run unfused: a workgroup loads a step of keys whatever their number. (us a pass,
-  // fused / unfused: f32 200000 x 4 x 64 187 / 142, x 16 x 64 365 / 437, 60000 x 64 x 8 93 / 63, x 128 x 8 115 / 127,
-  // 6000 x 32 x 8 10.5 / 13.1; bf16 200000 x 8 x 64 314 / 197, x 32 x 64 473 / 567, x 128 x 16 548 / 378, while up to 65535
-  // heads, whose 16-bit contractions run on tiles, none is slower fused: 20000 x 4 x 64 33 / 100.)
-  const int64_t step = 4 * 8 * (64 / lanes);  // decode.h step_keys
-  if (L.sk < (lanes <= 2 ? step / 4 : step / 8) && L.nb > (d.result.dtype == DType::f32 ? 8192 : 65535)) return false;
+  // Very many heads of a few keys run unfused: a workgroup loads a step of keys whatever their number, the more of them
+  // the fewer lanes a key takes. (us a pass, fused / unfused: f32 200000 x 4 x 64 187 / 142, x 16 x 64 365 / 437,
+  // 60000 x 64 x 8 93 / 63, x 128 x 8 115 / 127, 6000 x 32 x 8 10.5 / 13.1; bf16 200000 x 8 x 64 314 / 197, x 8 x 128
+  // 330 / 431, x 128 x 16 548 / 378, while up to 65535 heads, whose 16-bit contractions run on tiles, none is slower
+  // fused: 20000 x 4 x 64 33 / 100.)
+  const bool f32 = d.result.dtype == DType::f32;
+  if (L.sk * lanes < (lanes > 4 ? 128 : f32 || lanes > 2 ? 256 : 512) && L.nb > (f32 ? 8192 : 65535)) return false;
   return L.nb > 0 && launchable((uint64_t)L.nb, 256);  // a workgroup for every batch index
 }
 
@@ -416,18 +417,24 @@ double Planner::attention_pairs(const Attn& at, const AttnLayout& L) {
 
 void Planner::attention_f32(uint32_t pv, const Attn& at, const AttnLayout& L) {
   int out = slots_.slot_of[pv] >= 0 ? slots_.slot_of[pv] : temp_slot(pv);
-  // Eight waves: 128 queries in two key groups where that makes two workgroups for every CU and more, else
-  // 64 queries in four; four waves of 32 queries where even 64 would leave half of the CUs idle. (us a pass,
-  // 4 x 2 / 2 x 4 / 1 x 4: 64 x 1024 causal 91 / 102 / 145, 16 x 2048 causal 149 / 93 / 126, 1 x 4096 283 / 157 / 108; before,
-  // four waves of 128 queries: 158, 174, 325.)
-  const int64_t queries = L.nb * L.sq;
-  int waves = 1, groups = 4;
+  // 128 queries per workgroup where that makes two workgroups for every CU and more, else 64 where 32 would not
+  // leave half of the CUs idle, else 32. Key groups share a workgroup's queries so that every SIMD has two waves, but
+  // each takes 32 KB of LDS and at least a block of keys: fewer where workgroups abound or the keys are few.
+  // (us a pass with 1 / 2 / 4 groups. 32 queries: 4 x 2016 182 / 97 / 57, 16 x 2016 causal 187 / 106 / 124, 512 x 160
+  // 48 / 55 / 91, 1 x 32 4.8 / 5.3 / 6.5. 64: 16 x 2048 causal 228 / 122 / 93, 256 x 448 170 / 131 / 147, 2000 x 64
+  // 33 / 41 / 54. 128: 64 x 1024 causal 119 / 92, 700 x 128 34 / 39.)
+  const int64_t queries = L.nb * L.sq, blocks = L.sk / 32;
+  int waves = 1, groups = 1;
   if (L.sq % 128 == 0 && queries / 128 >= 512) {
     waves = 4;
-    groups = 2;
+    groups = blocks >= 16 ? 2 : 1;
   } else if (L.sq % 64 == 0 && queries / 64 > 128) {
     waves = 2;
+    groups = queries / 64 > 512 ? (blocks > 2 ? 2 : 1) : (blocks >= 16 ? 4 : 2);
+  } else {
+    groups = queries / 32 <= 256 ? 4 : (queries / 32 <= 1024 || blocks >= 8 ? 2 : 1);
   }
+  while (groups > 1 && (groups / 2 >= blocks || !launchable((uint64_t)(queries / (32 * waves)), (uint64_t)(64 * waves * groups)))) groups /= 2;
   KernelWriter w(g_, slots_, "i64_t");
   std::string q = w.arg(L.q.slot, false), k = w.arg(L.k.slot, false), v = w.arg(L.v.slot, false),
               o = w.arg(out, true);

@@ -379,8 +379,11 @@ def test_contractions_of_any_size_can_be_launched(dtype, m, k, n):
 
 # (heads, queries, keys, causal, waves, groups): fewer key blocks than groups, a last round that not every group
 # takes part in, more keys than queries and fewer, every workgroup shape
-F32_ATTENTION = [(1, 32, 32, False, 1, 4), (3, 32, 160, False, 1, 4), (2, 96, 96, True, 1, 4), (2, 128, 64, True, 1, 4),
-                 (70, 128, 96, False, 2, 4), (72, 192, 192, True, 2, 4), (512, 128, 160, True, 4, 2), (520, 128, 32, False, 4, 2)]
+F32_ATTENTION = [(1, 32, 32, False, 1, 1), (3, 32, 160, False, 1, 4), (2, 96, 96, True, 1, 4), (2, 128, 64, True, 1, 2),
+                 (70, 128, 96, False, 2, 2), (72, 192, 192, True, 2, 2), (512, 128, 160, True, 4, 1), (520, 128, 32, False, 4, 1),
+                 (9, 1056, 96, False, 1, 2), (513, 96, 64, True, 1, 1), (1030, 32, 288, False, 1, 2), (600, 64, 64, True, 2, 1),
+                 (600, 64, 96, False, 2, 2), (70, 128, 544, True, 2, 4), (65, 192, 512, False, 2, 4), (129, 512, 544, True, 4, 2),
+                 (512, 128, 512, False, 4, 2)]
 
 
 @pytest.mark.gpu
@@ -491,7 +494,8 @@ def test_single_query_attention_of_computed_operands(heads, keys, dim):
 
 
 @pytest.mark.parametrize("heads,keys,dim,dtype,fused", [
-    (200000, 4, 64, "f32", False), (200000, 16, 64, "f32", True), (60000, 64, 8, "f32", False), (60000, 300, 8, "f32", True),
+    (200000, 4, 64, "f32", False), (200000, 16, 64, "f32", True), (60000, 64, 8, "f32", False), (60000, 128, 8, "f32", True),
+    (200000, 8, 128, "bf16", True), (200000, 128, 16, "bf16", False),
     (6000, 4, 64, "f32", True), (200000, 8, 64, "bf16", False), (200000, 32, 64, "bf16", True), (60000, 4, 64, "bf16", True),
     (1 << 20, 2, 8, "bf16", False), (300, 1, 8, "f16", True)])
 def test_single_query_attention_of_a_few_keys(heads, keys, dim, dtype, fused):
