@@ -9,17 +9,19 @@
 // took 989 us for 4096 updates of a 32000 x 1024 f32 table after a 43 us copy: one dependent load, add
 // and store per update and only 1024 threads in flight.
 //
-// A workgroup owns ROWS = LOOP x 4 x GROUPS rows of one p and one tile of q: LOOP x 4 blocks of GROUPS
+// A workgroup owns ROWS = LOOP x 4 x KG rows of PG x PLOOP positions of p and one tile of q: LOOP x 4 blocks of KG
 // consecutive rows, ROW_TILES blocks apart, so that the frequent tokens, whose ids are small in most
 // vocabularies, fall to different workgroups (four consecutive rows per workgroup took 194 us
 // instead of 87 us for the table above, now 66-77, with ids whose frequency falls as 1 / rank). It
 // reads the whole index list (from L2) and keeps the entries of its rows: (row, j) pairs in LDS, in
 // the order of j (ballot ranks). A batch of up to CAP of them is sorted stably by row (the rank of every key among
 // the batch: keys are row * CAP + position, all distinct), and each group of TC threads (along a row) then adds
-// the runs of its four rows. When more entries remain, the next batch continues from the rows just written
+// the runs of its four rows. The lists are the same for every p: where KG groups cover the rows of one, the workgroup's
+// other groups take the next PG - 1 positions, and all of them PLOOP positions in turn. (1048576 x 8 f32 with
+// 64 updates along the last axis: 5886 us with a workgroup for every p, now 150; 300 with a thread for every p.) When more entries remain, the next batch continues from the rows just written
 // (the same thread wrote them).
 //
-// S supplies the sizes (NI updates, EXT rows, POST elements per row, PRE), TC, LOOP, VEC (4 when POST
+// S supplies the sizes (NI updates, EXT rows, POST elements per row, PRE), TC, KG, LOOP, PLOOP, VEC (4 when POST
 // is a multiple of it), index(j), plus(a, u), and on the VEC elements c0 .. c0 + VEC - 1 of a row
 // init(p, k, c0, v), again(p, k, c0, v), update(p, j, c0, v) and store(p, k, c0, v).
 #pragma once
@@ -50,10 +52,11 @@ __device__ __forceinline__ void rows(const S& s) {
   typedef typename S::T T;
   constexpr int VEC = S::VEC, LOOP = S::LOOP;
   constexpr long VECS = S::POST / VEC;
-  constexpr int TC = S::TC, GROUPS = BLOCK / TC, ROWS = LOOP * GROUPS * RR;
+  constexpr int TC = S::TC, KG = S::KG, PG = BLOCK / TC / KG, ROWS = LOOP * KG * RR;
   constexpr int DEPTH = TC <= 64 ? 16 : 32 / VEC;
-  constexpr long COL_TILES = (VECS + TC - 1) / TC, ROW_TILES = (S::EXT + ROWS - 1) / ROWS;  // blocks of GROUPS rows a tile apart
-  constexpr long TILES = ROW_TILES * COL_TILES * S::PRE;
+  constexpr long COL_TILES = (VECS + TC - 1) / TC, ROW_TILES = (S::EXT + ROWS - 1) / ROWS;  // blocks of KG rows a tile apart
+  constexpr long TILES = ROW_TILES * COL_TILES * ((S::PRE + PG * S::PLOOP - 1) / (PG * S::PLOOP));
+  static_assert(PG * KG * TC == BLOCK, "whole groups");
   static_assert((long)ROWS * CAP < (1l << 31), "keys fit an int");
   __shared__ __attribute__((aligned(16))) int key[CAP];
   __shared__ int row_of[CAP];
@@ -62,20 +65,22 @@ __device__ __forceinline__ void rows(const S& s) {
   __shared__ int wave_count[BLOCK / 64];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int group = tid / TC;
+  const int group = tid / TC % KG;
   for (long tile = blockIdx.x; tile < TILES; tile += gridDim.x) {
     const I mine = (I)(tile % ROW_TILES);
     // local row (block i, group g) <-> row of the table
-    auto row_at = [&](int i, int g) { return ((I)i * (I)ROW_TILES + mine) * GROUPS + g; };
-    const I p = (I)(tile / ROW_TILES / COL_TILES);
+    auto row_at = [&](int i, int g) { return ((I)i * (I)ROW_TILES + mine) * KG + g; };
+    const I p0 = (I)(tile / ROW_TILES / COL_TILES) * (PG * S::PLOOP) + tid / TC / KG;
     const I c0 = ((I)(tile / ROW_TILES % COL_TILES) * TC + (I)(tid % TC)) * VEC;
     const bool in_row = c0 < (I)S::POST;
+    // the last workgroup's positions may reach past the end
+    auto exists = [](I p) { return PG * S::PLOOP == 1 || p < (I)S::PRE; };
     T v[RR][VEC];
     // The first rows of the tile are loaded before the scan, so that the scan hides their latency.
 #pragma unroll
     for (int i = 0; i < RR; ++i) {
       const I k = row_at(i, group);
-      if (in_row && k < (I)S::EXT) s.init(p, k, c0, v[i]);
+      if (in_row && exists(p0) && k < (I)S::EXT) s.init(p0, k, c0, v[i]);
     }
     I next = 0;
     bool begun = false;
@@ -89,9 +94,9 @@ __device__ __forceinline__ void rows(const S& s) {
         for (int h = 0; h < 2; ++h) {
           const I j = next + wave * 128 + h * 64 + lane;
           const I k = j < (I)S::NI ? s.index(j) : (I)0;
-          const I block = k / GROUPS;
+          const I block = k / KG;
           const bool hit = j < (I)S::NI && block % (I)ROW_TILES == mine;
-          row[h] = hit ? (int)(block / (I)ROW_TILES) * GROUPS + (int)(k % GROUPS) : -1;
+          row[h] = hit ? (int)(block / (I)ROW_TILES) * KG + (int)(k % KG) : -1;
           hits[h] = __ballot(hit);
         }
         if (lane == 0) wave_count[wave] = __popcll(hits[0]) + __popcll(hits[1]);
@@ -150,23 +155,26 @@ __device__ __forceinline__ void rows(const S& s) {
         }
         __syncthreads();
       }
-      for (int t = 0; t < LOOP; ++t) {
+      for (int pl = 0; pl < S::PLOOP; ++pl) {
+        const I p = p0 + pl * PG;
+        for (int t = 0; t < LOOP; ++t) {
 #pragma unroll
-        for (int i = 0; i < RR; ++i) {
-          const I k = row_at(t * RR + i, group);
-          if (!in_row || k >= (I)S::EXT) continue;
-          const int r = (t * RR + i) * GROUPS + group;
-          int x = n ? first[r] : 0;
-          const int e = n ? last[r] : 0;
-          if (begun) {
-            if (x == e) continue;
-            s.again(p, k, c0, v[i]);
-          } else if (t > 0) {
-            s.init(p, k, c0, v[i]);
+          for (int i = 0; i < RR; ++i) {
+            const I k = row_at(t * RR + i, group);
+            if (!in_row || !exists(p) || k >= (I)S::EXT) continue;
+            const int r = (t * RR + i) * KG + group;
+            int x = n ? first[r] : 0;
+            const int e = n ? last[r] : 0;
+            if (begun) {
+              if (x == e) continue;
+              s.again(p, k, c0, v[i]);
+            } else if (t > 0 || pl > 0) {
+              s.init(p, k, c0, v[i]);
+            }
+            for (; e - x > 4; x += DEPTH) add_run<DEPTH>(s, sorted, x, e, p, c0, v[i]);
+            if (x < e) add_run<4>(s, sorted, x, e, p, c0, v[i]);
+            s.store(p, k, c0, v[i]);
           }
-          for (; e - x > 4; x += DEPTH) add_run<DEPTH>(s, sorted, x, e, p, c0, v[i]);
-          if (x < e) add_run<4>(s, sorted, x, e, p, c0, v[i]);
-          s.store(p, k, c0, v[i]);
         }
       }
       begun = true;

@@ -4,7 +4,7 @@
 #include "common.h"
 #include "scatter.h"
 
-template <class IT, int V, int THREADS, int L, long N, long ROWS, long WIDTH>
+template <class IT, int V, int THREADS, int GROUPS, int L, int PL, long N, long ROWS, long WIDTH>
 struct CheckTable {
   const float* in;
   const i32_t* ids;
@@ -13,7 +13,7 @@ struct CheckTable {
   typedef IT I;
   typedef float T;
   static constexpr long NI = N, EXT = ROWS, POST = WIDTH, PRE = 2;
-  static constexpr int VEC = V, TC = THREADS, LOOP = L;
+  static constexpr int VEC = V, TC = THREADS, KG = GROUPS, LOOP = L, PLOOP = PL;
   static __device__ __forceinline__ T plus(T a, T u) { return a + u; }
   __device__ __forceinline__ I index(I j) const { return (I)ids[j]; }
   __device__ __forceinline__ void init(I p, I k, I c0, T (&v)[VEC]) const {
@@ -30,9 +30,12 @@ struct CheckTable {
   }
 };
 
-extern "C" __global__ void __launch_bounds__(256) check_scatter_wide(CheckTable<i32_t, 4, 256, 1, 4096, 32000, 1024> t) {
+extern "C" __global__ void __launch_bounds__(256) check_scatter_wide(CheckTable<i32_t, 4, 256, 1, 1, 1, 4096, 32000, 1024> t) {
   accy::scatter::rows(t);
 }
-extern "C" __global__ void __launch_bounds__(256) check_scatter_narrow(CheckTable<i64_t, 1, 4, 8, 100000, 50000, 3> t) {
+extern "C" __global__ void __launch_bounds__(256) check_scatter_narrow(CheckTable<i64_t, 1, 4, 64, 8, 1, 100000, 50000, 3> t) {
+  accy::scatter::rows(t);
+}
+extern "C" __global__ void __launch_bounds__(256) check_scatter_positions(CheckTable<i32_t, 1, 1, 2, 1, 4, 64, 8, 1> t) {
   accy::scatter::rows(t);
 }

@@ -459,37 +459,55 @@ void Planner::scatter_add(uint32_t v) {
     store = "    " + w.store(out, at, d, "v[0]") + "\n";
   }
   // Threads along a row: enough for its vectors, more (idle while adding) where the rows are too few for
-  // a workgroup on every CU. Each workgroup reads the whole index list, so it owns more rows when
-  // tiles x updates passes 2^25 reads, while 1024 tiles remain (8192 updates of 100000 x 1024 f32: 209 us, 292 with
+  // a workgroup on every CU. Each workgroup reads the whole index list, so it owns more rows, then more leading
+  // positions, when tiles x updates passes 2^25 reads, while 1024 tiles remain (8192 updates of 100000 x 1024 f32: 209 us, 292 with
   // one tile of four rows for every workgroup; a limit of 2^24: 232).
   const uint64_t vecs = post / vec;
-  uint64_t tc = 1;
+  uint64_t tc = 1, kg = 1, loop = 1, ploop = 1;
+  auto up = [](uint64_t a, uint64_t b) { return (a + b - 1) / b; };
+  // Tiles with a workgroup's rows and leading positions. Where the positions are several, groups that the rows
+  // of one do not need take the next ones (a row to each group up to eight rows, whose updates then share cache
+  // lines: 1048576 x 8 f32 with 64 updates 150 us, 246 with four rows to a group; 65536 x 128 with 1000 the other way
+  // round: 1788 / 498), while 512 tiles remain.
+  auto tiles = [&](uint64_t rows, uint64_t positions) { return up((uint64_t)ext, rows) * up(vecs, tc) * up(pre, positions); };
+  auto shape = [&]() {
+    for (kg = 256 / tc; pre > 1 && kg > 1 && kg / 2 * (ext <= 8 ? 1 : 4) >= (uint64_t)ext;) kg /= 2;
+    while (kg < 256 / tc && tiles(kg * 4, 256 / tc / kg) < 512) kg *= 2;
+    return tiles(kg * 4, 256 / tc / kg);
+  };
   while (tc < 256 && tc < vecs) tc *= 2;
-  auto tiles_of = [&](uint64_t rows) { return ((uint64_t)ext + rows - 1) / rows * ((vecs + tc - 1) / tc) * pre; };
-  while (tc < 256 && tiles_of(256 / tc * 4) < 512) tc *= 2;
-  const uint64_t group_rows = 256 / tc * 4;
-  uint64_t loop = 1;
-  while (2 * loop * group_rows <= 4096 && tiles_of(2 * loop * group_rows) >= 1024 &&
-         tiles_of(loop * group_rows) > (1ull << 25) / ni)
-    loop *= 2;
+  while (shape() < 512 && tc < 256) tc *= 2;
+  const uint64_t rows = kg * 4, pg = 256 / tc / kg;
+  auto reads = [&]() { return tiles(loop * rows, ploop * pg) > (1ull << 25) / ni; };
+  while (2 * loop * rows <= 4096 && loop * rows < (uint64_t)ext && tiles(2 * loop * rows, pg) >= 1024 && reads()) loop *= 2;
+  // Positions in turn, also where sorting a tile's hits takes longer than its rows (16384 x 1000 f32 with 512 updates
+  // 471 us, now 104; 16384 x 8 x 256 with 64 the other way round: 247 / 272) or a workgroup has few elements.
+  const uint64_t own = std::min<uint64_t>((uint64_t)ext, loop * rows), width = std::min(post, tc * vec);
+  const double hits = (double)ni * (double)own / (double)ext;
+  const bool sorts = hits * hits >= 4.0 * (double)(own * width);
+  while (ploop < 1024 && ploop * pg < pre && tiles(loop * rows, 2 * ploop * pg) >= 1024 &&
+         (reads() || sorts || own * width * pg * ploop < 1024))
+    ploop *= 2;
   std::string nm = name("scatter", v);
   const KernelWriter::Members members = w.members();
   std::ostringstream src;
+  // Four waves per SIMD, so that 128 registers hold the updates in flight. (Left to itself the compiler takes 62
+  // for some shapes and waits: 100 x 3 f32 with 1000 updates 17.4 us, 12.6.)
   src << "#include \"scatter\"\n"
       << "struct Tab_" << nm << " {\n" << members.decls << "  typedef " << w.itype << " I;\n  typedef " << compute_type(d) << " T;\n"
       << "  static constexpr long NI = " << ni << ", EXT = " << ext << ", POST = " << post << ", PRE = " << pre << ";\n"
-      << "  static constexpr int VEC = " << vec << ", TC = " << tc << ", LOOP = " << loop << ";\n"
+      << "  static constexpr int VEC = " << vec << ", TC = " << tc << ", KG = " << kg << ", LOOP = " << loop << ", PLOOP = " << ploop << ";\n"
       << "  __device__ __forceinline__ I index(I j) const {\n" << index_body.str() << "    return (I)(" << idx << " < 0 ? 0 : ("
       << idx << " > " << ext - 1 << " ? " << ext - 1 << " : " << idx << "));\n  }\n"
       << "  static __device__ __forceinline__ T plus(T a, T u) { return " << plus << "; }\n" << init << update
       << "  __device__ __forceinline__ void again(I p, I k, I c0, T (&v)[VEC]) const {\n" << again << "  }\n"
       << "  __device__ __forceinline__ void store(I p, I k, I c0, const T (&v)[VEC]) const {\n" << store << "  }\n};\n"
-      << "extern \"C\" __global__ void __launch_bounds__(256) " << nm << "(" << w.params() << ") {\n"
+      << "extern \"C\" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) " << nm << "(" << w.params() << ") {\n"
       << "  accy::scatter::rows(Tab_" << nm << "{" << members.inits << "});\n}\n";
   KernelStep k;
   k.source = src.str();
   k.name = nm;
-  k.grid[0] = (uint32_t)std::min<uint64_t>(tiles_of(loop * group_rows), 1u << 20);
+  k.grid[0] = (uint32_t)std::min<uint64_t>(tiles(loop * rows, ploop * pg), 1u << 20);
   k.block[0] = 256;
   k.klass = "scatter";
   k.label = "scatter:%" + std::to_string(v);

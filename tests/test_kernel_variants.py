@@ -133,6 +133,31 @@ def test_scatter_add_keeps_the_order_of_the_updates(shape, dtype):
         assert np.array_equal(got.view(np.uint8), ref.view(np.uint8))   # every sum rounded in order: bit for bit
 
 
+# (positions before the axis, rows, row elements, updates): several positions per workgroup, with one element per row
+# and tails of vectors; positions in turn and several batches of hits
+POSITIONS = [(70001, 8, 0, 40), (66000, 5, 3, 33), (9001, 3, 260, 17), (5001, 512, 0, 14000)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", POSITIONS, ids=str)
+def test_scatter_add_over_many_leading_positions(shape):
+    pre, ext, post, n = shape
+    prog = scatter("f32", pre, ext, post, n)
+    src = hip.plan_source(prog)
+    tc, kg, loop, ploop = (int(x) for x in re.search(r"TC = (\d+), KG = (\d+), LOOP = (\d+), PLOOP = (\d+)", src).groups())
+    assert tc * kg < 256 or ploop > 1
+    rng = np.random.default_rng(ext)
+    ids = rng.integers(-1, ext + 1, n).astype(np.int32)
+    size = lambda e: [x for x in (pre, e, post) if x]
+    ins = [rng.random(size(ext), np.float32), ids, rng.random(size(n), np.float32)]
+    assert np.array_equal(hip_run(prog, ins)[0], oracle_run(prog, ins)[0])   # every sum rounded in order: bit for bit
+
+
+def test_scatter_add_of_short_rows_shares_its_lists_between_positions():
+    """A workgroup for every leading position would read and sort the index list once for each."""
+    assert max(work_items(scatter("f32", 1 << 20, 8, 0, 64))) <= (1 << 20) * 8 and max(work_items(scatter("f32", 1 << 20, 2, 4, 16))) <= (1 << 20) * 8
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("width", [64, 63])
 def test_scatter_add_of_gathered_updates(width):
