@@ -9,8 +9,10 @@ namespace planning {
 
 namespace {
 
-// A fold in chunks: a long range of few outputs, where a thread per output leaves most of the GPU idle.
-bool long_fold(uint64_t nred, uint64_t nout) { return nred >= 256 && nout * nred >= (1ull << 17) && nout < (1ull << 18); }
+// A fold in chunks: a long range of few outputs, where a thread per output leaves most of the GPU idle. From a wave
+// per SIMD on a thread per output is faster (us a pass, a thread / chunks: 300 x 262143 bf16 28 / 43, 600 x 100000 f32 35 / 40,
+// 1000 x 60000 f32 44 / 38).
+bool long_fold(uint64_t nred, uint64_t nout) { return nred >= 256 && nout * nred >= (1ull << 17) && nout < (1ull << 16); }
 
 }  // namespace
 
@@ -112,7 +114,9 @@ std::string Planner::fold_body(KernelWriter& w, const std::vector<uint32_t>& gro
     const std::string res = is_int(d) ? "(" + std::string(compute_type(d)) + ")" + acc : round_to(d, acc);
     stores << "    " << w.store(out, "o", d, res) << "\n";
   }
-  body << "#pragma unroll 8\n    for (I r = 0; r < (I)" << nred << "; ++r) {\n" << steps.str() << "    }\n" << stores.str();
+  // (Unrolled by eight, a single fold ends in up to seven rows waited for one by one: 250 x 300 9.9 us, 6.0 as the
+  // compiler unrolls it; two folds of 40 sines each 7.2 us, 7.8.)
+  body << (group.size() > 1 ? "#pragma unroll 8\n" : "") << "    for (I r = 0; r < (I)" << nred << "; ++r) {\n" << steps.str() << "    }\n" << stores.str();
   return body.str();
 }
 
@@ -144,15 +148,18 @@ void Planner::fold_chunked(uint32_t v, int out, const Type& in, const std::vecto
   const Op& op = g_.ops[v];
   const uint32_t B = 256;
   // Four adjacent outputs per lane where they are adjacent in the input too; 64 lanes x 4 waves per workgroup,
-  // each wave a quarter of the workgroup's chunk, put together in order in LDS.
+  // each wave a quarter of the workgroup's chunk, put together in order in LDS. Many outputs one by one take all 256
+  // lanes of one chunk instead, so that a workgroup reads whole lines (4000 x 30001 bf16: 66 us, 49; 1000 x 5001 the other way round: 6.7, 8.7).
   const bool flat = kdims.size() == 1 && keep.back() + 1 == in.rank() && nout % 4 == 0;
-  const uint64_t VEC = flat ? 4 : 1, tiles = (nout + 64 * VEC - 1) / (64 * VEC);
-  // Two workgroups for every CU, of 32 reduced elements each at least. (3000 x 2048 bf16 summed over 3000:
-  // one output per lane and chunks of 256 and more took 24 us in two launches, now 13; 1142 x 1110, one thread per
-  // output before, 160 us, now 9.)
-  uint64_t S = std::min<uint64_t>({(512 + tiles - 1) / tiles, nred / 32, 65535});
-  S = std::max<uint64_t>(S, 1);
-  const uint64_t chunk = (nred + S - 1) / S, quarter = (chunk + 3) / 4;
+  const uint64_t parts = !flat && nout >= 8192 && nred > 512 ? 1 : 4, lanes = B / parts;
+  const uint64_t VEC = flat ? 4 : 1, tiles = (nout + lanes * VEC - 1) / (lanes * VEC);
+  // One launch up to 512 reduced elements (256 x 4096 f32: 4.0 us, 6.0 in two launches); else two workgroups for every CU, of
+  // 32 reduced elements each at least, or one of vectors, since the chunks' partials are then folded one by one (100000 x 64
+  // f32: 512 chunks 37 us, 256 16; 1000000 x 4 43 and 66). (3000 x 2048 bf16 summed over 3000: one output per lane and
+  // chunks of 256 and more took 24 us in two launches, now 13; 1142 x 1110, one thread per output before, 160 us, now 9.)
+  const uint64_t want = flat && nred < (1ull << 18) ? 256 : 512;
+  uint64_t S = nred <= 512 ? 1 : std::min<uint64_t>({(want + tiles - 1) / tiles, nred / 32, 65535});
+  const uint64_t chunk = (nred + S - 1) / S, quarter = (chunk + parts - 1) / parts;
   S = (nred + chunk - 1) / chunk;
   const DType pd = partial_dtype(d, r);
   const std::string at = acc_type(d, r);
@@ -192,9 +199,9 @@ void Planner::fold_chunked(uint32_t v, int out, const Type& in, const std::vecto
     std::string nm = name(S > 1 ? "fold_chunks" : "fold", v);
     std::ostringstream src;
     src << "extern \"C\" __global__ void __launch_bounds__(" << B << ") " << nm << "(" << w.params() << ") {\n"
-        << "  typedef " << w.itype << " I;\n" << w.align_hints() << "  __shared__ " << at << " parts[4][" << 64 * VEC << "];\n"
-        << "  const I lane = (I)(threadIdx.x & 63), wave = (I)(threadIdx.x >> 6), s = (I)blockIdx.y;\n"
-        << "  const I c0 = ((I)blockIdx.x * 64 + lane) * " << VEC << ";\n"
+        << "  typedef " << w.itype << " I;\n" << w.align_hints() << "  __shared__ " << at << " parts[" << parts << "][" << lanes * VEC << "];\n"
+        << "  const I lane = (I)(threadIdx.x & " << lanes - 1 << "), wave = (I)(threadIdx.x / " << lanes << "), s = (I)blockIdx.y;\n"
+        << "  const I c0 = ((I)blockIdx.x * " << lanes << " + lane) * " << VEC << ";\n"
         << "  const I last = s * (I)" << chunk << " + (I)" << chunk << " < (I)" << nred << " ? s * (I)" << chunk << " + (I)" << chunk
         << " : (I)" << nred << ";\n"
         << "  const I r0 = s * (I)" << chunk << " + wave * (I)" << quarter << ";\n"
@@ -204,9 +211,9 @@ void Planner::fold_chunked(uint32_t v, int out, const Type& in, const std::vecto
         << "  if (c0 < (I)" << nout << ") {\n#pragma unroll 8\n    for (I r = r0; r < r1; ++r) {\n" << hoisted
         << "#pragma unroll\n      for (int u = 0; u < " << VEC << "; ++u) {\n        const I c = c0 + u;\n" << body.str() << "      }\n    }\n  }\n"
         << "#pragma unroll\n  for (int u = 0; u < " << VEC << "; ++u) parts[wave][lane * " << VEC << " + u] = mine[u];\n  __syncthreads();\n"
-        << pre.str() << "  for (I i = (I)threadIdx.x; i < " << 64 * VEC << "; i += " << B << ") {\n"
-        << "    const I c = (I)blockIdx.x * " << 64 * VEC << " + i;\n    if (c >= (I)" << nout << ") continue;\n    " << at << " acc = " << start
-        << ";\n#pragma unroll\n    for (int k = 0; k < 4; ++k) acc = " << serial_fold_step(d, r, "acc", "parts[k][i]") << ";\n    " << store << "\n  }\n}\n";
+        << pre.str() << "  for (I i = (I)threadIdx.x; i < " << lanes * VEC << "; i += " << B << ") {\n"
+        << "    const I c = (I)blockIdx.x * " << lanes * VEC << " + i;\n    if (c >= (I)" << nout << ") continue;\n    " << at << " acc = " << start
+        << ";\n#pragma unroll\n    for (int k = 0; k < " << parts << "; ++k) acc = " << serial_fold_step(d, r, "acc", "parts[k][i]") << ";\n    " << store << "\n  }\n}\n";
     KernelStep k;
     k.source = src.str();
     k.name = nm;

@@ -438,7 +438,18 @@ def test_f32_attention_key_groups(case):
 # (reduced, kept, and a kept axis before the reduced one): vectors of four outputs and single ones, one chunk,
 # quarters that the chunk does not fill, a last chunk shorter than a quarter, one output
 FOLDS = [(256, 512, 0), (257, 1110, 0), (1142, 1110, 0), (3000, 2048, 0), (131072, 1, 0), (40000, 4, 0), (300, 128, 5),
-         (16387, 12, 2), (999, 6, 30)]
+         (16387, 12, 2), (999, 6, 30), (513, 8193, 0), (1100, 8199, 0), (700, 2741, 3)]
+
+
+def test_folds_choose_their_split_by_size():
+    plan = lambda r, c: hip.plan_source(T.define("fold", [T.spec("f32", r=r, c=c)], lambda b, a: a[0].sum("r")))
+    for r, c in [(300, 262143), (300, 262144), (600, 100000), (255, 4096)]:     # a thread per output
+        assert "parts[" not in plan(r, c) and plan(r, c).count("__global__") == 1 and "unroll" not in plan(r, c)
+    for r, c in [(256, 512), (260, 5001), (512, 256)]:                           # one launch of workgroups
+        assert "parts[4]" in plan(r, c) and plan(r, c).count("__global__") == 1
+    for r, c, parts in [(100000, 64, 4), (1142, 1110, 4), (4000, 30001, 1), (1000, 9001, 1), (1000, 5001, 4)]:
+        assert f"parts[{parts}]" in plan(r, c) and plan(r, c).count("__global__") == 2
+    assert "s < (I)256" in plan(100000, 64)
 
 
 @pytest.mark.gpu
@@ -450,7 +461,7 @@ def test_chunked_folds_of_a_leading_axis(shape, dtype):
     r, c, p = shape
     dims = ([("p", p)] if p else []) + [("r", r), ("c", c)]
     prog = T.define("folds", [T.spec(dtype, *dims)], lambda b, a: [a[0].neg().sum("r"), a[0].max("r"), a[0].neg().min("r")])
-    assert "parts[4]" in hip.plan_source(prog)
+    assert f"parts[{1 if c * max(p, 1) > 8192 and r > 512 else 4}]" in hip.plan_source(prog)
     rng = np.random.default_rng(r)
     x = rng.standard_normal([e for _, e in dims]) * 100
     x = x.astype(np.int32) if dtype == "i32" else W.to_dtype(x, dtype)
