@@ -255,10 +255,18 @@ std::string KernelWriter::store(int slot, const std::string& off, DType d, const
   }
 }
 
-bool KernelWriter::cosine_too(uint32_t arg) const {
-  for (const Op& op : g_.ops)
-    if (op.kind == Kind::unary && (Unary)op.code == Unary::cos && op.args[0] == arg) return true;
-  return false;
+void share_reductions(std::string& source) {
+  const std::string sine = "accy::sin_f32(", cosine = "accy::cos_f32(", both = "accy::sin_with_cos_f32(";
+  for (size_t at = source.find(sine); at != std::string::npos; at = source.find(sine, at + 1)) {
+    const size_t arg = at + sine.size();
+    const std::string call = cosine + source.substr(arg, source.find(')', arg) + 1 - arg);
+    // beside it: no loop begins in between
+    auto beside = [&](size_t cos) {
+      if (cos == std::string::npos) return false;
+      return source.substr(std::min(at, cos), std::max(at, cos) - std::min(at, cos)).find("for (") == std::string::npos;
+    };
+    if (beside(source.find(call, at)) || beside(source.rfind(call, at))) source.replace(at, sine.size(), both);
+  }
 }
 
 std::string KernelWriter::value(uint32_t vid, const std::vector<std::string>& coords, Scope& sc) {
@@ -314,7 +322,7 @@ std::string KernelWriter::value(uint32_t vid, const std::vector<std::string>& co
           case Unary::log: e = (f ? "logf(" : "log(") + x + ")"; break;
           case Unary::sqrt: e = (f ? "sqrtf(" : "sqrt(") + x + ")"; break;
           case Unary::tanh: e = (f ? "accy::tanh_f32(" : "tanh(") + x + ")"; break;
-          case Unary::sin: e = (!f ? "sin(" : cosine_too(op.args[0]) ? "accy::sin_with_cos_f32(" : "accy::sin_f32(") + x + ")"; break;
+          case Unary::sin: e = (f ? "accy::sin_f32(" : "sin(") + x + ")"; break;
           case Unary::cos: e = (f ? "accy::cos_f32(" : "cos(") + x + ")"; break;
           case Unary::tan: e = (f ? "tanf(" : "tan(") + x + ")"; break;
         }

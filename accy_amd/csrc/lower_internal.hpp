@@ -53,6 +53,11 @@ struct Scope {
   Scope(std::ostringstream& o, std::string ind) : out(o), indent(std::move(ind)) {}
 };
 
+// Gives the sines of a finished kernel whose argument, the same variable, has its cosine taken there too the form that
+// shares the cosine's reduction (common.h sin_with_cos_f32). A cosine of the value in another kernel, or evaluated again in
+// another pass of this one, shares nothing.
+void share_reductions(std::string& source);
+
 // Builds the body of one generated kernel: collects the slots it touches (its parameters) and
 // emits each value at a multi-index given as C expressions.
 class KernelWriter {
@@ -88,7 +93,6 @@ class KernelWriter {
   std::string itype;
 
  private:
-  bool cosine_too(uint32_t arg) const;  // some operation takes the cosine of value `arg`
   const Graph& g_;
   Slots& slots_;
   int ntmp_ = 0;

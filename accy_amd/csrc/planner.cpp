@@ -125,6 +125,7 @@ std::string Planner::name(const char* klass, uint32_t v) {
 }
 
 void Planner::push(KernelStep k, const KernelWriter& w) {
+  share_reductions(k.source);
   k.args = w.args;
   double bytes = 0;
   for (size_t i = 0; i < w.args.size(); ++i) bytes += (double)plan_.slots[(size_t)w.args[i]].bytes;

@@ -320,6 +320,7 @@ bool Planner::row_group(uint32_t r0) {
 }
 
 void Planner::push_row(KernelStep k) {
+  share_reductions(k.source);
   k.args = last_args_;
   double bytes = 0;
   for (int s : k.args) bytes += (double)plan_.slots[(size_t)s].bytes;

@@ -73,6 +73,25 @@ def test_folds_that_share_a_launch_keep_their_order(r, c, dtype):
         assert np.array_equal(g, f)     # serial left-to-right folds: bit for bit
 
 
+def sine_or_cosine(b, a):
+    """Both of every element in one kernel: [sine, cosine] along a last axis."""
+    n = a[0].ty.dims[0][1]
+    first = b.iota("f32", "k", ("k", 2), ("i", n)).compare("lt", b.full_float(F32, 0.5))
+    return first.select(a[0].sin(), a[0].cos())
+
+
+def test_sines_share_a_reduction_only_with_a_cosine_beside_them():
+    """In two kernels, or two passes of one, each evaluates its own: sin_f32 is the cheaper form alone."""
+    spec = [T.spec("f32", r=64, i=4096)]
+    for body in (lambda b, a: [a[0].sin(), a[0].cos()], lambda b, a: [a[0].sin().sum("i"), a[0].cos()],
+                 lambda b, a: [a[0].sin().sum("r"), a[0].cos().sum("i")]):
+        src = hip.plan_source(T.define("pair", spec, body))
+        assert "sin_with_cos_f32" not in src and "sin_f32" in src and "cos_f32" in src
+    for body in (lambda b, a: [a[0].sin().sum("i"), a[0].cos().sum("i")], lambda b, a: a[0].sin().mul(a[0].cos())):
+        src = hip.plan_source(T.define("pair", spec, body))
+        assert "sin_with_cos_f32" in src and "accy::sin_f32" not in src
+
+
 @pytest.mark.gpu
 def test_sine_and_cosine_of_one_value_against_float64():
     """The pair shares one reduction: each within 2 ulp of float64 below 2^17, the library's beyond,
@@ -83,14 +102,14 @@ def test_sine_and_cosine_of_one_value_against_float64():
                         np.nextafter(near, np.float32(np.inf)), np.geomspace(1e-30, 1, 2000),
                         -np.geomspace(1e-30, 1, 2000), [1e6, -3.5e7, 1e30]]).astype(np.float32)
     xs = np.concatenate([x, np.array([np.inf, -np.inf, np.nan, -0.0, 0.0], np.float32)])
-    prog = T.define("pair", [T.spec("f32", i=len(xs))], lambda b, a: [a[0].sin(), a[0].cos()])
+    prog = T.define("pair", [T.spec("f32", i=len(xs))], sine_or_cosine)
     assert "sin_with_cos_f32" in hip.plan_source(prog)
-    for got, f64 in zip(hip_run(prog, [xs]), (np.sin, np.cos)):
+    for got, f64 in zip(hip_run(prog, [xs])[0].T, (np.sin, np.cos)):
         ref = f64(x.astype(np.float64))
         ulp = np.spacing(np.abs(ref).astype(np.float32)).astype(np.float64)
         assert (np.abs(got[:len(x)].astype(np.float64) - ref) / ulp).max() <= 2.0
         assert np.isnan(got[len(x):len(x) + 3]).all()
-    s, c = hip_run(prog, [xs])
+    s, c = hip_run(prog, [xs])[0].T
     assert np.signbit(s[-2]) and s[-2] == 0 and s[-1] == 0 and not np.signbit(s[-1]) and c[-2] == c[-1] == 1.0
 
 
