@@ -311,6 +311,9 @@ class Planner {
   std::map<uint32_t, int> row_keep_;
   // Every leaf that several passes of the last trial read is a row of 16-bit floats.
   bool row_leaves_16bit() const;
+  // A transcendental or a division; and whether evaluating a value inline takes one.
+  bool costly(uint32_t v) const;
+  bool costly_inside(uint32_t v) const;
   void keep_row_values(const RowShape& rs, const RowKernel& rk, uint64_t per_thread, bool pairs);
 
   // ---- launch tuning ----

@@ -155,10 +155,12 @@ void Planner::fold_chunked(uint32_t v, int out, const Type& in, const std::vecto
   const uint64_t VEC = flat ? 4 : 1, tiles = (nout + lanes * VEC - 1) / (lanes * VEC);
   // One launch up to 512 reduced elements (256 x 4096 f32: 4.0 us, 6.0 in two launches); else two workgroups for every CU, of
   // 32 reduced elements each at least, or one of vectors, since the chunks' partials are then folded one by one (100000 x 64
-  // f32: 512 chunks 37 us, 256 16; 1000000 x 4 43 and 66). (3000 x 2048 bf16 summed over 3000: one output per lane and
+  // f32: 512 chunks 37 us, 256 16; 1000000 x 4 43 and 66). A transcendental per element takes all the waves that there
+  // can be (the sines of 300 x 30000 beside their cosines: 67 us in one launch, 33). (3000 x 2048 bf16 summed over 3000: one output per lane and
   // chunks of 256 and more took 24 us in two launches, now 13; 1142 x 1110, one thread per output before, 160 us, now 9.)
-  const uint64_t want = flat && nred < (1ull << 18) ? 256 : 512;
-  uint64_t S = nred <= 512 ? 1 : std::min<uint64_t>({(want + tiles - 1) / tiles, nred / 32, 65535});
+  const bool light = !costly_inside(op.args[0]);
+  const uint64_t want = flat && light && nred < (1ull << 18) ? 256 : 512;
+  uint64_t S = light && nred <= 512 ? 1 : std::min<uint64_t>({(want + tiles - 1) / tiles, nred / 32, 65535});
   const uint64_t chunk = (nred + S - 1) / S, quarter = (chunk + parts - 1) / parts;
   S = (nred + chunk - 1) / chunk;
   const DType pd = partial_dtype(d, r);
@@ -369,6 +371,21 @@ bool Planner::row_leaves_16bit() const {
   return true;
 }
 
+bool Planner::costly(uint32_t v) const {
+  const Op& op = g_.ops[v];
+  if (op.kind == Kind::binary) return (Binary)op.code == Binary::div || (Binary)op.code == Binary::pow;
+  return op.kind == Kind::unary && (Unary)op.code != Unary::neg && (Unary)op.code != Unary::abs;
+}
+
+bool Planner::costly_inside(uint32_t v) const {
+  std::set<uint32_t> seen;
+  std::function<bool(uint32_t)> walk = [&](uint32_t x) {
+    if (!seen.insert(x).second || slots_.available(x) >= 0 || !is_inlinable(g_.ops[x].kind)) return false;
+    return costly(x) || std::any_of(g_.ops[x].args.begin(), g_.ops[x].args.end(), walk);
+  };
+  return walk(v);
+}
+
 // Values of the whole row that cost more than a register to evaluate again (a transcendental, a division) and
 // that a later pass reads too: the pass that computes them first leaves them in registers, as a row
 // read by several passes is. The outermost such value is taken first (what it was computed from is
@@ -377,11 +394,6 @@ bool Planner::row_leaves_16bit() const {
 // with one row to a CU, evaluated twice or kept, as its loads, arithmetic and stores then take turns;
 // 151 us kept, in pairs, with two rows to a CU.)
 void Planner::keep_row_values(const RowShape& rs, const RowKernel& rk, uint64_t per_thread, bool pairs) {
-  auto costly = [&](uint32_t v) {
-    const Op& op = g_.ops[v];
-    if (op.kind == Kind::binary) return (Binary)op.code == Binary::div || (Binary)op.code == Binary::pow;
-    return op.kind == Kind::unary && (Unary)op.code != Unary::neg && (Unary)op.code != Unary::abs;
-  };
   auto fits = [&]() {
     int last = 0;
     std::map<int, uint64_t> live;  // pass: registers holding values needed after it

@@ -466,6 +466,8 @@ def test_folds_choose_their_split_by_size():
         assert "parts[" not in plan(r, c) and plan(r, c).count("__global__") == 1 and "unroll" not in plan(r, c)
     for r, c in [(256, 512), (260, 5001), (512, 256)]:                           # one launch of workgroups
         assert "parts[4]" in plan(r, c) and plan(r, c).count("__global__") == 1
+    sines = hip.plan_source(T.define("fold", [T.spec("f32", r=300, c=30000)], lambda b, a: a[0].sin().sum("r")))
+    assert sines.count("__global__") == 2                                        # a transcendental per element: more waves
     for r, c, parts in [(100000, 64, 4), (1142, 1110, 4), (4000, 30001, 1), (1000, 9001, 1), (1000, 5001, 4)]:
         assert f"parts[{parts}]" in plan(r, c) and plan(r, c).count("__global__") == 2
     assert "s < (I)256" in plan(100000, 64)
