@@ -87,7 +87,7 @@ struct LowerOptions {
   bool allow_gemm = true;       // MFMA contraction kernels for f32 / f16 / bf16
   bool allow_attention = true;  // fused QK^T -> softmax -> V
   bool allow_row = true;        // fused row pipelines (else serial folds)
-  bool allow_split = true;      // contractions and single-query attention split over workgroups (partial sums in temporaries)
+  bool allow_split = true;      // contractions, single-query attention and folds split over workgroups (partial results in temporaries)
   // Launch candidate per kernel index (the order of the plan's kernel steps), for measuring; a
   // kernel not listed takes the table's selection for its key, else candidate 0.
   std::map<size_t, uint32_t> force_candidate;

@@ -619,7 +619,7 @@ uint64_t scratch_need(const Plan& plan) {
 Plan lower_expanded(const Graph& g, const LowerOptions& options) {
   Plan plan = planning::Planner(g, options).run();
   if (!options.allow_split || scratch_need(plan) <= kScratchBytes) return plan;
-  // The partial sums of splits must not be what keeps a program out of the scratch array.
+  // The partial results of splits must not be what keeps a program out of the scratch array.
   LowerOptions whole = options;
   whole.allow_split = false;
   Plan without = planning::Planner(g, whole).run();

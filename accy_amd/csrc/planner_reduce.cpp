@@ -151,7 +151,7 @@ void Planner::fold_chunked(uint32_t v, int out, const Type& in, const std::vecto
   // each wave a quarter of the workgroup's chunk, put together in order in LDS. Many outputs one by one take all 256
   // lanes of one chunk instead, so that a workgroup reads whole lines (4000 x 30001 bf16: 66 us, 49; 1000 x 5001 the other way round: 6.7, 8.7).
   const bool flat = kdims.size() == 1 && keep.back() + 1 == in.rank() && nout % 4 == 0;
-  const uint64_t parts = !flat && nout >= 8192 && nred > 512 ? 1 : 4, lanes = B / parts;
+  const uint64_t parts = !flat && nout >= 8192 && nred > 512 && opt_.allow_split ? 1 : 4, lanes = B / parts;
   const uint64_t VEC = flat ? 4 : 1, tiles = (nout + lanes * VEC - 1) / (lanes * VEC);
   // One launch up to 512 reduced elements (256 x 4096 f32: 4.0 us, 6.0 in two launches); else two workgroups for every CU, of
   // 32 reduced elements each at least, or one of vectors, since the chunks' partials are then folded one by one (100000 x 64
@@ -160,7 +160,7 @@ void Planner::fold_chunked(uint32_t v, int out, const Type& in, const std::vecto
   // chunks of 256 and more took 24 us in two launches, now 13; 1142 x 1110, one thread per output before, 160 us, now 9.)
   const bool light = !costly_inside(op.args[0]);
   const uint64_t want = flat && light && nred < (1ull << 18) ? 256 : 512;
-  uint64_t S = light && nred <= 512 ? 1 : std::min<uint64_t>({(want + tiles - 1) / tiles, nred / 32, 65535});
+  uint64_t S = !opt_.allow_split || (light && nred <= 512) ? 1 : std::min<uint64_t>({(want + tiles - 1) / tiles, nred / 32, 65535});
   const uint64_t chunk = (nred + S - 1) / S, quarter = (chunk + parts - 1) / parts;
   S = (nred + chunk - 1) / chunk;
   const DType pd = partial_dtype(d, r);

@@ -364,6 +364,17 @@ def test_partial_sums_do_not_keep_a_program_out_of_the_scratch_array():
     assert "split_sum" in hip.plan_source(prog(4096)) and "split_sum" not in hip.plan_source(prog(8352))
 
 
+def test_partial_folds_do_not_keep_a_program_out_of_the_scratch_array():
+    """A temporary of 511.9 MiB and a fold whose chunks' partials are 256 KiB: planned in one launch; with half the
+    rows, in chunks."""
+    def prog(rows):
+        def body(b, a):
+            e = a[0].sub(a[0].max("k")).exp()
+            return [e.div(e.sum("k")).contract(a[1], "k"), a[2].sum("r")]
+        return T.define("wide", [T.spec("bf16", m=rows, k=32000), T.spec("bf16", k=32000, n=64), T.spec("f32", r=3000, c=2048)], body)
+    assert "chunks grid" in hip.plan_source(prog(4096)) and "chunks grid" not in hip.plan_source(prog(8387))
+
+
 # extents of no multiple of 8, K below one step and below a vector, shallow aligned rows, splits, batches
 STAGED_SHAPES = [(1, 33, 1), (7, 65, 9), (130, 67, 131), (129, 1001, 255), (200, 64, 264), (33, 2049, 7), (1, 40, 1000),
                  (1100, 5, 1003), (16, 4097, 300), (3, 1030, 1887)]
