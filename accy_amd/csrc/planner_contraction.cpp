@@ -177,6 +177,15 @@ void Planner::pack_f32_operands(GemmShape& gs) {
   }
 }
 
+// Only the direct kernel needs another layout; the staged one reads every layout that has a unit stride. (us a pass, repacked /
+// as they are: A along M 2048^3 165 / 152, 1024^3 31 / 23; B along K 4000 x 1024 x 1024 86 / 78, 64 x 8192 x 2048 50 / 31.
+// With both along K and a split 128-wide tile the other way round: 2048 x 8192 x 1024 308 / 347, 3000 x 2048 x 2048 236 / 250.)
+bool Planner::f32_packs(const GemmShape& gs) const {
+  const Tile t = f32_tile(gs);
+  bool a_kc, b_kc;
+  return !t.bm || (t.bm == 128 && t.splits > 1 && staged_layout(gs, 4, a_kc, b_kc) && a_kc && b_kc);
+}
+
 bool Planner::f32_direct(const GemmShape& gs) {
   // 256 x 256 x 32 tiles, A K-contiguous and B N-contiguous with 16-byte aligned rows. Exact tiles, or
   // M / N off the tile grid (N a multiple of 4) when the problem is large (2^27 multiply-adds and more).
@@ -393,7 +402,7 @@ void Planner::dot(uint32_t v) {
   }
   GemmShape gs;
   if (gemm_eligible(op, gs)) {
-    if (op.result.dtype == DType::f32 && f32_direct(gs) && !f32_layout_ok(gs)) pack_f32_operands(gs);
+    if (op.result.dtype == DType::f32 && f32_direct(gs) && !f32_layout_ok(gs) && f32_packs(gs)) pack_f32_operands(gs);
     std::vector<std::pair<uint32_t, GemmShape>> group;
     if (gemm_siblings(v, gs, group)) {
       gemm_group(group);

@@ -453,7 +453,9 @@ class Planner {
   // written along c, so both sides touch whole lines; otherwise element by element along c.
   int pack_f32(int slot, int64_t off, int64_t batch, int64_t R, int64_t C, int64_t sb, int64_t sr, int64_t sc);
 
-  // Repacks the operands of a large f32 contraction whose layout the MFMA kernel does not take.
+  // Repacks the operands of a large f32 contraction whose layout the MFMA kernel does not take, or (f32_packs) takes
+  // more slowly.
+  bool f32_packs(const GemmShape& gs) const;
   void pack_f32_operands(GemmShape& gs);
 
   // The MFMA templates take operands whose K or M/N stride is 1.

@@ -590,11 +590,13 @@ def test_gemm_f32_on_mfma(m, k, n, spelling):
     assert_normwise(hip_run(prog, ins)[0], oracle_run(prog, ins)[0], 1e-3, "f32")
 
 
-@pytest.mark.parametrize("case", ["nt-1024x256x1024", "tn-520x512x516", "nt-batched-4x1024x64x1024"])
+@pytest.mark.parametrize("case", ["nt-1024x256x1024", "tn-520x512x516", "nt-batched-4x1024x64x1024", "nt-4096x64x4096",
+                                  "tn-3900x96x4092", "nt-batched-16x1024x64x1024"])
 def test_gemm_f32_other_layouts_repacked_onto_mfma(case):
-    """Large f32 contractions whose operand layout the f32 kernel does not take (A stored [k, m], B
-    stored [n, k]): the operand is copied into a contiguous temporary (a tiled transpose), then the
-    MFMA kernel runs; 1e-3 normwise, as for every f32 contraction on the matrix cores."""
+    """Large f32 contractions whose operand layout the 256-wide f32 kernel does not take (A stored [k, m],
+    B stored [n, k]): where that kernel fills the CUs the operand is copied into a contiguous temporary (a
+    tiled transpose) for it, else the staged kernel reads it as it is; 1e-3 normwise, as for every f32
+    contraction on the matrix cores."""
     say(f"gemm f32 repacked {case}")
     parts = case.split("-")
     if parts[0] == "nt" and parts[1] == "batched":
@@ -614,7 +616,8 @@ def test_gemm_f32_other_layouts_repacked_onto_mfma(case):
         prog = T.define(parts[0], specs, lambda b, a: a[0].contract(a[1], "k"))
         ins = [W.normal(43 + i, int(np.prod(sh))).astype(np.float32).reshape(sh) for i, sh in enumerate(shapes)]
     src = hip.plan_source(prog)
-    assert "accy::gemm::mma32f<" in src and "// pack:" in src
+    assert "accy::gemm::mma32f<" in src
+    assert ("// pack:" in src) == (case in ("nt-4096x64x4096", "tn-3900x96x4092", "nt-batched-16x1024x64x1024"))
     assert_normwise(hip_run(prog, ins)[0], oracle_run(prog, ins)[0], 1e-3, "f32")
 
 

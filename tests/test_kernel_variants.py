@@ -253,6 +253,9 @@ def test_f32_contractions_choose_their_kernel_by_size():
     assert "BM = 64" in plan(1000, 1000, 1000) and "SPLITS = 1" in plan(1000, 1000, 1000)
     assert "BM = 32" in plan(16, 4096, 4096) and "split_sum" in plan(16, 4096, 4096)
     assert "accy::gemm::" not in plan(200, 100, 200)
+    for layout in ("NT", "TN", "TT"):    # the staged kernel reads every layout, the direct one needs A along K and B along N
+        assert "pack" not in hip.plan_source(contraction("f32", 2048, 2048, 2048, layout))
+        assert "pack" in hip.plan_source(contraction("f32", 8192, 8192, 8192, layout))
     hip.plan_source(contraction("f32", 16, 4096, 4096, epilogue=True), compile=True)
 
 
