@@ -20,7 +20,6 @@ extern "C" __global__ void __launch_bounds__(256) accy_check_common(const float*
 struct CheckDmaNN : accy::gemm::Strided<0, 8192, 1, 0, 8192, 1> {
   static constexpr int DT = 0;
   static constexpr long M = 8192, N = 8192, K = 8192;
-  static constexpr long A_B = 0, A_M = 8192, A_K = 1, B_B = 0, B_K = 8192, B_N = 1;
   static constexpr bool A_KC = true, B_KC = false;
   static constexpr int BM = 256, BN = 256, STAGES = 4;
 };
@@ -35,7 +34,6 @@ struct CheckDmaNN2 : CheckDmaNN {
 struct CheckDmaTN : accy::gemm::Strided<0, 1, 384, 0, 1, 256> {
   static constexpr int DT = 1;
   static constexpr long M = 384, N = 128, K = 256;
-  static constexpr long A_B = 0, A_M = 1, A_K = 384, B_B = 0, B_K = 1, B_N = 256;
   static constexpr bool A_KC = false, B_KC = true;
   static constexpr int BM = 128, BN = 128, STAGES = 4;
 };
@@ -54,7 +52,6 @@ extern "C" __global__ void __launch_bounds__(256) accy_check_gemm_dma_tn(const u
 
 struct CheckF32NN : accy::gemm::Strided<0, 8192, 1, 0, 8192, 1> {
   static constexpr long M = 8192, N = 8192, K = 8192;
-  static constexpr long A_B = 0, A_M = 8192, B_B = 0, B_K = 8192;
 };
 
 struct CheckEpiF32 {

@@ -474,23 +474,10 @@ void Planner::gemm_group(const std::vector<std::pair<uint32_t, GemmShape>>& grou
     cases << "      case " << i << ": return " << w.arg(out, true) << ";\n";
     if (i) label += "&%" + std::to_string(u);
   }
-  std::ostringstream members, inits;
-  {
-    std::string pl = w.params();
-    size_t start = 0;
-    while (start < pl.size()) {
-      size_t comma = pl.find(", ", start);
-      std::string decl = pl.substr(start, comma == std::string::npos ? std::string::npos : comma - start);
-      members << "  " << decl << ";\n";
-      size_t sp = decl.rfind(' ');
-      inits << (inits.tellp() > 0 ? ", " : "") << decl.substr(sp + 1);
-      if (comma == std::string::npos) break;
-      start = comma + 2;
-    }
-  }
+  const KernelWriter::Members members = w.members();
   std::ostringstream src;
   src << "#include \"gemm\"\n";
-  src << "struct Epi_" << nm << " {\n" << members.str()
+  src << "struct Epi_" << nm << " {\n" << members.decls
       << "  __device__ __forceinline__ u16_t* out(int g) const {\n"
       << "    switch (g) {\n" << cases.str() << "      default: return nullptr;\n    }\n  }\n"
       << "  __device__ __forceinline__ void operator()(u16_t* __restrict__ o, long b, long m, long n, float v) const {\n"
@@ -498,8 +485,6 @@ void Planner::gemm_group(const std::vector<std::pair<uint32_t, GemmShape>>& grou
   src << "struct Cfg_" << nm << " {\n"
       << "  static constexpr int DT = " << (d == DType::bf16 ? 0 : 1) << ";\n"
       << "  static constexpr long M = " << gs.m << ", N = " << gs.n << ", K = " << gs.k << ";\n"
-      << "  static constexpr long A_B = " << gs.a_b << ", A_M = " << gs.a_m << ", A_K = " << gs.a_k << ";\n"
-      << "  static constexpr long B_B = " << gs.b_b << ", B_K = " << gs.b_k << ", B_N = " << gs.b_n << ";\n"
       << "  static constexpr bool A_KC = " << (gs.a_k == 1 ? "true" : "false")
       << ", B_KC = " << (gs.b_k == 1 ? "true" : "false") << ";\n"
       << gs.ga_b.fn("a_b") << gs.ga_m.fn("a_m") << gs.ga_k.fn("a_k") << gs.gb_b.fn("b_b") << gs.gb_k.fn("b_k")
@@ -508,7 +493,7 @@ void Planner::gemm_group(const std::vector<std::pair<uint32_t, GemmShape>>& grou
       << "  const u16_t* const bs[" << G << "] = {";
   for (size_t i = 0; i < G; ++i) src << (i ? ", " : "") << bs[i];
   src << "};\n  accy::gemm::mma16_dma_group<Cfg_" << nm << ", " << G << ">(" << a << " + " << gs.a.offset
-      << "L, bs, Epi_" << nm << "{" << inits.str() << "});\n}\n";
+      << "L, bs, Epi_" << nm << "{" << members.inits << "});\n}\n";
   KernelStep k;
   k.source = src.str();
   k.name = nm;
@@ -758,8 +743,6 @@ void Planner::gemm(uint32_t v, const GemmShape& gs, const OutStrides& os) {
     src << "struct Cfg_" << nm << " {\n"
         << "  static constexpr int DT = " << (d == DType::bf16 ? 0 : 1) << ";\n"
         << "  static constexpr long BATCH = " << gs.batch << ", M = " << gs.m << ", N = " << gs.n << ", K = " << gs.k << ";\n"
-        << "  static constexpr long A_B = " << gs.a_b << ", A_M = " << gs.a_m << ", A_K = " << gs.a_k << ";\n"
-        << "  static constexpr long B_B = " << gs.b_b << ", B_K = " << gs.b_k << ", B_N = " << gs.b_n << ";\n"
         << "  static constexpr bool A_KC = " << (akc ? "true" : "false") << ", B_KC = " << (bkc ? "true" : "false")
         << ";\n"
         << gs.ga_b.fn("a_b") << gs.ga_m.fn("a_m") << gs.ga_k.fn("a_k") << gs.gb_b.fn("b_b") << gs.gb_k.fn("b_k")
