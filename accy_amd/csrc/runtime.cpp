@@ -71,6 +71,25 @@ std::string full_kernel_source(const std::string& body) {
   return out + rest;
 }
 
+namespace {
+
+// Whether the process's hiprtc knows -amdgpu-mfma-vgpr-form. A process that loaded another ROCm's libraries first
+// (PyTorch's wheel brings its own) compiles with those, and LLVM ends the process at an option that it does
+// not know: so the compiler's version is asked first, by compiling a line that only newer ones accept.
+bool has_mfma_vgpr_form() {
+  static const bool known = [] {
+    hiprtcProgram prog;
+    if (hiprtcCreateProgram(&prog, "#if __clang_major__ < 22\n#error\n#endif\n", "version.hip", 0, nullptr, nullptr) != HIPRTC_SUCCESS) return false;
+    const char* arch = "--offload-arch=gfx950";
+    const bool ok = hiprtcCompileProgram(prog, 1, &arch) == HIPRTC_SUCCESS;
+    hiprtcDestroyProgram(&prog);
+    return ok;
+  }();
+  return known;
+}
+
+}  // namespace
+
 std::vector<char> compile_kernel_source(const std::string& source, const std::string& name) {
   hiprtcProgram prog;
   if (hiprtcCreateProgram(&prog, source.c_str(), (name + ".hip").c_str(), 0, nullptr, nullptr) != HIPRTC_SUCCESS)
@@ -84,7 +103,7 @@ std::vector<char> compile_kernel_source(const std::string& source, const std::st
   // the array moves to scratch memory).
   std::vector<const char*> opts = {"--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature",
                                    "-Xclang", "-packed-fp32-ops", "-mllvm", "-pragma-unroll-threshold=65536"};
-  if (source.find(kMfmaVgprForm) != std::string::npos) {
+  if (source.find(kMfmaVgprForm) != std::string::npos && has_mfma_vgpr_form()) {
     opts.push_back("-mllvm");
     opts.push_back("-amdgpu-mfma-vgpr-form");
   }

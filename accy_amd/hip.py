@@ -10,7 +10,8 @@ Mirrors the reference's execution API for the runCpu path:
 ``program`` is a recorded ``accy_amd.tensor.Program`` or its ACTP v1 wire bytes. Inputs are
 bytes-like objects or numpy arrays (their raw bytes are used); outputs are writable buffers
 (numpy arrays or bytearrays), each exactly its slot's size. ``launch_device`` takes device pointers
-(e.g. ``torch.Tensor.data_ptr()``) and a HIP stream handle, for data already resident in HBM.
+and a HIP stream handle, for data already resident in HBM (from ``DeviceBuffer``, or
+``torch.Tensor.data_ptr()`` in a process that imported torch before loading this library).
 
 The library is built in-tree by ``accy_amd.build``; loading fails loudly if it is missing — there is
 no CPU fallback in the product.

@@ -1,6 +1,9 @@
 """Kernel variants that the planner chooses by size, layout or neighbouring operations, each at the sizes
 where it can go wrong: compared with the CPU oracle, or with the float64 formula where stated."""
 import re
+import subprocess
+import sys
+from pathlib import Path
 
 import numpy as np
 import pytest
@@ -634,3 +637,43 @@ def test_mlp_block_of_odd_sizes(tokens, model, ffn):
     exact = x + 0.5 * h * (1 + np.tanh(0.7978845608028654 * (h + 0.044715 * h ** 3))) @ w2
     got, ref = (to_f32(r[0], "bf16").astype(np.float64) for r in (hip_run(prog, ins), oracle_run(prog, ins)))
     assert np.abs(got - exact).max() <= 1.5 * np.abs(ref - exact).max() + 2.0 ** -7 * np.abs(exact).max()
+
+
+# ---- a process that loaded PyTorch, whose wheel brings another ROCm's compiler, before the library ----
+
+AFTER_TORCH = """
+import sys
+import torch
+import numpy as np
+sys.path[:0] = [{root!r}, {tests!r}]
+from accy_amd import hip, workloads as W
+from conftest import exact_attention, hip_run, to_f32
+for dtype, dim, seq, causal in [("f16", 64, 96, True), ("bf16", 128, 128, True), ("f16", 128, 192, False)]:
+    print(dtype, dim, seq, causal, flush=True)
+    prog = W.attention_program(2, seq, dim, dtype, causal)
+    assert "accy::attn::flash<" in hip.plan_source(prog, compile=True)
+    if {run}:
+        ins = W.attention_inputs(2, seq, dim, dtype, seed=dim)
+        exact = exact_attention(*ins, 1.0 / np.sqrt(dim), causal, dtype)
+        got = to_f32(hip_run(prog, ins)[0], dtype)
+        assert np.linalg.norm(got - exact) <= 1e-2 * np.linalg.norm(exact)
+print("all ran")
+"""
+
+
+def after_torch(run):
+    tests = Path(__file__).resolve().parent
+    done = subprocess.run([sys.executable, "-c", AFTER_TORCH.format(root=str(tests.parent), tests=str(tests), run=run)],
+                          capture_output=True, text=True, timeout=110)
+    assert done.returncode == 0 and "all ran" in done.stdout, done.stdout + done.stderr
+
+
+def test_16bit_attention_compiles_in_a_process_that_loaded_torch():
+    """That compiler ends the process at an option it does not know."""
+    after_torch(False)
+
+
+@pytest.mark.gpu
+def test_16bit_attention_runs_in_a_process_that_loaded_torch():
+    """1e-2 normwise of float64, the bound of 16-bit attention everywhere."""
+    after_torch(True)
