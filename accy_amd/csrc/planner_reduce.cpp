@@ -464,7 +464,9 @@ KernelStep Planner::gen_row(const RowShape& rs, const RowKernel& rk, bool commit
   size_t passes = (size_t)reduce_passes + (rk.full_vals.empty() ? 0 : 1);
   // No more rows than CUs: as many threads per row as have a vector each, up to 1024, so that a CU has more than two
   // waves. (us a pass, 128 threads / now: logsumexp 1 x 100000 f32 61 / 14, tone 200 x 16384 19.2 / 7.7, 1 x 8395 10.1 /
-  // 7.7; rows that 128 threads keep in registers stay at a launch's 7.3.)
+  // 7.7; rows that 128 threads keep in registers stay at a launch's 7.3.) The line is where rows outnumber the CUs, not
+  // where it pays: 512 threads are faster for up to about 1000 long rows as well (128 / 512: tone 300 x 16384 19.2 / 8.0,
+  // 1000 x 16384 18.2 / 14.4, logsumexp 500 x 8192 5.8 / 4.1, but 2000 x 4096 6.5 / 7.0).
   if (kn <= 256)
     for (uint32_t wide : {1024u, 512u, 256u})
       if (lanes >= wide) {

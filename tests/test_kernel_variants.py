@@ -420,6 +420,27 @@ def test_contraction_tail_ignores_what_lies_past_k(m, k, n, layout):
     assert np.array_equal(got[1:-1, 1:-1], clean[1:-1, 1:-1])
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,m,k,n,layout", [("bf16", 136, 1001, 264, "TN"), ("f16", 300, 1000, 264, "NN"), ("bf16", 300, 1000, 135, "NT"),
+                                                ("bf16", 131, 1005, 137, "NN"), ("f16", 131, 1005, 137, "TT"), ("bf16", 9, 70, 11, "NT"),
+                                                ("f32", 130, 1030, 66, "NN"), ("f32", 33, 1130, 65, "TT"), ("f32", 130, 1030, 66, "NT")])
+def test_contraction_tail_repeats_nothing_that_is_infinite(dtype, m, k, n, layout):
+    """The last element of K, which loads past the end repeat, is infinite in one row of A and one column of B;
+    everything is positive, so those outputs are infinite (0 x inf, from an operand that is not cleared past K, would be
+    NaN) and the rest as without."""
+    prog = contraction(dtype, m, k, n, layout)
+    ins, _, _, _ = contraction_inputs(dtype, m, k, n, layout, 0, False, 4)
+    ins = [x & 0x7fff if dtype == "bf16" else np.abs(x) for x in ins]
+    clean = to_f32(hip_run(prog, ins)[0], dtype)
+    inf = 0x7f80 if dtype == "bf16" else np.inf
+    (ins[0] if layout[0] == "N" else ins[0].T)[2, -1] = inf
+    (ins[1] if layout[1] == "N" else ins[1].T)[-1, 3] = inf
+    got = to_f32(hip_run(prog, ins)[0], dtype)
+    hit = np.zeros((m, n), bool)
+    hit[2], hit[:, 3] = True, True
+    assert np.all(got[hit] == np.inf) and np.array_equal(got[~hit], clean[~hit])
+
+
 def test_contractions_choose_their_tile_by_size():
     plan = lambda m, k, n, layout="NN": hip.plan_source(contraction("bf16", m, k, n, layout))
     assert "BM = 256, BN = 256" in plan(8192, 8192, 8192) and "SPLITS" not in plan(8192, 8192, 8192)

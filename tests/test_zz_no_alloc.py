@@ -93,9 +93,9 @@ def test_scratch_entry_point_matches_invoke_device(big, small):
 
 
 def test_scratch_entry_point_refuses_programs_beyond_the_scratch():
-    # an f32 contraction with A stored [k, m] repacks A into a temporary of m * k * 4 bytes = 576 MiB
+    # a large f32 contraction with A stored [k, m] repacks A into a temporary of m * k * 4 bytes = 576 MiB
     n = 12288
-    prog = T.define("tn", [T.spec("f32", k=n, m=n), T.spec("f32", k=n, n=256)], lambda b, a: a[0].contract(a[1], "k"))
+    prog = T.define("tn", [T.spec("f32", k=n, m=n), T.spec("f32", k=n, n=n)], lambda b, a: a[0].contract(a[1], "k"))
     assert "pack" in hip.plan_source(prog)
     s = hip.Session()
     h = s.compile(prog)
