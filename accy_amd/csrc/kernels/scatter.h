@@ -65,12 +65,12 @@ __device__ __forceinline__ void rows(const S& s) {
   __shared__ int wave_count[BLOCK / 64];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int group = tid / TC % KG;
+  const int group = PG > 1 ? tid / TC % KG : tid / TC;
   for (long tile = blockIdx.x; tile < TILES; tile += gridDim.x) {
     const I mine = (I)(tile % ROW_TILES);
     // local row (block i, group g) <-> row of the table
     auto row_at = [&](int i, int g) { return ((I)i * (I)ROW_TILES + mine) * KG + g; };
-    const I p0 = (I)(tile / ROW_TILES / COL_TILES) * (PG * S::PLOOP) + tid / TC / KG;
+    const I p0 = (I)(tile / ROW_TILES / COL_TILES) * (PG * S::PLOOP) + (PG > 1 ? tid / TC / KG : 0);
     const I c0 = ((I)(tile / ROW_TILES % COL_TILES) * TC + (I)(tid % TC)) * VEC;
     const bool in_row = c0 < (I)S::POST;
     // the last workgroup's positions may reach past the end
@@ -155,8 +155,7 @@ __device__ __forceinline__ void rows(const S& s) {
         }
         __syncthreads();
       }
-      for (int pl = 0; pl < S::PLOOP; ++pl) {
-        const I p = p0 + pl * PG;
+      auto add = [&](I p, bool loaded) {
         for (int t = 0; t < LOOP; ++t) {
 #pragma unroll
           for (int i = 0; i < RR; ++i) {
@@ -168,7 +167,7 @@ __device__ __forceinline__ void rows(const S& s) {
             if (begun) {
               if (x == e) continue;
               s.again(p, k, c0, v[i]);
-            } else if (t > 0 || pl > 0) {
+            } else if (t > 0 || !loaded) {
               s.init(p, k, c0, v[i]);
             }
             for (; e - x > 4; x += DEPTH) add_run<DEPTH>(s, sorted, x, e, p, c0, v[i]);
@@ -176,7 +175,10 @@ __device__ __forceinline__ void rows(const S& s) {
             s.store(p, k, c0, v[i]);
           }
         }
-      }
+      };
+      add(p0, true);
+#pragma unroll 1
+      for (int pl = 1; pl < S::PLOOP; ++pl) add(p0 + pl * PG, false);
       begun = true;
       __syncthreads();  // the lists are rewritten by the next batch
     } while (next < (I)S::NI);

@@ -460,8 +460,8 @@ void Planner::scatter_add(uint32_t v) {
     store = "    " + w.store(out, at, d, "v[0]") + "\n";
   }
   // Threads along a row: enough for its vectors, more (idle while adding) where the rows are too few for
-  // a workgroup on every CU. Each workgroup reads the whole index list, so it owns more rows, then more leading
-  // positions, when tiles x updates passes 2^25 reads, while 1024 tiles remain (8192 updates of 100000 x 1024 f32: 209 us, 292 with
+  // a workgroup on every CU. Each workgroup reads the whole index list, so it owns more rows when
+  // tiles x updates passes 2^25 reads, while 1024 tiles remain (8192 updates of 100000 x 1024 f32: 209 us, 292 with
   // one tile of four rows for every workgroup; a limit of 2^24: 232).
   const uint64_t vecs = post / vec;
   uint64_t tc = 1, kg = 1, loop = 1, ploop = 1;
@@ -481,19 +481,18 @@ void Planner::scatter_add(uint32_t v) {
   const uint64_t rows = kg * 4, pg = 256 / tc / kg;
   auto reads = [&]() { return tiles(loop * rows, ploop * pg) > (1ull << 25) / ni; };
   while (2 * loop * rows <= 4096 && loop * rows < (uint64_t)ext && tiles(2 * loop * rows, pg) >= 1024 && reads()) loop *= 2;
-  // Positions in turn, also where sorting a tile's hits takes longer than its rows (16384 x 1000 f32 with 512 updates
+  // Positions in turn where sorting a tile's hits takes longer than its rows (16384 x 1000 f32 with 512 updates
   // 471 us, now 104; 16384 x 8 x 256 with 64 the other way round: 247 / 272) or a workgroup has few elements.
   const uint64_t own = std::min<uint64_t>((uint64_t)ext, loop * rows), width = std::min(post, tc * vec);
   const double hits = (double)ni * (double)own / (double)ext;
   const bool sorts = hits * hits >= 4.0 * (double)(own * width);
   while (ploop < 1024 && ploop * pg < pre && tiles(loop * rows, 2 * ploop * pg) >= 1024 &&
-         (reads() || sorts || own * width * pg * ploop < 1024))
+         (sorts || own * width * pg * ploop < 1024))
     ploop *= 2;
   std::string nm = name("scatter", v);
   const KernelWriter::Members members = w.members();
   std::ostringstream src;
-  // Four waves per SIMD, so that 128 registers hold the updates in flight. (Left to itself the compiler takes 62
-  // for some shapes and waits: 100 x 3 f32 with 1000 updates 17.4 us, 12.6.)
+  // Four waves per SIMD at least (8 x 50000 x 64 f32: 129 registers, 112 us; 128 and 96).
   src << "#include \"scatter\"\n"
       << "struct Tab_" << nm << " {\n" << members.decls << "  typedef " << w.itype << " I;\n  typedef " << compute_type(d) << " T;\n"
       << "  static constexpr long NI = " << ni << ", EXT = " << ext << ", POST = " << post << ", PRE = " << pre << ";\n"
@@ -503,7 +502,7 @@ void Planner::scatter_add(uint32_t v) {
       << "  static __device__ __forceinline__ T plus(T a, T u) { return " << plus << "; }\n" << init << update
       << "  __device__ __forceinline__ void again(I p, I k, I c0, T (&v)[VEC]) const {\n" << again << "  }\n"
       << "  __device__ __forceinline__ void store(I p, I k, I c0, const T (&v)[VEC]) const {\n" << store << "  }\n};\n"
-      << "extern \"C\" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) " << nm << "(" << w.params() << ") {\n"
+      << "extern \"C\" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) " << nm << "(" << w.params() << ") {\n"
       << "  accy::scatter::rows(Tab_" << nm << "{" << members.inits << "});\n}\n";
   KernelStep k;
   k.source = src.str();
