@@ -434,11 +434,20 @@ void Planner::keep_row_values(const RowShape& rs, const RowKernel& rk, uint64_t 
 
 KernelStep Planner::gen_row(const RowShape& rs, const RowKernel& rk, bool commit) {
   uint64_t tn = prod(rs.T, 0, rs.T.size()), kn = prod(rs.K, 0, rs.K.size());
+  // Reductions that need no other's result share one pass over the row: pass_of[j] is one more than the
+  // latest pass whose result reduction j reads. (A pass for each made every one of them load, or keep
+  // in registers, the same row and evaluate the same elementwise values again: the mismatch and its
+  // slope over 8192 x 16384 took 694 us in two passes of a cached, fully unrolled row, 82 us in one.)
+  const std::vector<int> pass_of = reduction_passes(rk);
+  const int reduce_passes = 1 + *std::max_element(pass_of.begin(), pass_of.end());
+  const size_t passes = (size_t)reduce_passes + (rk.full_vals.empty() ? 0 : 1);
   // Four consecutive elements per thread, also of rows whose length is no multiple of four (their vectors
   // begin at any element). Shorter ones than one vector per lane of a wave keep one element per thread
-  // (30000 rows of 67 f16: 7.4 us against 9.0 with 17 of 64 lanes at work), rows of several axes too.
-  const bool flat = rs.T.size() == 1;
-  const uint32_t VEC = tn % 4 == 0 || (flat && tn >= 256) ? 4 : 1;
+  // (30000 rows of 67 f16: 7.4 us against 9.0 with 17 of 64 lanes at work), rows of several axes too, and of several
+  // passes those whose second iteration is mostly a partial one (layernorm of 100000 rows of 510 f32: 92 us in vectors,
+  // 75; of 300: 48, 53; of 514: 75, 167).
+  const bool flat = rs.T.size() == 1, partly = passes >= 2 && tn > 320 && tn < 512;
+  const uint32_t VEC = tn % 4 == 0 || (flat && tn >= 256 && !partly) ? 4 : 1;
   uint64_t lanes = (tn + VEC - 1) / VEC;
   // Two waves per row: against one workgroup of four waves per row, C2's logsumexp went from 163-165 to
   // 159-161 µs and C1's tone from 58 to 56 µs on one box (four rounds), 162.0 -> 159.0 and 53.4 ->
@@ -447,12 +456,6 @@ KernelStep Planner::gen_row(const RowShape& rs, const RowKernel& rk, bool commit
   // meeting two waves at its barriers instead of four.
   uint32_t B = lanes >= 128 ? 128 : (uint32_t)std::max<uint64_t>(64, (lanes + 63) / 64 * 64);
   uint64_t E = (tn + (uint64_t)B * VEC - 1) / ((uint64_t)B * VEC);
-  // Reductions that need no other's result share one pass over the row: pass_of[j] is one more than the
-  // latest pass whose result reduction j reads. (A pass for each made every one of them load, or keep
-  // in registers, the same row and evaluate the same elementwise values again: the mismatch and its
-  // slope over 8192 x 16384 took 694 us in two passes of a cached, fully unrolled row, 82 us in one.)
-  const std::vector<int> pass_of = reduction_passes(rk);
-  const int reduce_passes = 1 + *std::max_element(pass_of.begin(), pass_of.end());
   if (commit) {
     row_keep_.clear();
     gen_row(rs, rk, false);  // what the passes read
@@ -463,7 +466,6 @@ KernelStep Planner::gen_row(const RowShape& rs, const RowKernel& rk, bool commit
   // where a row has no shorter share.
   const bool pairs_ok = commit && VEC == 4 && flat && row_leaves_16bit();
   auto keepable = [&](uint32_t threads) -> uint64_t { return !pairs_ok ? 64 : threads == 1024 ? 128 : 104; };
-  size_t passes = (size_t)reduce_passes + (rk.full_vals.empty() ? 0 : 1);
   // No more rows than CUs: as many threads per row as have a vector each, up to 1024, so that a CU has more than two
   // waves. (us a pass, 128 threads / now: logsumexp 1 x 100000 f32 61 / 14, tone 200 x 16384 19.2 / 7.7, 1 x 8395 10.1 /
   // 7.7; rows that 128 threads keep in registers stay at a launch's 7.3.) The line is where rows outnumber the CUs, not

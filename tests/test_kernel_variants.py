@@ -299,6 +299,14 @@ def test_ragged_rows_match_the_oracle(rows, cols, dtype):
         assert np.all(np.abs(g - r) <= tol * np.abs(r))
 
 
+def test_ragged_rows_choose_vectors_by_length():
+    rows = lambda cols, body: hip.plan_source(T.define("rows", [T.spec("f32", r=5000, c=cols)], body))
+    softmax = lambda b, a: a[0].sub(a[0].max("c")).exp().sum("c")
+    for cols, vectors in [(255, False), (257, True), (321, False), (385, False), (511, False), (514, True)]:
+        assert ("const I cr =" in rows(cols, softmax)) == vectors
+    assert "const I cr =" in rows(385, lambda b, a: a[0].sum("c"))     # one pass
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows,cols,threads", [(1, 100003, 1024), (3, 80000, 1024), (256, 2050, 512), (9, 1030, 256), (257, 2050, 128)])
 def test_few_rows_take_more_threads(rows, cols, threads):
