@@ -6,20 +6,20 @@
 // What bounds it is the table's copy (read and write of every row) and the updates read once; the
 // rows that many updates hit (a frequent token) are the serial part, so their updates are loaded
 // eight to 32 at a time (32 registers' worth) ahead of the dependent additions. One thread per (p, q) walking all j, as before,
-// took 989 us for 4096 updates of a 32000 x 1024 f32 table after a 43 us copy: one dependent load, add
-// and store per update and only 1024 threads in flight.
+// took 1004 us a pass for 4096 updates of a 32000 x 1024 f32 table, the 43 us copy of the table among them (1390 as
+// PyTorch's wheel compiles it): one dependent load, add and store per update and only 1024 threads in flight.
 //
 // A workgroup owns ROWS = LOOP x 4 x KG rows of PG x PLOOP positions of p and one tile of q: LOOP x 4 blocks of KG
 // consecutive rows, ROW_TILES blocks apart, so that the frequent tokens, whose ids are small in most
 // vocabularies, fall to different workgroups (four consecutive rows per workgroup took 194 us
-// instead of 87 us for the table above, now 66-77, with ids whose frequency falls as 1 / rank). It
+// instead of 87 us for the table above, now 66-78, with ids whose frequency falls as 1 / rank). It
 // reads the whole index list (from L2) and keeps the entries of its rows: (row, j) pairs in LDS, in
 // the order of j (ballot ranks). A batch of up to CAP of them is sorted stably by row (the rank of every key among
 // the batch: keys are row * CAP + position, all distinct), and each group of TC threads (along a row) then adds
 // the runs of its four rows. The lists are the same for every p: where KG groups cover the rows of one, the workgroup's
 // other groups take the next PG - 1 positions, and all of them PLOOP positions in turn. (1048576 x 8 f32 with
-// 64 updates along the last axis: 5886 us with a workgroup for every p, now 150; 300 with a thread for every p.) When more entries remain, the next batch continues from the rows just written
-// (the same thread wrote them).
+// 64 updates along the last axis: 5886 us with a workgroup for every p, now 150; 300 with a thread for every p.)
+// When more entries remain, the next batch continues from the rows just written (the same thread wrote them).
 //
 // S supplies the sizes (NI updates, EXT rows, POST elements per row, PRE), TC, KG, LOOP, PLOOP, VEC (4 when POST
 // is a multiple of it), index(j), plus(a, u), and on the VEC elements c0 .. c0 + VEC - 1 of a row

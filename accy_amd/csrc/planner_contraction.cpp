@@ -307,16 +307,20 @@ Planner::Tile Planner::staged16_tile(const GemmShape& gs) const {
 // 16-bit rows in whole vectors along k or not), the operands from memory. Measured (us a pass, tiles / folded):
 // f32 65535 x (4 x 128 x 4) 397 / 48, 4194304 x 4 x 4 329 / 30, 1048576 x 16 x 8 87 / 32, 2 x 130 x 3 6.0 / 3.8, but
 // 20000 x 130 x 9 7.8 / 15.8, 10000 x (20 x 130 x 20) 100 / 129; bf16 65535 x (4 x 128 x 4) 348 / 36, 3000000 x 3 x 3
-// 98 / 16, but 1000 x (50 x 130 x 50) 16 / 115. A single round of the 16-bit kernel is as fast as a launch of the fold.
+// 98 / 16, 300000 x 300 x 3 131 / 92, but 1000 x (50 x 130 x 50) 16 / 115. A single round of the 16-bit kernel is as fast as a launch of the fold.
 bool Planner::fold_wins(const GemmShape& gs, const Tile& t, bool f32) {
   const int64_t tiles = (gs.m + 127) / 128 * ((gs.n + 127) / 128) * gs.batch;
   if (!f32 && tiles <= 512) return false;
   const bool along_n = gs.gb_n.inner_str() == 1 && gs.gb_n.inner_ext() % 4 == 0, along_k = gs.k % 4 == 0;
-  const double rate = f32 ? (along_n ? 1300 : 700) : along_n ? (along_k ? 2200 : 1200) : (along_k ? 1800 : 1000);
+  const bool short_k = gs.gb_k.inner_str() == 1 && gs.k <= 32;  // B's rows share lines
+  const double rate = f32 ? (along_n ? 1300 : short_k ? 1000 : 700) : along_n ? (along_k ? 2200 : 1200) : (along_k ? 1800 : 1000);
   const double step = gs.batch > 1 && gs.m == 1 && gs.n == 1 ? 350 : f32 ? 55 : 80;
   const double bytes = (double)gs.batch * (double)gs.k * (double)(gs.m + gs.n) * (f32 ? 4 : 2);
+  // 16-bit operands read along fewer than eight rows or columns are loaded element by element
+  bool a_kc, b_kc;
+  const bool slow = !f32 && staged_layout(gs, 8, a_kc, b_kc) && ((!a_kc && gs.m < 8) || (!b_kc && gs.n < 8));
   const double rest = !f32 ? 1000 : gs.k % 64 ? 500 : -1500;  // a launch against the other's, the last K step's edges
-  return std::max({step * (double)gs.k, macs(gs) / rate, bytes / 1400}) < t.cost + rest;
+  return std::max({step * (double)gs.k, macs(gs) / rate, bytes / 1400}) < (slow ? 3.5 : 1.0) * t.cost + rest;
 }
 
 bool Planner::gemm_eligible(const Op& op, GemmShape& gs) const {
