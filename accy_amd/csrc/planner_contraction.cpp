@@ -308,9 +308,9 @@ Planner::Tile Planner::staged16_tile(const GemmShape& gs) const {
 // f32 65535 x (4 x 128 x 4) 397 / 48, 4194304 x 4 x 4 329 / 30, 1048576 x 16 x 8 87 / 32, 2 x 130 x 3 6.0 / 3.8, but
 // 20000 x 130 x 9 7.8 / 15.8, 10000 x (20 x 130 x 20) 100 / 129; bf16 65535 x (4 x 128 x 4) 348 / 36, 3000000 x 3 x 3
 // 98 / 16, 300000 x 300 x 3 131 / 92, but 1000 x (50 x 130 x 50) 16 / 115. A single round of the 16-bit kernel is as fast as a launch of the fold.
-bool Planner::fold_wins(const GemmShape& gs, const Tile& t, bool f32) {
+bool Planner::fold_wins(const GemmShape& gs, const Tile& t, bool f32, bool rows) {
   const int64_t tiles = (gs.m + 127) / 128 * ((gs.n + 127) / 128) * gs.batch;
-  if (!f32 && tiles <= 512) return false;
+  if (!f32 && !rows && tiles <= 512) return false;
   const bool along_n = gs.gb_n.inner_str() == 1 && gs.gb_n.inner_ext() % 4 == 0, along_k = gs.k % 4 == 0;
   const bool short_k = gs.gb_k.inner_str() == 1 && gs.k <= 32;  // B's rows share lines
   const double rate = f32 ? (along_n ? 1300 : short_k ? 1000 : 700) : along_n ? (along_k ? 2200 : 1200) : (along_k ? 1800 : 1000);
@@ -320,10 +320,12 @@ bool Planner::fold_wins(const GemmShape& gs, const Tile& t, bool f32) {
   bool a_kc, b_kc;
   const bool slow = !f32 && staged_layout(gs, 8, a_kc, b_kc) && ((!a_kc && gs.m < 8) || (!b_kc && gs.n < 8));
   const double rest = !f32 ? 1000 : gs.k % 64 ? 500 : -1500;  // a launch against the other's, the last K step's edges
+  // Row kernels (us a pass, tiles / rows: f32 127 x 131 x 129 6.8 / 3.7, 64 x 2000 x 64 10.1 / 6.4, 300^3 9.7 / 20).
+  if (rows) return macs(gs) / 560 < t.cost + rest;
   return std::max({step * (double)gs.k, macs(gs) / rate, bytes / 1400}) < (slow ? 3.5 : 1.0) * t.cost + rest;
 }
 
-bool Planner::gemm_eligible(const Op& op, GemmShape& gs) const {
+bool Planner::gemm_eligible(const Op& op, GemmShape& gs, bool rows) const {
   if (!opt_.allow_gemm) return false;
   DType d = op.result.dtype;
   if (d != DType::bf16 && d != DType::f16 && d != DType::f32) return false;
@@ -337,7 +339,7 @@ bool Planner::gemm_eligible(const Op& op, GemmShape& gs) const {
     if (f32_direct(gs)) return true;
     if ((gs.k < 128 && macs(gs) < (double)(1ull << 23)) || !staged_layout(gs, 4, akc, bkc)) return false;
     const Tile t = f32_tile(gs);
-    return t.bm && !fold_wins(gs, t, true);
+    return t.bm && !fold_wins(gs, t, true, rows);
   }
   int dm, dn;
   bool akc, bkc;
@@ -349,7 +351,7 @@ bool Planner::gemm_eligible(const Op& op, GemmShape& gs) const {
   if (!t.bm) return false;
   auto ok8 = [](int64_t x) { return x % 8 == 0; };
   const bool aligned = ok8(akc ? gs.k : gs.m) && ok8(bkc ? gs.k : gs.n);
-  return aligned || ((gs.k >= 32 || macs(gs) >= (double)(1ull << 20)) && !fold_wins(gs, t, false));
+  return aligned || ((gs.k >= 32 || macs(gs) >= (double)(1ull << 20)) && !fold_wins(gs, t, false, rows));
 }
 
 void Planner::mark_gemm_operands() {
@@ -898,7 +900,8 @@ bool Planner::mulsum(uint32_t v) {
     for (const Dim& x : *g) dot.result.dims.push_back(x);
   if (dot.lhs_contract.empty()) return false;
   GemmShape gs;
-  if (!gemm_eligible(dot, gs)) return false;
+  RowShape rows;
+  if (!gemm_eligible(dot, gs, row_shape(v, rows) && prod(rows.T, 0, rows.T.size()) >= 64)) return false;
   // Matrix cores only pay when both output extents fill a tile; x * x summed over an axis (a
   // norm) stays a row reduction.
   if (gs.m < 32 || gs.n < 32) return false;

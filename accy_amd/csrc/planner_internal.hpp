@@ -424,8 +424,9 @@ class Planner {
     double cost = 0;  // clocks, of the staged kernels
   };
 
-  // Whether one thread per output that folds k (dot_serial) is faster than the staged kernel with tile t.
-  static bool fold_wins(const GemmShape& gs, const Tile& t, bool f32);
+  // Whether one thread per output that folds k (dot_serial, fold), or with `rows` a row kernel over k, is faster than the
+  // staged kernel with tile t.
+  static bool fold_wins(const GemmShape& gs, const Tile& t, bool f32, bool rows);
 
   // Tile and K split of the direct-to-LDS 16-bit kernel.
   Tile dma_tile(const GemmShape& gs) const;
@@ -459,7 +460,8 @@ class Planner {
   void pack_f32_operands(GemmShape& gs);
 
   // The MFMA templates take operands whose K or M/N stride is 1.
-  bool gemm_eligible(const Op& op, GemmShape& gs) const;
+  // `rows`: spelled as a product summed over trailing axes, which without these kernels is a row kernel.
+  bool gemm_eligible(const Op& op, GemmShape& gs, bool rows = false) const;
 
   // Marks dot operands that are not plain views of a buffer: they are materialised first (by the
   // kernel that produces them, e.g. as a full-row output of a row kernel).

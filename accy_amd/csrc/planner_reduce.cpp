@@ -114,11 +114,10 @@ std::string Planner::fold_body(KernelWriter& w, const std::vector<uint32_t>& gro
     const std::string res = is_int(d) ? "(" + std::string(compute_type(d)) + ")" + acc : round_to(d, acc);
     stores << "    " << w.store(out, "o", d, res) << "\n";
   }
-  // (Unrolled by eight, a single fold of a buffer ends in up to seven rows waited for one by one: 250 x 300 9.9 us, 6.0
-  // as the compiler unrolls it. With arithmetic per row it is the other way round: two folds of 40 sines 7.2 us, 7.8; a softmax's
-  // two folds of 57 keys, one launch each, 1.4 us more.)
-  View plain;
-  body << (group.size() > 1 || !resolve_view(g_.ops[group[0]].args[0], plain) ? "#pragma unroll 8\n" : "") << "    for (I r = 0; r < (I)" << nred << "; ++r) {\n" << steps.str() << "    }\n" << stores.str();
+  // (Unrolled by eight, a single fold ends in up to seven rows waited for one by one: 250 x 300 9.9 us, 6.0 as the compiler
+  // unrolls it; products summed over 130 rows 6.6, 4.6. With more arithmetic per row it is the other way round: two
+  // folds of 40 sines 7.2 us, 7.8; a softmax's folds of 57 keys 1.4 us more.)
+  body << (group.size() > 1 || costly_inside(g_.ops[group[0]].args[0]) ? "#pragma unroll 8\n" : "") << "    for (I r = 0; r < (I)" << nred << "; ++r) {\n" << steps.str() << "    }\n" << stores.str();
   return body.str();
 }
 

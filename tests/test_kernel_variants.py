@@ -273,6 +273,18 @@ def test_contractions_that_leave_tiles_empty_are_folded(dtype, shape, folded):
     assert ("accy::gemm::" not in hip.plan_source(contraction(dtype, m, k, n, "NN", batch))) == folded
 
 
+def test_small_contractions_spelled_as_products_and_sums():
+    """Summed over a middle axis their other form is a fold, a thread per output as for a contraction; over the last axis
+    a row kernel."""
+    def spelled(m, k, n, last):
+        shape = [("m", m), ("n", n), ("k", k)] if last else [("m", m), ("k", k), ("n", n)]
+        def body(b, a):
+            return b.broadcast_in_dim(a[0], shape, [0, 2] if last else [0, 1]).mul(b.broadcast_in_dim(a[1], shape, [1, 2])).sum("k")
+        return hip.plan_source(T.define("mulsum", [T.spec("f32", m=m, k=k), T.spec("f32", n=n, k=k) if last else T.spec("f32", k=k, n=n)], body))
+    for m, k, n, middle, last in [(127, 131, 129, False, False), (33, 130, 65, False, False), (300, 300, 300, True, True), (64, 2000, 64, True, False)]:
+        assert ("accy::gemm::" in spelled(m, k, n, False)) == middle and ("accy::gemm::" in spelled(m, k, n, True)) == last
+
+
 # ---- rows whose length is no multiple of four, or that the threads' vectors do not cover exactly ----
 
 def softmax_rows(b, a):
