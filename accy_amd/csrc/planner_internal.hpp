@@ -314,6 +314,8 @@ class Planner {
   // A transcendental or a division; and whether evaluating a value inline takes one.
   bool costly(uint32_t v) const;
   bool costly_inside(uint32_t v) const;
+  // Registers per thread that hold the row's elements between two passes, at most.
+  uint64_t row_registers(uint64_t per_thread, bool pairs) const;
   void keep_row_values(const RowShape& rs, const RowKernel& rk, uint64_t per_thread, bool pairs);
 
   // ---- launch tuning ----

@@ -387,6 +387,21 @@ bool Planner::costly_inside(uint32_t v) const {
   return walk(v);
 }
 
+uint64_t Planner::row_registers(uint64_t per_thread, bool pairs) const {
+  std::map<int, uint64_t> live;  // pass: registers holding values needed after it
+  auto count = [&](const std::set<int>& uses, bool bits16) {
+    for (int p = *uses.begin(); p < *uses.rbegin(); ++p) live[p] += pairs && bits16 ? per_thread / 2 : per_thread;
+  };
+  for (const auto& leaf : probe_use_) count(leaf.second, dtype_size(plan_.slots[std::stoul(leaf.first)].dtype) == 2);
+  for (const auto& kept : row_keep_) {
+    const auto uses = probe_values_.find(kept.first);
+    if (uses != probe_values_.end()) count(uses->second, dtype_size(g_.type(kept.first).dtype) == 2);
+  }
+  uint64_t most = 0;
+  for (const auto& pass : live) most = std::max(most, pass.second);
+  return most;
+}
+
 // Values of the whole row that cost more than a register to evaluate again (a transcendental, a division) and
 // that a later pass reads too: the pass that computes them first leaves them in registers, as a row
 // read by several passes is. The outermost such value is taken first (what it was computed from is
@@ -395,22 +410,6 @@ bool Planner::costly_inside(uint32_t v) const {
 // with one row to a CU, evaluated twice or kept, as its loads, arithmetic and stores then take turns;
 // 151 us kept, in pairs, with two rows to a CU.)
 void Planner::keep_row_values(const RowShape& rs, const RowKernel& rk, uint64_t per_thread, bool pairs) {
-  auto fits = [&]() {
-    int last = 0;
-    std::map<int, uint64_t> live;  // pass: registers holding values needed after it
-    auto count = [&](const std::set<int>& uses, bool bits16) {
-      for (int p = *uses.begin(); p < *uses.rbegin(); ++p) live[p] += pairs && bits16 ? per_thread / 2 : per_thread;
-      last = std::max(last, *uses.rbegin());
-    };
-    for (const auto& leaf : probe_use_) count(leaf.second, dtype_size(plan_.slots[std::stoul(leaf.first)].dtype) == 2);
-    for (const auto& kept : row_keep_) {
-      const auto uses = probe_values_.find(kept.first);
-      if (uses != probe_values_.end()) count(uses->second, dtype_size(g_.type(kept.first).dtype) == 2);
-    }
-    for (int p = 0; p < last; ++p)
-      if (live[p] > 64) return false;
-    return true;
-  };
   std::set<uint32_t> refused;
   for (int round = 0; round < 8; ++round) {
     uint32_t best = 0;
@@ -423,7 +422,7 @@ void Planner::keep_row_values(const RowShape& rs, const RowKernel& rk, uint64_t 
     if (!found) return;
     row_keep_[best] = *probe_values_.at(best).begin();
     gen_row(rs, rk, false);
-    if (!fits()) {
+    if (row_registers(per_thread, pairs) > 64) {
       row_keep_.erase(best);
       refused.insert(best);
       gen_row(rs, rk, false);
@@ -462,17 +461,22 @@ KernelStep Planner::gen_row(const RowShape& rs, const RowKernel& rk, bool commit
   // Elements of a row that a thread may keep in registers: 64. 16-bit rows too long for that are kept two
   // elements to a register, up to 104 of them (with 128 the addresses and sums beside them spill:
   // 4096 x 32000 bf16 cross-entropy took 264 us with 256 threads of 128, 174 us with 512 of 64), or 128
-  // where a row has no shorter share.
+  // where a row has no shorter share. 256 threads keep 64 also in pairs: two rows that a gradient reads would take 104
+  // registers of each thread (us, 256 threads of 104 / 512 of 64: gradient of a softmax 1000 x 20000 bf16 52 / 35,
+  // 3000 x 24000 160 / 113, of a layer norm 1000 x 20000 50 / 46, 3000 x 24000 158 / 166).
   const bool pairs_ok = commit && VEC == 4 && flat && row_leaves_16bit();
-  auto keepable = [&](uint32_t threads) -> uint64_t { return !pairs_ok ? 64 : threads == 1024 ? 128 : 104; };
+  auto keepable = [&](uint32_t threads) -> uint64_t { return !pairs_ok || threads <= 256 ? 64 : threads == 1024 ? 128 : 104; };
   // No more rows than CUs: as many threads per row as have a vector each, up to 1024, so that a CU has more than two
   // waves. (us a pass, 128 threads / now: logsumexp 1 x 100000 f32 61 / 14, tone 200 x 16384 19.2 / 7.7, 1 x 8395 10.1 /
   // 7.7; rows that 128 threads keep in registers stay at a launch's 7.3.) The line is where rows outnumber the CUs, not
   // where it pays: 512 threads are faster for up to about 1000 long rows as well (128 / 512: tone 300 x 16384 19.2 / 8.0,
   // 1000 x 16384 18.2 / 14.4, logsumexp 500 x 8192 5.8 / 4.1, but 2000 x 4096 6.5 / 7.0).
-  if (kn <= 256)
+  // Up to 1024 rows that one pass reads take 256 or 512 threads with four vectors each: 128 threads hold the waves of
+  // one or two rows per SIMD (sum, sum of squares and maximum, 128 / now: 500 x 32000 f32 22.4 / 11.2, bf16 21.9 / 9.8,
+  // 1000 x 9000 f32 12.8 / 8.1; with fewer vectors each it loses, 600 x 6000 5.0 / 5.9).
+  if (kn <= 256 || (passes == 1 && kn <= 1024))
     for (uint32_t wide : {1024u, 512u, 256u})
-      if (lanes >= wide) {
+      if (kn <= 256 ? lanes >= wide : wide <= 512 && lanes >= 4 * wide) {
         B = wide;
         E = (tn + (uint64_t)B * VEC - 1) / ((uint64_t)B * VEC);
         break;
@@ -521,10 +525,12 @@ KernelStep Planner::gen_row(const RowShape& rs, const RowKernel& rk, bool commit
   std::map<std::string, std::string> leaf_array;
   std::map<std::string, int> leaf_first;
   int cur_pass = 0;
+  uint64_t registers = 0;  // of the row, per thread
   std::string decls;
   std::set<std::string> declared;
   if (commit) {
     if (cache) keep_row_values(rs, rk, E * VEC, pairs);
+    registers = row_registers(E * VEC, pairs);
     leaf_use = probe_use_;
     int na = 0;
     for (auto& [key, uses] : leaf_use) {
@@ -687,8 +693,12 @@ KernelStep Planner::gen_row(const RowShape& rs, const RowKernel& rk, bool commit
       cache ? std::vector<int>{0} : (unrolled ? std::vector<int>{4, 2, 1, 8} : std::vector<int>{2, 1, 4});
   std::string unroll = cache ? "#pragma unroll\n" : kUnrollMark;
   // A wide row's passes each compute their own offsets (carried from pass to pass they would take as many
-  // registers as the row: 316 bytes of scratch for the loss above).
-  const bool wide = cache && B >= 256;
+  // registers as the row: 316 bytes of scratch for the loss above). A row of 256 threads carries them, unless its last
+  // iteration is incomplete or it keeps 65 to 112 registers: us, computed / carried, for 1500 x 16384 f32 (whole, 128
+  // to 192 registers) gradients of a softmax 66 / 55, of a layer norm 140 / 64, 1000 x 12288 bf16 softmax 35 / 21; for
+  // 1000 x 12288 f32 (whole, 96) softmax 29 / 35; for 2000 x 16000 bf16 (incomplete, 192) layer norm 59 / 90.
+  // Whole rows of 144 registers go either way (1000 x 12288 f32: layer norm 43 / 37, RMS norm 28 / 35).
+  const bool wide = cache && (B >= 512 || (B == 256 && (tail || (registers > 64 && registers <= 112))));
   const std::string first_elem = "((I)e * " + std::to_string(B) + " + " + tid + ") * " + std::to_string(VEC);
   const std::string vec_elem = wide ? "(I)e * " + std::to_string(B * VEC) + " + t0" : first_elem;
   const std::string head = "      const I c0 = " + vec_elem + ";\n";
@@ -797,9 +807,13 @@ KernelStep Planner::gen_row(const RowShape& rs, const RowKernel& rk, bool commit
   std::string nm = name("row", rk.reduces[0]);
   std::ostringstream src;
   // A wide row kept in registers: four waves per SIMD, so that two workgroups of 512 threads share a CU and
-  // one computes while the other loads or stores.
+  // one computes while the other loads or stores. Not where the row itself takes the 128 registers that this leaves a
+  // thread (us, four waves / the compiler's choice: layer norm's gradient 3000 x 32000, 192 registers, f32 450 / 322,
+  // bf16 380 / 223; with 120 and 512 threads 1000 x 20000 f32 58 / 67; softmax's 2000 x 16000 bf16, 128 and 256 threads,
+  // 70 / 54).
+  const bool four_waves = wide && registers <= (B >= 512 ? 128 : 112);
   src << "extern \"C\" __global__ void __launch_bounds__(" << B * R << ") "
-      << (wide ? "__attribute__((amdgpu_waves_per_eu(4))) " : "") << nm << "(" << w.params() << ") {\n"
+      << (four_waves ? "__attribute__((amdgpu_waves_per_eu(4))) " : "") << nm << "(" << w.params() << ") {\n"
       << "  typedef " << w.itype << " I;\n" << w.align_hints() << lds_decl;
   if (R > 1)
     src << "  for (I row = (I)blockIdx.x * " << R << " + (I)(threadIdx.x >> 6); row < (I)" << kn

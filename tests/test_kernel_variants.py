@@ -337,6 +337,54 @@ def test_few_rows_take_more_threads(rows, cols, threads):
         assert np.all(np.abs(got - r) <= 1e-5 * r)
 
 
+def norm_backward(dtype):
+    """Three values of the row, the gradient and two inputs, live between its passes."""
+    def body(b, a):
+        x, g, w = a
+        inv = b.full_float(T.Type(dtype, ()), 1.0 / 256)   # any constant does: each side computes the same
+        rs = x.mul(x).sum("c").mul(inv).sqrt()
+        xh, gw = x.div(rs), g.mul(w)
+        return gw.sub(xh.mul(gw.mul(xh).sum("c").mul(inv))).div(rs)
+    return body
+
+
+def norm_backward_program(rows, cols, dtype):
+    return T.define("norm", [T.spec(dtype, r=rows, c=cols)] * 2 + [T.spec(dtype, c=cols)], norm_backward(dtype))
+
+
+def test_rows_of_gradients_choose_threads_and_waves_by_registers():
+    """Threads per row, whether the kernel asks for four waves per SIMD, whether each pass computes its own offsets."""
+    softmax = lambda rows, cols, dtype: T.define("softmax", [T.spec(dtype, r=rows, c=cols)] * 2, lambda b, a: (
+        lambda p: p.mul(a[1].sub(p.mul(a[1]).sum("c"))))((lambda e: e.div(e.sum("c")))(a[0].sub(a[0].max("c")).exp())))
+    moments = lambda rows, cols, dtype: T.define("moments", [T.spec(dtype, r=rows, c=cols)], lambda b, a: [
+        a[0].sum("c"), a[0].mul(a[0]).sum("c"), a[0].max("c")])
+    for prog, threads, waves, offsets in [
+            (norm_backward_program(3000, 32000, "f32"), 512, False, True), (norm_backward_program(1500, 16384, "f32"), 256, False, False),
+            (norm_backward_program(1000, 20000, "bf16"), 512, True, True), (norm_backward_program(1000, 9000, "f32"), 256, True, True),
+            (softmax(1000, 12288, "f32"), 256, True, True), (softmax(1500, 16384, "f32"), 256, False, False),
+            (softmax(2000, 16000, "bf16"), 256, False, True), (softmax(3000, 24000, "bf16"), 512, True, True),
+            (moments(500, 32000, "f32"), 512, False, False), (moments(600, 6000, "f32"), 256, False, False),
+            (moments(600, 3000, "f32"), 128, False, False), (moments(2000, 16384, "f32"), 128, False, False)]:
+        src = hip.plan_source(prog)
+        assert f" block {threads}\n" in src and ("amdgpu_waves_per_eu(4)" in src) == waves and ("+ t0;" in src) == offsets
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,cols,dtype", [(3, 16384, "f32"), (3, 32000, "f32"), (300, 9000, "f32"), (300, 16000, "bf16"), (300, 20000, "bf16")])
+def test_rows_of_gradients_match_float64(rows, cols, dtype):
+    """Positive inputs. f32: the sums are read from 1e-5 (their order) and the result cancels to a third of its terms
+    at most, six roundings of each: 4e-5 of the larger term. 16 bits: ten operations that round to 2^-8."""
+    prog = norm_backward_program(rows, cols, dtype)
+    ins = [W.to_dtype(1.0 + np.abs(W.normal(i, n)), dtype).reshape(s) for i, (n, s) in enumerate([(rows * cols, (rows, cols))] * 2 + [(cols, (cols,))])]
+    x, g, w = (to_f32(i, dtype).astype(np.float64).reshape(i.shape) for i in ins)
+    inv = 1.0 / 256
+    rs = np.sqrt((x * x).sum(1, keepdims=True) * inv)
+    sub = x / rs * ((g * w * x / rs).sum(1, keepdims=True) * inv)
+    got = to_f32(hip_run(prog, ins)[0], dtype).astype(np.float64).reshape(rows, cols)
+    bound = {"f32": 4e-5, "bf16": 10 * 2.0 ** -8}[dtype]
+    assert np.all(np.abs(got - (g * w - sub) / rs) <= bound * (g * w + np.abs(sub)) / rs)
+
+
 @pytest.mark.gpu
 def test_ragged_rows_write_only_their_own_elements():
     """Exact integer rows of 67 and 70 next to each other: every element of the full-row output, and the
